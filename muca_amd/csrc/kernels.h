@@ -46,8 +46,8 @@ struct Launch {
 hipError_t launch_init_lattice(hipStream_t st, int8_t *lat, uint64_t W, uint32_t N,
                                int keying, int rounds, uint32_t mm, uint32_t gpu,
                                uint32_t seed, uint32_t w_offset, uint32_t strat_W = 0);
-hipError_t launch_state(hipStream_t st, const int8_t *lat, uint64_t W, uint32_t N,
-                        const uint32_t *naver, int32_t *E, int32_t *D, int32_t *M);
+hipError_t launch_state(hipStream_t st, const int8_t *lat, uint64_t W, uint32_t L, int32_t *E,
+                        int32_t *D, int32_t *M);
 hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a);
 
 // team kernel (muca_team.hip): LDS layout of one workgroup of 16 walkers

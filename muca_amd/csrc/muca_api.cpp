@@ -318,7 +318,7 @@ int muca_compute_state(muca_ctx *c)
 {
     if (!c) return fail(MUCA_E_ARG, "NULL context");
     HIP_TRY(hipSetDevice(c->p.device));
-    HIP_TRY(muca::launch_state(c->st, c->lat, c->W, c->N, c->naver, c->E, c->D, c->M));
+    HIP_TRY(muca::launch_state(c->st, c->lat, c->W, c->p.L, c->E, c->D, c->M));
     HIP_TRY(hipStreamSynchronize(c->st));
     return MUCA_OK;
 }

@@ -590,36 +590,11 @@ int batch_init(muca_batch *b, uint32_t mm, int stratified)
     b->stratified = stratified;
     BHIP(hipSetDevice(b->device));
     muca::BatchArgs &A = b->a;
-    uint32_t maxN = 0;
-    for (const auto &I : b->inst) maxN = std::max(maxN, I.N);
-    struct DevBuf {
-        uint32_t *p = nullptr;
-        ~DevBuf()
-        {
-            if (p) hipFree(p);
-        }
-    } naver_d;
-    BHIP(hipMalloc((void **)&naver_d.p, 16ull * maxN));
-    std::vector<uint32_t> naver;
-    uint32_t cur_L = 0;
     for (size_t i = 0; i < b->inst.size(); i++) {
         muca::BatchInst &I = b->inst[i];
         BHIP(muca::launch_init_lattice(b->st, A.lat + I.lat_off, I.W, I.N, MUCA_KEYING_WEIGHT, 7,
                                        mm, 0, I.seed, 0, stratified ? I.W : 0));
-        if (I.L != cur_L) {   // neighbour table of this L (muca_delta_multigpu.cu:157-172)
-            BHIP(hipStreamSynchronize(b->st));   // the previous table may still be read
-            naver.assign(4ull * I.N, 0);
-            for (uint32_t s = 0; s < I.N; s++) {
-                const uint32_t x = s % I.L, y = s / I.L;
-                naver[4 * s + 0] = y * I.L + (x + 1) % I.L;
-                naver[4 * s + 1] = y * I.L + (x + I.L - 1) % I.L;
-                naver[4 * s + 2] = ((y + 1) % I.L) * I.L + x;
-                naver[4 * s + 3] = ((y + I.L - 1) % I.L) * I.L + x;
-            }
-            BHIP(hipMemcpy(naver_d.p, naver.data(), naver.size() * 4, hipMemcpyHostToDevice));
-            cur_L = I.L;
-        }
-        BHIP(muca::launch_state(b->st, A.lat + I.lat_off, I.W, I.N, naver_d.p, A.E + I.st_off,
+        BHIP(muca::launch_state(b->st, A.lat + I.lat_off, I.W, I.L, A.E + I.st_off,
                                 A.D + I.st_off, A.M + I.st_off));
         I.iter = 0;
         I.nup = b->init_nup[i];

@@ -74,42 +74,116 @@ hipError_t launch_init_lattice(hipStream_t st, int8_t *lat, uint64_t W, uint32_t
 // ---------------------------------------------------------------------------
 // per-walker E_J, D, M (muca_delta_multigpu.cu:69-83,548-571; produce2_multigpu.cu:66-89)
 // ---------------------------------------------------------------------------
-// sixteen lanes per walker: lane l sums sites l, l+16, ...; the row of
-// sixteen lanes is then reduced (integer sums, so the order does not matter)
-__global__ __launch_bounds__(256) void k_state(const int8_t *lat, uint64_t W, uint32_t N,
-                                               const uint32_t *naver, int32_t *E, int32_t *D,
-                                               int32_t *M)
+// The lattice is read once: the kernel is bound by HBM.  A lane holds four
+// walkers in the bytes of a dword (one walker where W or the lattice is not
+// 4-aligned), 32 lanes read a whole 128-byte line, and each of a workgroup's
+// 32 parts walks down strips of kStrip columns with the row above in
+// registers, so that a site is loaded once (and once more as the right
+// neighbour of the strip before: 9/8 of the lattice).  A bond is counted once,
+// as right and lower neighbour; spins are 0x00, 0x01, 0xFF, so a product of
+// two is nonzero iff bit 0 of their AND is set and then negative iff bit 1 of
+// their XOR is.  Counts are kept in bytes and widened every kFlush rows.
+// L = 72, 524 288 walkers: 0.62 ms (4.4 TB/s of lattice) against 24.5 ms for
+// sixteen lanes per walker that gathered bytes through the neighbour table;
+// L = 256, 16 384 walkers: 0.37 ms against 10.1 ms; 4096 walkers at L = 72:
+// 33 against 269 us.
+constexpr int kStateParts = 32, kStateLanes = 32, kStrip = 8, kFlush = 8;
+
+template <bool VEC>
+__global__ __launch_bounds__(kStateParts *kStateLanes) void k_state(const int8_t *lat, uint64_t W,
+                                                                    uint32_t L, int32_t *E,
+                                                                    int32_t *D, int32_t *M)
 {
-    const uint64_t w = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-    const uint32_t tl = threadIdx.x & 15;
-    if (w >= W) return;   // whole rows of 16 lanes share w
-    int32_t e = 0, d = 0, m = 0;
-    for (uint32_t i = tl; i < N; i += 16) {
-        const int32_t s = lat[(uint64_t)i * W + w];
-        const uint32_t *nv = naver + 4u * i;
-        const int32_t nb = lat[(uint64_t)nv[0] * W + w] + lat[(uint64_t)nv[1] * W + w] +
-                           lat[(uint64_t)nv[2] * W + w] + lat[(uint64_t)nv[3] * W + w];
-        e += -s * nb;
-        d += s * s;
-        m += s;
+    constexpr int V = VEC ? 4 : 1;                 // walkers per lane
+    constexpr uint32_t kOne = 0x01010101u;
+    __shared__ int32_t part[3][kStateParts / 2][kStateLanes * V];
+    const uint32_t lane = threadIdx.x % kStateLanes, p = threadIdx.x / kStateLanes;
+    const uint64_t w = ((uint64_t)blockIdx.x * kStateLanes + lane) * V;
+    int32_t sum[3][V] = {};                        // bonds, D, M
+    if (w < W) {
+        const uint8_t *base = (const uint8_t *)lat + w;
+        auto at = [&](uint32_t y, uint32_t x) -> uint32_t {
+            const uint8_t *q = base + (uint64_t)(y * L + x) * W;
+            return VEC ? *(const uint32_t *)q : (uint32_t)*q;
+        };
+        const uint32_t strips = (L + kStrip - 1) / kStrip;
+        const uint32_t segs = strips < kStateParts ? kStateParts / strips : 1;
+        for (uint32_t it = p; it < strips * segs; it += kStateParts) {
+            const uint32_t strip = it % strips, seg = it / strips;
+            const uint32_t x0 = strip * kStrip, n = min((uint32_t)kStrip, L - x0);
+            const uint32_t y0 = (uint32_t)((uint64_t)L * seg / segs);
+            const uint32_t y1 = (uint32_t)((uint64_t)L * (seg + 1) / segs);
+            if (y0 == y1) continue;
+            const uint32_t xn = x0 + n == L ? 0 : x0 + n;   // the column right of the strip
+            // columns past a narrow last strip repeat its last one on load
+            // and count nothing
+            uint32_t cur[kStrip], right = at(y0, xn);
+#pragma unroll
+            for (int c = 0; c < kStrip; c++) cur[c] = at(y0, x0 + min((uint32_t)c, n - 1));
+            uint32_t nz = 0, ng = 0, ds = 0, ms = 0, rows = 0;
+            for (uint32_t y = y0; y < y1; y++) {
+                const uint32_t yn = y + 1 == L ? 0 : y + 1;
+                uint32_t nxt[kStrip];
+#pragma unroll
+                for (int c = 0; c < kStrip; c++) nxt[c] = at(yn, x0 + min((uint32_t)c, n - 1));
+                const uint32_t rn = at(yn, xn);
+#pragma unroll
+                for (int c = 0; c < kStrip; c++) {
+                    const uint32_t s = (uint32_t)c < n ? cur[c] : 0u;
+                    const uint32_t r = (uint32_t)c + 1 < n ? cur[(c + 1) % kStrip] : right;
+                    const uint32_t br = s & r & kOne, bu = s & nxt[c] & kOne;
+                    nz += br + bu;
+                    ng += (((s ^ r) >> 1) & br) + (((s ^ nxt[c]) >> 1) & bu);
+                    ds += s & kOne;
+                    ms += (s >> 1) & kOne;
+                    cur[c] = nxt[c];
+                }
+                right = rn;
+                if (++rows == kFlush || y + 1 == y1) {
+#pragma unroll
+                    for (int v = 0; v < V; v++) {
+                        auto byte = [&](uint32_t q) { return (int32_t)((q >> (8 * v)) & 0xffu); };
+                        sum[0][v] += byte(nz) - 2 * byte(ng);
+                        sum[1][v] += byte(ds);
+                        sum[2][v] += byte(ds) - 2 * byte(ms);
+                    }
+                    nz = ng = ds = ms = rows = 0;
+                }
+            }
+        }
     }
-    for (int off = 8; off > 0; off >>= 1) {
-        e += __shfl_xor(e, off, 16);
-        d += __shfl_xor(d, off, 16);
-        m += __shfl_xor(m, off, 16);
-    }
-    if (tl == 0) {
-        E[w] = e >> 1;
-        D[w] = d;
-        if (M) M[w] = m;
+    // two parts per wavefront, then the workgroup's sixteen wavefronts
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+            const int32_t t = sum[k][v] + __shfl_xor(sum[k][v], kStateLanes);
+            if (p % 2 == 0) part[k][p / 2][lane * V + v] = t;
+        }
+    __syncthreads();
+    const uint32_t i = threadIdx.x;
+    const uint64_t wi = (uint64_t)blockIdx.x * kStateLanes * V + i;
+    if (i < kStateLanes * V && wi < W) {
+        int32_t t[3] = {};
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            for (int q = 0; q < kStateParts / 2; q++) t[k] += part[k][q][i];
+        E[wi] = -t[0];
+        D[wi] = t[1];
+        if (M) M[wi] = t[2];
     }
 }
 
-hipError_t launch_state(hipStream_t st, const int8_t *lat, uint64_t W, uint32_t N,
-                        const uint32_t *naver, int32_t *E, int32_t *D, int32_t *M)
+hipError_t launch_state(hipStream_t st, const int8_t *lat, uint64_t W, uint32_t L, int32_t *E,
+                        int32_t *D, int32_t *M)
 {
-    hipLaunchKernelGGL(k_state, dim3((unsigned)((W * 16 + 255) / 256)), dim3(256), 0, st, lat, W,
-                       N, naver, E, D, M);
+    const bool vec = W % 4 == 0 && ((uintptr_t)lat & 3) == 0;
+    const uint64_t per = kStateLanes * (vec ? 4 : 1);
+    const dim3 grid((unsigned)((W + per - 1) / per)), block(kStateParts * kStateLanes);
+    if (vec)
+        hipLaunchKernelGGL(k_state<true>, grid, block, 0, st, lat, W, L, E, D, M);
+    else
+        hipLaunchKernelGGL(k_state<false>, grid, block, 0, st, lat, W, L, E, D, M);
     return hipGetLastError();
 }
 
