@@ -9,19 +9,23 @@
 // neighbour of a half-row was last written by an earlier half-row.  So per
 // chunk of a half-row (up to 64 attempts) the team
 //   A. computes in parallel, attempt j on lane j % 16: the Philox blocks,
-//      the proposed spin, dE, dDel, (T)(-dE*beta) and an acceptance bitmask
-//      over a window of 8 (weight path) or 6 (produce path) D values around
-//      the D the chunk starts from,
+//      the proposed spin, dE, dDel, (T)(-dE*beta) and, for each of a window
+//      of 8 (weight path) or 6 (produce path) D values around the D the chunk
+//      starts from, whether the attempt accepts there (one byte each),
 //      screened with the hardware log (the exact log only where the screen
 //      is inconclusive);
-//   B. runs only the D chain serially: attempt j's mask is broadcast from
-//      its lane with a DPP row broadcast and the accept bit is read at the
-//      current D -- no memory access and no branch on the chain.  A round of
-//      16 steps that starts outside the window gets its masks recomputed
-//      around the current D; one in which D leaves the window resumes, with
-//      masks recomputed, from the step that started outside (and, if D
-//      leaves that window too, is replayed with an exact per-step path);
+//   B. resolves the D chain: an attempt is a map of window positions, eight
+//      bytes wide, and v_perm_b32 looks four of them up at once, so sixteen
+//      lanes' maps compose in a prefix scan of four DPP steps and only one
+//      lookup per round of sixteen attempts depends on the D before it.  A
+//      round that starts outside the window, or leaves it, gets the masks of
+//      its undecided attempts recomputed around the D reached;
 //   C. writes the accepted spins, sums dE and dM and fills the histogram.
+// What the scan measured against a serial chain of one DPP broadcast, bit
+// extract and add per attempt: L = 72, 4096 walkers, from ln W = 0: 341 us per
+// launch against 381; L = 128, seeded, NUPDATES = N: 2.19 against 2.51 ms;
+// L = 72 thermalisation in FP64: 0.63 against 0.96 ms; L = 256, 16 384
+// walkers with moments: 15.8 against 19.5 ms.
 // Every acceptance is computed with the reference's operations and rounding:
 //   diff = ((T)(-dE*beta) + lnW[D+dDel]) - lnW[D];  accept iff diff >= 0 or
 //   acclog(r1) < diff.  Because acclog(r1) < 0 always, that is exactly
@@ -56,6 +60,11 @@ constexpr uint32_t kXcds = 8;   // accelerator dies of an MI355X, one L2 each
 constexpr int kWin = 8;
 template <int KEYING>
 constexpr int kWinFor = KEYING == 1 ? 6 : 8;
+// Rounds per chunk where ln W is in HBM: those launches have 128 VGPRs (four
+// wavefronts per SIMD), which two rounds' state fits without spills.  L = 256,
+// 16 384 walkers, 65 536 attempts each, with moments / without: 15.8 / 15.5 ms
+// with two rounds, 16.8 / 16.1 with three, 18.5 / 16.0 with four.
+constexpr int kLnwgRounds = 2;
 constexpr int kGuard = 24;   // ln W guard entries on each side (> kWin / 2 + 2)
 
 __device__ __forceinline__ void wave_sync()
@@ -86,6 +95,88 @@ template <int L>
 __device__ __forceinline__ int32_t row_bcast(int32_t v)
 {
     return __builtin_amdgcn_mov_dpp(v, 0x150 + L, 0xf, 0xf, false);
+}
+
+// a monotone FP32 image of |x|'s order: x itself, or the high word of a double
+// read as a float (magnitudes above 2^1016 read as NaN, which a minimum skips)
+__device__ __forceinline__ float mag_word(float x)
+{
+    return x;
+}
+__device__ __forceinline__ float mag_word(double x)
+{
+    return __uint_as_float((uint32_t)(__double_as_longlong(x) >> 32));
+}
+
+// ---- maps of window positions, KW <= 8 positions as bytes 0..3 (lo), 4..7 (hi)
+
+// byte k of (lo, hi) = 0xff iff bit 31 of sg[k] is set, k < KW; other bytes 0.
+// v_perm_b32(a, b, sel): selector bytes 0x00-0x03 take b's bytes, 0x0b and
+// 0x09 replicate the sign of a and of b, 0x0c is 0x00
+template <int KW>
+__device__ __forceinline__ void sign_bytes(const uint32_t *sg, uint32_t &lo, uint32_t &hi)
+{
+    auto four = [&](int k0, int n) -> uint32_t {
+        uint32_t v = n > 1 ? __builtin_amdgcn_perm(sg[k0 + 1], sg[k0], 0x0c0c0b09u)
+                           : __builtin_amdgcn_perm(sg[k0], sg[k0], 0x0c0c0c09u);
+        if (n > 2) v = __builtin_amdgcn_perm(sg[k0 + 2], v, 0x0c0b0100u);
+        if (n > 3) v = __builtin_amdgcn_perm(sg[k0 + 3], v, 0x0b020100u);
+        return v;
+    };
+    lo = four(0, KW < 4 ? KW : 4);
+    hi = KW > 4 ? four(4, KW - 4) : 0u;
+}
+
+// the identity: byte k = k for k < KW, else 0xff
+template <int KW>
+__device__ __forceinline__ constexpr uint32_t window_id(int word)
+{
+    uint32_t v = 0;
+    for (int k = 0; k < 4; k++) {
+        const int q = 4 * word + k;
+        v |= (q < KW ? (uint32_t)q : 0xffu) << (8 * k);
+    }
+    return v;
+}
+
+// the map of one attempt: k + dDel where its accept byte k is set, else k;
+// 0xff outside 0..KW-1.  dp1 = dDel + 1 in its low two bits: the moved
+// positions are the four bytes from dp1 on of ff 00 01 .. KW-1 ff ff
+template <int KW>
+__device__ __forceinline__ void window_map(uint32_t alo, uint32_t ahi, uint32_t dp1, uint32_t &lo,
+                                           uint32_t &hi)
+{
+    auto seq = [](int i) -> uint32_t { return i >= 1 && i <= KW ? (uint32_t)(i - 1) : 0xffu; };
+    auto word = [&](int i) { return seq(i) | seq(i + 1) << 8 | seq(i + 2) << 16 | seq(i + 3) << 24; };
+    const uint32_t s = dp1 & 3u;
+    const uint32_t mlo = __builtin_amdgcn_alignbyte(word(4), word(0), s);
+    lo = (alo & mlo) | (~alo & window_id<KW>(0));
+    if (KW > 4) {
+        const uint32_t mhi = __builtin_amdgcn_alignbyte(word(8), word(4), s);
+        hi = (ahi & mhi) | (~ahi & window_id<KW>(1));
+    } else {
+        hi = 0xffffffffu;
+    }
+}
+
+// byte `at` of (lo, hi), 0xff for at = 0xff
+__device__ __forceinline__ uint32_t window_at(uint32_t lo, uint32_t hi, uint32_t at)
+{
+    return __builtin_amdgcn_perm(hi, lo, at | 0x0c0c0c00u);
+}
+
+// one level of the inclusive prefix scan: the map of the lane DPP points at
+// (row_shr), then this lane's; q holds the identity where there is no such lane
+template <int KW, int DPP>
+__device__ __forceinline__ void scan_level(uint32_t &lo, uint32_t &hi, uint32_t &ql, uint32_t &qh)
+{
+    ql = (uint32_t)__builtin_amdgcn_update_dpp((int)ql, (int)lo, DPP, 0xf, 0xf, false);
+    const uint32_t l = __builtin_amdgcn_perm(hi, lo, ql);
+    if (KW > 4) {
+        qh = (uint32_t)__builtin_amdgcn_update_dpp((int)qh, (int)hi, DPP, 0xf, 0xf, false);
+        hi = __builtin_amdgcn_perm(hi, lo, qh);
+    }
+    lo = l;
 }
 
 }  // namespace team_detail
@@ -245,6 +336,14 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
         int32_t pf_s[NR], pf_r[NR], pf_l[NR], pf_u[NR], pf_d[NR], fin[NR];
         bool pf_have = false, pf_fwd = false;
         int32_t de_lane = 0, dm_lane = 0;
+        // the scan's shifted-in maps per level: the lanes that have no source
+        // lane at a level keep the identity from here on
+        uint32_t ql[4], qh[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            ql[k] = window_id<KW>(0);
+            qh[k] = window_id<KW>(1);
+        }
         // a workgroup adds at most 16 NUPDATES counts to one u32 bin
         const bool may_wrap = a.hist_preload != 0 || (uint64_t)kTeams * a.nup >= (1ull << 32);
         for (int phase = 0; phase < 2; phase++) {
@@ -304,18 +403,23 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 const int32_t dlo_a = dlo;            // the window of every mask made here
                 const uint32_t yu = (y + 1 == L) ? 0 : y + 1, yd = (y == 0) ? L - 1 : y - 1;
                 const uint32_t s4 = slot0 * 4, ringw = RB * 4;   // ring word of attempt j: s4 + j (mod ringw)
-                uint32_t mask[NR];
-                // dDel (2-bit signed) | (dE + 8) << 2 | (new - old + 2) << 7 | (new + 1) << 10
+                // attempt j's accept bytes: byte k is 0xff iff it accepts at
+                // D = dlo_a + k (bytes 0..3, 4..7)
+                uint32_t alo[NR], ahi[NR];
+                // (dDel + 1) | (dE + 8) << 2 | (new - old + 2) << 7 | (new + 1) << 10
                 int32_t info[NR];
-                // Bits k = 0..KW-1: accept at D = dlo + k, i.e. acclog(r1) <
+                // Byte k = 0..KW-1: accept at D = dlo + k, i.e. acclog(r1) <
                 // ((fde + lnW[D + dDel]) - lnW[D]), screened with the hardware
                 // log and its proven band: la + band < diff accepts, la - band
-                // >= diff rejects.  Bit k is the sign of e = thi - diff (e is
+                // >= diff rejects.  Byte k is the sign of e = thi - diff (e is
                 // -0 never, +0 iff thi == diff, which rejects); a diff with
                 // tlo < diff <= thi, i.e. 0 <= e < thi - tlo, needs the exact
                 // log -- flagged (with margin) by min |e| < 2 (thi - tlo).
-                auto accept_bits = [&](const T *wf, const T *wc, uint32_t r1, T fde,
-                                       int32_t ddel) -> uint32_t {
+                // The minimum is taken over mag_word (exact in FP32, the high
+                // words in FP64, compared there with <=).  An attempt past the
+                // chunk's end has fde = -inf and accepts nowhere.
+                auto accept_bytes = [&](const T *wf, const T *wc, uint32_t r1, T fde,
+                                        int32_t ddel, uint32_t &lo, uint32_t &hi) {
                     const T *wto = wc + ddel;
                     T diff[KW];
 #pragma unroll
@@ -326,26 +430,26 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     const float la = acclog_fast_u01(r1);
                     const float band = acclog_fast_band(la);
                     const T thi = (T)(la + band), tlo = (T)(la - band);
-                    uint32_t mk = 0;
-                    T emin = (T)1e30f;
+                    uint32_t sg[8];
+                    float emin = 1e30f;
 #pragma unroll
-                    for (int k = KW - 1; k >= 0; k--) {
+                    for (int k = 0; k < KW; k++) {
                         const T e = thi - diff[k];
-                        mk = __builtin_amdgcn_alignbit(mk, sign_word(e), 31);
-                        emin = fmin(emin, fabs(e));
+                        sg[k] = sign_word(e);
+                        emin = fminf(emin, fabsf(mag_word(e)));
                     }
-                    const bool amb = emin < (thi - tlo) + (thi - tlo);
+                    sign_bytes<KW>(sg, lo, hi);
+                    const float lim = mag_word((thi - tlo) + (thi - tlo));
+                    const bool amb = FP64 ? emin <= lim : emin < lim;
                     if (__builtin_amdgcn_ballot_w64(amb)) {   // rare: a diff within the band
                         if (amb) {
                             const T tlog =
                                 (T)(float)acclog_u01_double_tab(r1, logtab, logtab + 128);
-                            mk = 0;
 #pragma unroll
-                            for (int k = KW - 1; k >= 0; k--)
-                                mk = mk + mk + (tlog < diff[k] ? 1u : 0u);
+                            for (int k = 0; k < KW; k++) sg[k] = tlog < diff[k] ? 0x80000000u : 0u;
+                            sign_bytes<KW>(sg, lo, hi);
                         }
                     }
-                    return mk;
                 };
                 // Branch-free over the rounds so that the loads of all rounds
                 // can be in flight together: a lane past the end of the
@@ -377,17 +481,9 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     const int32_t ddel = new_s * new_s - old_s * old_s;
                     // (T)(-dE * beta) by arithmetic (the same operations as
                     // the table in LDS, without a dependent LDS load)
-                    const uint32_t mk =
-                        accept_bits(wfrom, wcen, r1, (T)(-(double)dE * a.beta), ddel);
-                    // bits 0..KW-1: accept at D = dlo + k; bits 16..17: dDel
-                    mask[r] = mk | (valid ? ((uint32_t)ddel & 3u) << 16 : 0u);
-                    if (JOINT)
-                        info[r] = valid ? ((ddel & 3) | ((dE + 8) << 2) | ((ds + 2) << 7) |
-                                           ((new_s + 1) << 10))
-                                        : ((8 << 2) | (2 << 7));
-                    else
-                        info[r] = valid ? ((dE + 8) << 2) | ((ds + 2) << 7) | ((new_s + 1) << 10)
-                                        : ((8 << 2) | (2 << 7));
+                    const T fde = (T)(-(double)dE * a.beta);
+                    accept_bytes(wfrom, wcen, r1, valid ? fde : -(T)INFINITY, ddel, alo[r], ahi[r]);
+                    info[r] = (ddel + 1) | ((dE + 8) << 2) | ((ds + 2) << 7) | ((new_s + 1) << 10);
                 }
                 wave_sync();
                 if (PF) {
@@ -443,264 +539,164 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                         }
                     }
                 }
-                // ---- B: the D chain.  The chain runs on `off` = D - dlo (the
-                // window position); per step one DPP broadcast of the attempt's
-                // mask word, the accept bit at the current position, its dDel,
-                // and the move.  A position outside the window reads a zero bit
-                // (bits KW..15 and 24..31 of the word are zero), so the chain
-                // then stays put; the D recovered after the round shows such an
-                // excursion, and the round is replayed exactly.
-                uint32_t accb[NR];
-                int32_t dv[NR], mv[NR];
+                // ---- B: the D chain.  Attempt j maps the window position k =
+                // D - dlo before it to the one after it: k + dDel where byte k
+                // of its accept bytes is set, else k; a position outside the
+                // window is 0xff and stays so.  A map is eight bytes, and
+                // v_perm_b32 looks up four of them at once (a selector of 0xff
+                // gives 0xff), so that two maps compose in two instructions
+                // and sixteen lanes' maps in a prefix scan of four levels.  The
+                // scans of all rounds are independent of D and of each other;
+                // only one lookup per round depends on the D the round before
+                // ended at.
                 const uint32_t sh = (uint32_t)(tid & 48);    // this team's 16 lanes of a ballot
                 const uint32_t upto = (2u << tl) - 1u;       // steps 0..tl of a round
-                int32_t off = d - dlo;
-                // D after this lane's step from the round's start, the accept bits
-                // and the dDel of every step (two ballots)
-                auto recover = [&](int r, int32_t off0, uint32_t ab) -> int32_t {
-                    const int32_t my = __builtin_amdgcn_sbfe((int32_t)mask[r], 16, 2);
-                    const uint32_t up =
-                        (uint32_t)(__builtin_amdgcn_ballot_w64(my > 0) >> sh) & 0xffffu & ab;
-                    const uint32_t dn =
-                        (uint32_t)(__builtin_amdgcn_ballot_w64(my < 0) >> sh) & 0xffffu & ab;
-                    return off0 + __builtin_popcount(up & upto) - __builtin_popcount(dn & upto);
-                };
-                // One chain step.  CHK = false: no memory access and no branch.
-                // CHK = true: a step that starts outside the window is decided
-                // exactly from the attempt's record in LDS.
-                // MODE 0: no memory access and no branch.  MODE 1: a step that
-                // starts outside the window is decided exactly from the
-                // attempt's record.  MODE 2: as 0 from step kres on, steps
-                // before kres left alone.
-                uint32_t kres = 0;
-                auto step = [&](auto lc, auto mode, int r, uint32_t &ab) {
-                    constexpr int l = decltype(lc)::value;
-                    constexpr int MODE = decltype(mode)::value;
-                    constexpr bool CHK = MODE == 1;
-                    const uint32_t mj = (uint32_t)row_bcast<l>((int32_t)mask[r]);
-                    const int32_t ddel = __builtin_amdgcn_sbfe((int32_t)mj, 16, 2);
-                    // v_bfe_u32 reads the offset modulo 32
-                    uint32_t acc = __builtin_amdgcn_ubfe(mj, (uint32_t)off, 1);
-                    if (MODE == 2) acc = (uint32_t)l >= kres ? acc : 0u;
-                    if (CHK) {
-                        // a step outside the window: the attempt's dE from its
-                        // info word, its r1 from the ring, the screened log
-                        // (exact only inside the band)
-                        const bool oob = (uint32_t)off >= (uint32_t)KW;
-                        if (__builtin_amdgcn_ballot_w64(oob)) {
-                            if (oob) {
-                                const int32_t ij = row_bcast<l>(info[r]);
-                                uint32_t w1 = s4 + 16 * r + l;
-                                w1 = w1 >= ringw ? w1 - ringw : w1;
-                                const uint32_t r1 = rng[w1];
-                                const int32_t dd = dlo + off;
-                                T diff = fdet[((ij >> 2) & 31) - 8] + lnw_at(dd + ddel);
-                                diff = diff - lnw_at(dd);
-                                const float la = acclog_fast_u01(r1);
-                                const float band = acclog_fast_band(la);
-                                acc = (T)(la + band) < diff ? 1u : 0u;
-                                const bool amb = !acc && (T)(la - band) < diff;
-                                if (__builtin_amdgcn_ballot_w64(amb)) {
-                                    if (amb)
-                                        acc = (T)(float)acclog_u01_double_tab(r1, logtab,
-                                                                              logtab + 128) < diff
-                                                  ? 1u
-                                                  : 0u;
-                                }
-                            }
-                        }
-                    }
-                    off += (int32_t)acc * ddel;
-                    ab |= acc << l;
-                };
-                using Fast = std::integral_constant<int, 0>;
-                using Checked = std::integral_constant<int, 1>;
-                using Resume = std::integral_constant<int, 2>;
-                // round r's masks recomputed around dlo by all lanes of the team
-                auto remask = [&](uint32_t &mk_r, int32_t inf_r, int r) {
-                    const T *wc = window();
-                    T wf[KW];
+                // made ahead of the rounds where registers allow
+                constexpr bool AHEAD = !LNWG;
+                auto scan = [&](uint32_t lo, uint32_t hi, int32_t inf, uint32_t &plo,
+                                uint32_t &phi) {
+                    window_map<KW>(lo, hi, (uint32_t)inf, plo, phi);
+                    if (!AHEAD)
 #pragma unroll
-                    for (int k = 0; k < KW; k++) wf[k] = wc[k];
-                    uint32_t w1 = s4 + min(16 * (uint32_t)r + tl, cnt - 1);
-                    w1 = w1 >= ringw ? w1 - ringw : w1;
-                    const int32_t dd = __builtin_amdgcn_sbfe((int32_t)mk_r, 16, 2);
-                    const uint32_t mk =
-                        accept_bits(wf, wc, rng[w1], fdet[((inf_r >> 2) & 31) - 8], dd);
-                    mk_r = mk | (mk_r & 0x30000u);
+                        for (int k = 0; k < 4; k++) {
+                            ql[k] = window_id<KW>(0);
+                            qh[k] = window_id<KW>(1);
+                        }
+                    scan_level<KW, 0x111>(plo, phi, ql[0], qh[0]);
+                    scan_level<KW, 0x112>(plo, phi, ql[1], qh[1]);
+                    scan_level<KW, 0x114>(plo, phi, ql[2], qh[2]);
+                    scan_level<KW, 0x118>(plo, phi, ql[3], qh[3]);
                 };
-#define MUCA_STEPS(K, AB)                                                                    \
-    if (left >= 16) {                                                                        \
-        step(std::integral_constant<int, 0>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 1>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 2>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 3>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 4>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 5>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 6>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 7>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 8>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 9>(), K(), r, AB);                                  \
-        step(std::integral_constant<int, 10>(), K(), r, AB);                                 \
-        step(std::integral_constant<int, 11>(), K(), r, AB);                                 \
-        step(std::integral_constant<int, 12>(), K(), r, AB);                                 \
-        step(std::integral_constant<int, 13>(), K(), r, AB);                                 \
-        step(std::integral_constant<int, 14>(), K(), r, AB);                                 \
-        step(std::integral_constant<int, 15>(), K(), r, AB);                                 \
-    } else {                                                                                 \
-        if (0 < left) step(std::integral_constant<int, 0>(), K(), r, AB);                    \
-        if (1 < left) step(std::integral_constant<int, 1>(), K(), r, AB);                    \
-        if (2 < left) step(std::integral_constant<int, 2>(), K(), r, AB);                    \
-        if (3 < left) step(std::integral_constant<int, 3>(), K(), r, AB);                    \
-        if (4 < left) step(std::integral_constant<int, 4>(), K(), r, AB);                    \
-        if (5 < left) step(std::integral_constant<int, 5>(), K(), r, AB);                    \
-        if (6 < left) step(std::integral_constant<int, 6>(), K(), r, AB);                    \
-        if (7 < left) step(std::integral_constant<int, 7>(), K(), r, AB);                    \
-        if (8 < left) step(std::integral_constant<int, 8>(), K(), r, AB);                    \
-        if (9 < left) step(std::integral_constant<int, 9>(), K(), r, AB);                    \
-        if (10 < left) step(std::integral_constant<int, 10>(), K(), r, AB);                  \
-        if (11 < left) step(std::integral_constant<int, 11>(), K(), r, AB);                  \
-        if (12 < left) step(std::integral_constant<int, 12>(), K(), r, AB);                  \
-        if (13 < left) step(std::integral_constant<int, 13>(), K(), r, AB);                  \
-        if (14 < left) step(std::integral_constant<int, 14>(), K(), r, AB);                  \
-    }
+                // the maps of steps 0..tl of each round
+                uint32_t plo[NR], phi[NR];
+                if (AHEAD)
+#pragma unroll
+                    for (int r = 0; r < NR; r++) scan(alo[r], ahi[r], info[r], plo[r], phi[r]);
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
-                    accb[r] = 0;
-                    dv[r] = d;
-                    mv[r] = m;
                     const uint32_t j0 = 16 * r;
+                    if (PF) fin[r] = -9;
                     if (j0 >= cnt) continue;
-                    const uint32_t left = cnt - j0;
+                    if (!AHEAD) scan(alo[r], ahi[r], info[r], plo[r], phi[r]);
+                    const bool valid = j0 + tl < cnt;
+                    // the window's accept bytes recomputed around dlo by all
+                    // lanes of the team; steps below `from` are decided and
+                    // become identities
+                    auto remask = [&](uint32_t from) {
+                        const T *wc = window();
+                        T wf[KW];
+#pragma unroll
+                        for (int k = 0; k < KW; k++) wf[k] = wc[k];
+                        uint32_t w1 = s4 + min(j0 + tl, cnt - 1);
+                        w1 = w1 >= ringw ? w1 - ringw : w1;
+                        const T fde = fdet[((info[r] >> 2) & 31) - 8];
+                        accept_bytes(wf, wc, rng[w1], valid && tl >= from ? fde : -(T)INFINITY,
+                                     (info[r] & 3) - 1, alo[r], ahi[r]);
+                        scan(alo[r], ahi[r], info[r], plo[r], phi[r]);
+                    };
                     // the window follows D from round to round: a round that
                     // starts outside the masks' window gets its masks
-                    // recomputed around the current D, by all lanes of the
-                    // team at once (only this round's: the later rounds'
-                    // masks stay relative to dlo_a)
+                    // recomputed around the current D (only this round's: the
+                    // later rounds' stay relative to dlo_a)
                     dlo = dlo_a;
-                    off = d - dlo_a;
-                    const bool shift = (uint32_t)off >= (uint32_t)KW;
+                    uint32_t off = (uint32_t)(d - dlo_a);
+                    const bool shift = off >= (uint32_t)KW;
                     if (__builtin_amdgcn_ballot_w64(shift)) {
                         if (shift) {
-                            dlo += off - KW / 2;
+                            dlo = d - KW / 2;
                             off = KW / 2;
-                            remask(mask[r], info[r], r);
+                            remask(0);
                         }
                     }
-                    const int32_t off0 = off;
-                    uint32_t ab = 0;
-                    MUCA_STEPS(Fast, ab)
-                    int32_t o = recover(r, off0, ab);
-                    // a step started outside the window iff one before it in the
-                    // round ended there (a lane past the chunk's end repeats
-                    // the last step's D)
-                    const bool out = (uint32_t)o >= (uint32_t)KW && tl + 1 < min(left, 16u);
-                    if (__builtin_amdgcn_ballot_w64(out)) {
-                        const uint32_t mine =
-                            (uint32_t)(__builtin_amdgcn_ballot_w64(out) >> sh) & 0xffffu;
+                    uint32_t o = window_at(plo[r], phi[r], off);
+                    uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(
+                        (int)off, (int)o, 0x111, 0xf, 0xf, false);
+                    // this lane's attempt: accepted, and D (and M) after it
+                    bool acc = window_at(alo[r], ahi[r], before) != 0;
+                    int32_t dv = dlo + (int32_t)o, mv = 0;
+                    // Rare: D left the window at step k.  Steps 0..k stand (step
+                    // k is accepted and moved D by its dDel); the masks of the
+                    // later ones are recomputed around D there, and so on until
+                    // the round is done.  k grows by KW / 2 at least each time.
+                    uint64_t outs;
+                    bool out = o == 0xffu;
+                    while ((outs = __builtin_amdgcn_ballot_w64(out)) != 0) {
+                        const uint32_t mine = (uint32_t)(outs >> sh) & 0xffffu;
                         if (mine) {
-                            // D left the window after step kres - 1: steps
-                            // 0 .. kres - 1 stand; the masks are recomputed
-                            // around D at the start of step kres and the chain
-                            // resumes there
-                            kres = (uint32_t)__builtin_ctz(mine) + 1u;
-                            const int32_t moved = __shfl(o, (int)kres - 1, kTeam) - KW / 2;
-                            dlo += moved;
-                            remask(mask[r], info[r], r);
-                            const int32_t offr0 = off0 - moved;   // the round's start, new window
-                            off = KW / 2;
-                            uint32_t abr = 0;
-                            MUCA_STEPS(Resume, abr)
-                            ab = (ab & ((1u << kres) - 1u)) | abr;
-                            o = recover(r, offr0, ab);
-                            // rare: D left the new window too -- replay exactly
-                            const bool out2 = (uint32_t)o >= (uint32_t)KW &&
-                                              tl + 1 < min(left, 16u) && (uint32_t)tl >= kres;
-                            if ((uint32_t)(__builtin_amdgcn_ballot_w64(out2) >> sh) & 0xffffu) {
-                                off = offr0;
-                                ab = 0;
-                                MUCA_STEPS(Checked, ab)
-                                o = recover(r, offr0, ab);
+                            const uint32_t k = (uint32_t)__builtin_ctz(mine);
+                            const int32_t dk = dlo + (int32_t)before + (info[r] & 3) - 1;
+                            if ((uint32_t)tl == k) dv = dk;
+                            dlo = __shfl(dk, (int)k, kTeam) - KW / 2;
+                            remask(k + 1);
+                            o = window_at(plo[r], phi[r], KW / 2);
+                            before = (uint32_t)__builtin_amdgcn_update_dpp(
+                                KW / 2, (int)o, 0x111, 0xf, 0xf, false);
+                            out = o == 0xffu;
+                            if ((uint32_t)tl > k) {
+                                acc = window_at(alo[r], ahi[r], before) != 0;
+                                dv = dlo + (int32_t)o;
                             }
                         }
                     }
-                    accb[r] = ab;
-                    dv[r] = dlo + o;
-                    d = dlo + off;
+                    d = row_bcast<15>(dv);
                     if (TRACKM) {
                         // M after this lane's step: an inclusive scan over the
                         // team of the accepted spin changes
-                        int32_t x = (int32_t)((ab >> tl) & 1u) * (((info[r] >> 7) & 7) - 2);
+                        int32_t x = acc ? ((info[r] >> 7) & 7) - 2 : 0;
                         x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
                         x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
                         x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
                         x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
-                        mv[r] = m + x;
+                        mv = m + x;
                         m += row_bcast<15>(x);
                     }
-                }
-#undef MUCA_STEPS
-                // ---- C: accepted spins, dE / dM sums, histogram
-                int32_t de = 0, dm = 0;
-#pragma unroll
-                for (int r = 0; r < NR; r++) {
-                    const uint32_t j = 16 * r + tl;
-                    if (PF) {
-                        // the site's spin after this chunk (info: new spin + 1
-                        // at bits 10-11, new - old + 2 at bits 7-9)
-                        const int32_t ns = ((info[r] >> 10) & 3) - 1;
-                        const int32_t os = ns - (((info[r] >> 7) & 7) - 2);
-                        fin[r] = j < cnt ? (((accb[r] >> tl) & 1u) ? ns : os) : -9;
+                    // ---- C: accepted spins, dE / dM sums, histogram of the round
+                    const uint32_t j = j0 + tl, left = min(cnt - j0, 16u);
+                    const int32_t ns = ((info[r] >> 10) & 3) - 1;    // the proposed spin
+                    const int32_t ds = ((info[r] >> 7) & 7) - 2;
+                    // the site's spin after this chunk
+                    if (PF) fin[r] = valid ? (acc ? ns : ns - ds) : -9;
+                    if (acc) {
+                        // the new spin is known from phase A: no site of
+                        // the chunk is written between its read and here
+                        sp(y * L + 2 * (jb + j) + h) = (int8_t)ns;
+                        de_lane += ((info[r] >> 2) & 31) - 8;
+                        dm_lane += ds;
                     }
-                    if (j < cnt) {
-                        if ((accb[r] >> tl) & 1u) {
-                            // the new spin is known from phase A: no site of
-                            // the chunk is written between its read and here
-                            const int32_t ds = ((info[r] >> 7) & 7) - 2;
-                            sp(y * L + 2 * (jb + j) + h) = (int8_t)(((info[r] >> 10) & 3) - 1);
-                            de += ((info[r] >> 2) & 31) - 8;
-                            dm += ds;
-                        }
-                        if (phase && JOINT) {
-                            const int64_t dd = dv[r];
-                            const int64_t mm = min(max((int64_t)mv[r], -dd), dd);
-                            const int64_t jbn = (mm + dd * dd + 2 * dd) / 2;
-                            if (jbn != jbin) {
-                                if (jbn == jpbin) {
-                                    const uint64_t t = jrun;
-                                    jrun = jprun;
-                                    jprun = t;
-                                    jpbin = jbin;
-                                } else {
-                                    if (jprun)
-                                        atomicAdd((unsigned long long *)&jbase[jpbin], jprun);
-                                    jprun = jrun;
-                                    jpbin = jbin;
-                                    jrun = 0;
-                                }
-                                jbin = jbn;
+                    if (JOINT && phase && valid) {
+                        const int64_t dd = dv;
+                        const int64_t mm = min(max((int64_t)mv, -dd), dd);
+                        const int64_t jbn = (mm + dd * dd + 2 * dd) / 2;
+                        if (jbn != jbin) {
+                            if (jbn == jpbin) {
+                                const uint64_t t = jrun;
+                                jrun = jprun;
+                                jprun = t;
+                                jpbin = jbin;
+                            } else {
+                                if (jprun)
+                                    atomicAdd((unsigned long long *)&jbase[jpbin], jprun);
+                                jprun = jrun;
+                                jpbin = jbin;
+                                jrun = 0;
                             }
-                            jrun++;
+                            jbin = jbn;
                         }
+                        jrun++;
                     }
-                }
-                if (phase && !MOMS) {
-                    // The D histogram: a round's steps split into runs at one D,
-                    // starting at step 0 and at every accepted step that
-                    // changed D; the first lane of a run adds its length (one
-                    // atomic per run instead of sixteen on the same bin)
-#pragma unroll
-                    for (int r = 0; r < NR; r++) {
-                        if (16 * r >= cnt) break;
-                        const uint32_t left = min(cnt - 16 * r, 16u);
-                        const bool moved = ((accb[r] >> tl) & 1u) && (mask[r] & 0x30000u);
+                    if (phase && !MOMS) {
+                        // The D histogram: a round's steps split into runs at one D,
+                        // starting at step 0 and at every accepted step that
+                        // changed D; the first lane of a run adds its length (one
+                        // atomic per run instead of sixteen on the same bin)
+                        const bool moved = acc && (info[r] & 3) != 1;
                         const uint32_t starts =
                             ((uint32_t)(__builtin_amdgcn_ballot_w64(moved) >> sh) & 0xffffu) | 1u;
                         const uint32_t later = starts & ~upto;
                         const uint32_t len =
                             (later ? (uint32_t)__builtin_ctz(later) : left) - (uint32_t)tl;
                         if (tl < left && ((starts >> tl) & 1u)) {
-                            const int32_t dd = dv[r];
+                            const int32_t dd = dv;
                             if (LDSHIST) {
                                 if (may_wrap) {
                                     // a u32 bin that wraps carries 2^32 into HBM
@@ -714,26 +710,22 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                             }
                         }
                     }
-                }
-                if (MOMS && phase) {
-                    // Attempt j records the (D, M) after its step.  Steps that
-                    // are not accepted keep the state, so a round splits into
-                    // segments that start at step 0 and at every accepted step
-                    // and share one (D, M); the first lane of each segment adds
-                    // len x (1, |M|, M^2, M^4) to the slot of its D.
-#pragma unroll
-                    for (int r = 0; r < NR; r++) {
-                        if (16 * r >= cnt) break;
-                        const uint32_t left = min(cnt - 16 * r, 16u);
-                        const uint32_t ab = accb[r];
-                        const bool lead = tl < left && (tl == 0 || ((ab >> tl) & 1u));
+                    if (MOMS && phase) {
+                        // Attempt j records the (D, M) after its step.  Steps that
+                        // are not accepted keep the state, so a round splits into
+                        // segments that start at step 0 and at every accepted step
+                        // and share one (D, M); the first lane of each segment adds
+                        // len x (1, |M|, M^2, M^4) to the slot of its D.
+                        const uint32_t ab =
+                            (uint32_t)(__builtin_amdgcn_ballot_w64(acc) >> sh) & 0xffffu;
+                        const bool lead = tl < left && (tl == 0 || acc);
                         const uint32_t later = ab & ~upto;
                         const uint32_t len =
                             (later ? (uint32_t)__builtin_ctz(later) : left) - (uint32_t)tl;
-                        const int32_t dd = dv[r];
+                        const int32_t dd = dv;
                         int32_t slot = dd - mwb;
-                        const bool out = lead && (uint32_t)slot >= (uint32_t)kMomSlots;
-                        const uint64_t ob = __builtin_amdgcn_ballot_w64(out);
+                        const bool past = lead && (uint32_t)slot >= (uint32_t)kMomSlots;
+                        const uint64_t ob = __builtin_amdgcn_ballot_w64(past);
                         if (ob) {
                             if ((ob >> sh) & 0xffffu) {   // the whole team: new window
                                 flush_slot();
@@ -742,7 +734,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                             }
                         }
                         if (lead) {
-                            const int32_t mm = min(max(mv[r], -dd), dd);
+                            const int32_t mm = min(max(mv, -dd), dd);
                             const uint64_t am = (uint64_t)(mm < 0 ? -mm : mm);
                             const uint64_t m2 = am * am;
                             const uint64_t q = m2 * m2, qh = __umul64hi(m2, m2);   // M^4
@@ -769,8 +761,6 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                         }
                     }
                 }
-                de_lane += de;
-                dm_lane += dm;
                 if (!LATLDS) __threadfence_block();
                 wave_sync();
                 rs += cnt;
@@ -871,7 +861,7 @@ hipError_t launch_team_nr(hipStream_t st, const McsArgs &a, const TeamLayout &la
     if (lay.lnw_global) {
         // ln W too large for LDS (L >= 136): lattices and histogram stay in
         // HBM as well
-        if constexpr (NR == 4) {
+        if constexpr (NR == kLnwgRounds) {
             k = moms ? k_mcs_team<R, FP64, KEYING, false, false, MO, true, NR>
                 : joint ? k_mcs_team<R, FP64, KEYING, false, false, 1, true, NR>
                         : k_mcs_team<R, FP64, KEYING, false, false, 0, true, NR>;
@@ -910,6 +900,7 @@ template <int R, bool FP64, int KEYING>
 hipError_t launch_team_r(hipStream_t st, const McsArgs &a, const TeamLayout &lay)
 {
     const uint32_t rounds = (lay.row + 15) / 16;
+    if (lay.lnw_global) return launch_team_nr<R, FP64, KEYING, kLnwgRounds>(st, a, lay);
     if (rounds <= 1) return launch_team_nr<R, FP64, KEYING, 1>(st, a, lay);
     if (rounds <= 2) return launch_team_nr<R, FP64, KEYING, 2>(st, a, lay);
     if (rounds <= 3) return launch_team_nr<R, FP64, KEYING, 3>(st, a, lay);
