@@ -110,6 +110,25 @@ __device__ static inline float acclog_fast_band(float la)
     return fabsf(la) * ACCLOG_FAST_REL + ACCLOG_FAST_ABS;
 }
 
+// The same screen with one bound and a margin, one multiply-add each after
+// the hardware log: thi = la + band up to 3/16 band (three roundings of
+// 2^-24 |la| = band / 16 each), so 0.31 band < thi - log(u) < 1.69 band; and
+// lim = 4 band (from |thi|, which differs from |la| by less than 2^-19 |la|)
+// exceeds thi - log(u).  thi < 0 always: |la| > band.  Hence
+//   thi < diff  => accept,   thi - diff >= lim  => reject,
+// and only 0 <= thi - diff < lim needs the exact log.
+__device__ static inline float acclog_screen(uint32_t r)
+{
+    const float u = (float)(1u | (r >> 8)) * 0x1p-24f;
+    return __builtin_fmaf(__builtin_amdgcn_logf(u), 0x1.62e430p-1f * (1.0f - ACCLOG_FAST_REL),
+                          ACCLOG_FAST_ABS);
+}
+
+__device__ static inline float acclog_screen_lim(float thi)
+{
+    return __builtin_fmaf(thi, -4.0f * ACCLOG_FAST_REL, 4.0f * ACCLOG_FAST_ABS);
+}
+
 // device: copy the 128-entry table into LDS (invc at dst[0..127], logc at dst[128..255])
 __device__ static inline void acclog_table_to_lds(double *dst, int tid, int nthreads)
 {

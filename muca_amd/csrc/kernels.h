@@ -54,7 +54,6 @@ hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a);
 struct TeamLayout {
     uint32_t row;         // L/2 attempts per half-row
     uint32_t team_bytes;  // per-team Philox ring and ln W window
-    uint32_t off_fde;     // (T)(-dE * beta) for dE = -8 .. 8
     uint32_t ring;        // Philox blocks per key held in a team's ring
     uint32_t off_win;     // inside a team's area: its ln W window (ln W in HBM)
     uint32_t off_mom;     // inside a team's area: its per-D moment slots (moments)

@@ -31,24 +31,23 @@ bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
     // them; then the team's ln W window
     lay.ring = (uint32_t)((row < 64 ? row : 64) / 4 + 8);
     lay.off_win = (uint32_t)al(2 * (size_t)lay.ring * 16);
-    lay.team_bytes = (uint32_t)(lay.off_win + al((kWin + 2) * tsz));
     // per-D moments (produce path, FP64): the team's window of moment slots;
     // they replace the D histogram
     const bool moms = fp64 && a.moms != nullptr && a.joint == nullptr;
-    lay.off_mom = lay.team_bytes;
-    if (moms) lay.team_bytes += (uint32_t)(kMomLdsWords * kMomSlots * sizeof(uint64_t));
+    const size_t mbytes = moms ? kMomLdsWords * kMomSlots * sizeof(uint64_t) : 0;
+    const size_t fixed = 256 * sizeof(double);   // the acceptance-log table
+    // ln W in LDS when it fits (with the guards), else read from HBM, where it
+    // stays in L2 (512 KB at L = 256 in FP64), one window per team at a time
+    const size_t wbytes = al((a.N + 1 + 2 * kGuard) * tsz);
+    lay.lnw_global = al((lay.off_win + mbytes) * kTeams) + fixed + wbytes > lds_max;
+    lay.off_mom = (uint32_t)(lay.off_win + (lay.lnw_global ? al(kWinCache * tsz) : 0));
+    lay.team_bytes = (uint32_t)(lay.off_mom + mbytes);
     size_t off = 0;
     lay.off_team = 0;
     off += al((size_t)lay.team_bytes * kTeams);
     lay.off_tab = (uint32_t)off;
-    off += 256 * sizeof(double);
-    lay.off_fde = (uint32_t)off;
-    off += al(17 * tsz);
+    off += fixed;
     lay.off_w = (uint32_t)off;
-    // ln W in LDS when it fits (with the guards), else read from HBM, where it
-    // stays in L2 (512 KB at L = 256 in FP64), one window per team at a time
-    const size_t wbytes = al((a.N + 1 + 2 * kGuard) * tsz);
-    lay.lnw_global = off + wbytes > lds_max;
     if (!lay.lnw_global) off += wbytes;
     // histogram and lattice in LDS when they fit (histogram first)
     const bool hist_fits = !moms && off + al((a.N + 1) * 4) <= lds_max;
@@ -65,6 +64,8 @@ bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
     lay.lat_lds = off + al((size_t)stride * kTeams) <= lds_max;
     if (lay.lat_lds) off += al((size_t)stride * kTeams);
     lay.bytes = off;
+    // lattices in HBM are addressed by a 32-bit offset within a row
+    if (!lay.lat_lds && (uint64_t)a.L * a.W > 0xffffffffull) return false;
     return off <= lds_max;
 }
 

@@ -8,24 +8,28 @@
 // a half-row of L/2 same-parity sites contains no two neighbours, and every
 // neighbour of a half-row was last written by an earlier half-row.  So per
 // chunk of a half-row (up to 64 attempts) the team
-//   A. computes in parallel, attempt j on lane j % 16: the Philox blocks,
-//      the proposed spin, dE, dDel, (T)(-dE*beta) and, for each of a window
-//      of 8 (weight path) or 6 (produce path) D values around the D the chunk
-//      starts from, whether the attempt accepts there (one byte each),
-//      screened with the hardware log (the exact log only where the screen
-//      is inconclusive);
-//   B. resolves the D chain: an attempt is a map of window positions, eight
-//      bytes wide, and v_perm_b32 looks four of them up at once, so sixteen
-//      lanes' maps compose in a prefix scan of four DPP steps and only one
-//      lookup per round of sixteen attempts depends on the D before it.  A
-//      round that starts outside the window, or leaves it, gets the masks of
-//      its undecided attempts recomputed around the D reached;
+//   A. computes in parallel, attempt j on lane j % 16 of round j / 16: the
+//      Philox blocks, the proposed spin, dE, dDel, (T)(-dE*beta) and the
+//      screened log of r1, for all rounds of the chunk at once;
+//   B. resolves the D chain round by round: for each of a window of 8 (weight
+//      path) or 6 (produce path) D values around the one the round starts at,
+//      whether the attempt accepts there (one byte each; the exact log only
+//      where the screen is inconclusive).  An attempt is then a map of window
+//      positions, eight bytes wide; v_perm_b32 looks four of them up at once,
+//      so sixteen lanes' maps compose in a prefix scan of four DPP steps.
+//      Where D leaves the window, the steps after that are done again around
+//      the D reached;
 //   C. writes the accepted spins, sums dE and dM and fills the histogram.
-// What the scan measured against a serial chain of one DPP broadcast, bit
-// extract and add per attempt: L = 72, 4096 walkers, from ln W = 0: 341 us per
-// launch against 381; L = 128, seeded, NUPDATES = N: 2.19 against 2.51 ms;
-// L = 72 thermalisation in FP64: 0.63 against 0.96 ms; L = 256, 16 384
-// walkers with moments: 15.8 against 19.5 ms.
+// Bound by one wavefront's issue and latency (a dependent VALU instruction
+// takes 8.6 cycles, an independent one 5.2, a branch 21 to 37).  Measured
+// against a serial chain of one DPP broadcast, bit extract and add per attempt
+// over masks made once per chunk: L = 72, 4096 walkers, from ln W = 0: 293 us
+// per launch against 381; L = 128, seeded, NUPDATES = N: 1.85 against 2.51 ms;
+// L = 72 thermalisation in FP64: 0.48 against 0.96 ms; L = 256, 16 384
+// walkers: 13.3 against 26.1 ms, with moments 15.0 against 19.5.  The scan
+// alone, over masks per chunk: 341 us, 2.19, 0.63, 15.5 and 15.8 ms: D leaves
+// a window of 8 around a chunk's start 0.2 to 1.3 times a round (L = 72 from
+// ln W = 0; seeded L = 128), one around the round's start 0.03 to 0.6 times.
 // Every acceptance is computed with the reference's operations and rounding:
 //   diff = ((T)(-dE*beta) + lnW[D+dDel]) - lnW[D];  accept iff diff >= 0 or
 //   acclog(r1) < diff.  Because acclog(r1) < 0 always, that is exactly
@@ -50,14 +54,11 @@ namespace team_detail {
 constexpr int kTeam = 16;
 constexpr int kTeams = 16;   // per workgroup of 256 lanes
 constexpr uint32_t kXcds = 8;   // accelerator dies of an MI355X, one L2 each
-// D values per acceptance mask (the most any launch uses).  Narrower
-// windows cut the mask work per attempt and make rounds in which D leaves
-// the window more frequent.  The weight path (D moves fast in the early
-// iterations from ln W = 0) uses 8: L = 72, 4096 walkers, 40.7 attempts/ns
-// per weight-loop step against 39.8 with 6.  The produce path (D drifts
-// slowly under near-flat weights) uses 6: L = 256, 16 384 walkers, 50.3
-// attempts/ns against 41.8 with 8.
-constexpr int kWin = 8;
+// D values per window (at most 8).  Narrower ones cut the mask work per pass and
+// make D leave them more often.  The weight path uses 8: L = 128, seeded 1.85
+// ms per launch against 1.90 with 6 and 2.03 with 4; L = 72 from ln W = 0 293,
+// 294 and 300 us.  The produce path (FP64 masks) uses 6: L = 256 with moments
+// 15.0 ms against 18.6 with 8, which spills; without 13.2 against 13.0.
 template <int KEYING>
 constexpr int kWinFor = KEYING == 1 ? 6 : 8;
 // Rounds per chunk where ln W is in HBM: those launches have 128 VGPRs (four
@@ -65,6 +66,7 @@ constexpr int kWinFor = KEYING == 1 ? 6 : 8;
 // 16 384 walkers, 65 536 attempts each, with moments / without: 15.8 / 15.5 ms
 // with two rounds, 16.8 / 16.1 with three, 18.5 / 16.0 with four.
 constexpr int kLnwgRounds = 2;
+constexpr int kWinCache = 64;   // ln W values per team in LDS where ln W is in HBM
 constexpr int kGuard = 24;   // ln W guard entries on each side (> kWin / 2 + 2)
 
 __device__ __forceinline__ void wave_sync()
@@ -106,6 +108,36 @@ __device__ __forceinline__ float mag_word(float x)
 __device__ __forceinline__ float mag_word(double x)
 {
     return __uint_as_float((uint32_t)(__double_as_longlong(x) >> 32));
+}
+
+// ---- proposals: new spin from the old one (-1, 0, 1) and the step's random
+// word (+1 below 2^31, else -1, wrapped into -1..1).  Bits 0-1 of a proposal
+// byte hold dDel + 1, 2-4 the spin change + 2, 5-6 the new spin + 1; the six
+// cases are the bytes of two dwords, indexed by old + 1 (+ 4 for a step down).
+// mds: minus the spin change.
+__device__ __forceinline__ void proposal_bytes(int32_t old_s, uint32_t r3, uint32_t &pr,
+                                               int32_t &mds)
+{
+    const uint32_t at = (uint32_t)old_s + 0x0c0c0c01u + ((r3 >> 29) & 4u);
+    pr = __builtin_amdgcn_perm(0x00240651u, 0x00014e2cu, at);
+    mds = (int32_t)(int8_t)__builtin_amdgcn_perm(0x000101feu, 0x0002ffffu, at);
+}
+// fields of an attempt's info word: a proposal byte and (dE + 8) << 8
+__device__ __forceinline__ int32_t i_ddel(int32_t i)
+{
+    return (i & 3) - 1;
+}
+__device__ __forceinline__ int32_t i_ds(int32_t i)
+{
+    return ((i >> 2) & 7) - 2;
+}
+__device__ __forceinline__ int32_t i_new(int32_t i)
+{
+    return ((i >> 5) & 3) - 1;
+}
+__device__ __forceinline__ int32_t i_dE(int32_t i)
+{
+    return (i >> 8) - 8;
 }
 
 // ---- maps of window positions, KW <= 8 positions as bytes 0..3 (lo), 4..7 (hi)
@@ -202,12 +234,11 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     uint32_t *hist = (uint32_t *)(lds + lay.off_hist);
     int8_t *latl = (int8_t *)(lds + lay.off_lat);
     double *logtab = (double *)(lds + lay.off_tab);
-    T *fdet = (T *)(lds + lay.off_fde) + 8;    // fdet[dE] = (T)(-dE * beta), |dE| <= 8
     const int tid = threadIdx.x, team = tid >> 4, tl = tid & 15;
     const uint32_t N = a.N, L = a.L, Rw = lay.row;
     unsigned char *tbase = lds + lay.off_team + (size_t)team * lay.team_bytes;
     uint32_t *rng = (uint32_t *)tbase;                          // [2][ring][4]
-    T *winb = (T *)(tbase + lay.off_win);                       // LNWG: lnW[dlo - 1 .. dlo + KW]
+    T *winb = (T *)(tbase + lay.off_win);                       // LNWG: lnW[wb .. wb + kWinCache - 1]
     // ln W at any D: from LDS, or from HBM (clamped into [0, N]; only
     // positions a walker cannot be at read a clamped value)
     auto lnw_at = [&](int32_t i) -> T {
@@ -237,7 +268,6 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     if (LDSHIST)
         for (uint32_t i = tid; i <= N; i += blockDim.x) hist[i] = a.hist_preload;
     acclog_table_to_lds(logtab, tid, blockDim.x);
-    if (tid < 17) fdet[tid - 8] = (T)(-(double)(tid - 8) * a.beta);
     // LATLDS: the tile's lattices move between the site-major layout in HBM
     // and walker-major LDS rows.  For sixteen whole walkers on 16-byte
     // aligned rows, a lane moves four consecutive sites at a time: four
@@ -278,8 +308,13 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     __syncthreads();
 
     if (active) {
-        auto sp = [&](uint32_t site) -> int8_t & {
-            return LATLDS ? latl[team * lay.lat_stride + site] : a.lat[(uint64_t)site * W + w];
+        // The walker's spin at x of a row: the row's address is the same in
+        // every lane where lattices are in HBM (one 32-bit offset per lane and
+        // x, site x W + w of a row; team_layout checks that it fits)
+        const uint32_t xw = LATLDS ? 1u : (uint32_t)W;
+        const uint32_t x0 = LATLDS ? team * lay.lat_stride : (uint32_t)w;
+        auto row_at = [&](uint32_t yy) -> int8_t * {
+            return LATLDS ? latl + yy * L : a.lat + (uint64_t)yy * ((uint64_t)L * W);
         };
         const uint32_t wid = a.w_offset + (uint32_t)w;
         const uint32_t k1a = KEYING == 0 ? 2u * wid : wid;
@@ -287,6 +322,9 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
         const uint32_t k3a = KEYING == 0 ? 2u * wid + 50000u : wid + 40000u;
         const uint32_t k3b = KEYING == 0 ? 0x11cafeadu : 0xdecafeadu;
         int32_t d = a.D[w], e = a.E[w], m = a.M[w];
+        // loaded before the loop, which would otherwise wait for them (and for
+        // every load after them) where it uses d
+        asm volatile("" : "+v"(d), "+v"(e), "+v"(m));
         uint64_t *jbase = nullptr;
         if (JOINT) jbase = a.joint + (w / a.block_walkers) * a.joint_stride;
         // MOMS: the walker's production attempts are summed per D in the
@@ -336,6 +374,21 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
         int32_t pf_s[NR], pf_r[NR], pf_l[NR], pf_u[NR], pf_d[NR], fin[NR];
         bool pf_have = false, pf_fwd = false;
         int32_t de_lane = 0, dm_lane = 0;
+        // lnW[dc - KW/2 + k] at [k], k = -1 .. KW.  LNWG: from the team's
+        // window of kWinCache values in LDS, staged again around dc when it
+        // does not hold them
+        int32_t wb = -(1 << 30);
+        auto window = [&](int32_t dc) -> const T * {
+            if (!LNWG) return wt + dc - KW / 2;
+            if (dc - KW / 2 - 1 < wb || dc + KW / 2 >= wb + kWinCache) {
+                wb = dc - kWinCache / 2;
+#pragma unroll
+                for (int i = 0; i < kWinCache / kTeam; i++)
+                    winb[kTeam * i + tl] = lnw_at(wb + kTeam * i + (int32_t)tl);
+                wave_sync();
+            }
+            return winb + (dc - KW / 2 - wb);
+        };
         // the scan's shifted-in maps per level: the lanes that have no source
         // lane at a level keep the identity from here on
         uint32_t ql[4], qh[4];
@@ -345,6 +398,21 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
             qh[k] = window_id<KW>(1);
         }
         // a workgroup adds at most 16 NUPDATES counts to one u32 bin
+        // this lane's sites in a row for a chunk of half h from jb on, and
+        // their right and left neighbours; they stay from row to row
+        uint32_t sx[NR], sxr[NR], sxl[NR], sx_h = ~0u, sx_jb = ~0u;
+        auto sites = [&](uint32_t sh, uint32_t sj) {
+            const uint32_t last = min(Rw - sj, 16u * NR) - 1;
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                const uint32_t x = 2 * (sj + min(16u * r + tl, last)) + sh;
+                sx[r] = x0 + x * xw;
+                sxr[r] = x0 + ((x + 1 == L) ? 0 : x + 1) * xw;
+                sxl[r] = x0 + ((x == 0) ? L - 1 : x - 1) * xw;
+            }
+            sx_h = sh;
+            sx_jb = sj;
+        };
         const bool may_wrap = a.hist_preload != 0 || (uint64_t)kTeams * a.nup >= (1ull << 32);
         for (int phase = 0; phase < 2; phase++) {
             const uint64_t n = phase ? a.nup : a.therm;
@@ -385,105 +453,60 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 cur_slot = cur_slot + nblk >= RB ? cur_slot + nblk - RB : cur_slot + nblk;
                 wave_sync();
                 // ---- A2: attempt j = 16 r + tl on this lane, everything in registers
-                int32_t dlo = d - KW / 2;           // mask bit k <-> D = dlo + k
-                // lnW[dlo + k] at wcen[k], k = -1 .. KW (LNWG: staged in the
-                // team's window from HBM)
-                auto window = [&]() -> const T * {
-                    if (LNWG) {
-                        if (tl < KW + 2) winb[tl] = lnw_at(dlo - 1 + tl);
-                        wave_sync();
-                        return winb + 1;
-                    }
-                    return wt + dlo;
-                };
-                const T *wcen = window();
-                T wfrom[KW];                        // lnW[dlo .. dlo + KW - 1]
-#pragma unroll
-                for (int k = 0; k < KW; k++) wfrom[k] = wcen[k];
-                const int32_t dlo_a = dlo;            // the window of every mask made here
-                const uint32_t yu = (y + 1 == L) ? 0 : y + 1, yd = (y == 0) ? L - 1 : y - 1;
+                int8_t *const row = row_at(y);
                 const uint32_t s4 = slot0 * 4, ringw = RB * 4;   // ring word of attempt j: s4 + j (mod ringw)
-                // attempt j's accept bytes: byte k is 0xff iff it accepts at
-                // D = dlo_a + k (bytes 0..3, 4..7)
-                uint32_t alo[NR], ahi[NR];
-                // (dDel + 1) | (dE + 8) << 2 | (new - old + 2) << 7 | (new + 1) << 10
+                // the proposal: kDdel, kDs, kNew (proposal_bytes) and dE + 8
+                // in bits 8..12
                 int32_t info[NR];
-                // Byte k = 0..KW-1: accept at D = dlo + k, i.e. acclog(r1) <
-                // ((fde + lnW[D + dDel]) - lnW[D]), screened with the hardware
-                // log and its proven band: la + band < diff accepts, la - band
-                // >= diff rejects.  Byte k is the sign of e = thi - diff (e is
-                // -0 never, +0 iff thi == diff, which rejects); a diff with
-                // tlo < diff <= thi, i.e. 0 <= e < thi - tlo, needs the exact
-                // log -- flagged (with margin) by min |e| < 2 (thi - tlo).
-                // The minimum is taken over mag_word (exact in FP32, the high
-                // words in FP64, compared there with <=).  An attempt past the
-                // chunk's end has fde = -inf and accepts nowhere.
-                auto accept_bytes = [&](const T *wf, const T *wc, uint32_t r1, T fde,
-                                        int32_t ddel, uint32_t &lo, uint32_t &hi) {
-                    const T *wto = wc + ddel;
-                    T diff[KW];
+                // Every load of the chunk's spins and random words first, then
+                // the proposals, without a branch between the rounds: one
+                // wavefront per SIMD hides no latency of its own.
+                // A lane past the end of the chunk works on an in-bounds
+                // attempt and keeps nothing of it.
+                if (LNWG || h != sx_h || jb != sx_jb) sites(h, jb);
+                uint32_t cx[NR];   // this chunk's sites (sx may move on to the next one's)
 #pragma unroll
-                    for (int k = 0; k < KW; k++) {
-                        diff[k] = fde + wto[k];
-                        diff[k] = diff[k] - wf[k];
-                    }
-                    const float la = acclog_fast_u01(r1);
-                    const float band = acclog_fast_band(la);
-                    const T thi = (T)(la + band), tlo = (T)(la - band);
-                    uint32_t sg[8];
-                    float emin = 1e30f;
+                for (int r = 0; r < NR; r++) cx[r] = sx[r];
+                int32_t old_s[NR], nb[NR];
+                uint32_t r1[NR], r3[NR];
+                float thi[NR];   // the screened log of r1 (acclog_screen)
+                if (PF && pf_have) {
 #pragma unroll
-                    for (int k = 0; k < KW; k++) {
-                        const T e = thi - diff[k];
-                        sg[k] = sign_word(e);
-                        emin = fminf(emin, fabsf(mag_word(e)));
+                    for (int r = 0; r < NR; r++) {
+                        old_s[r] = pf_s[r];
+                        nb[r] = pf_r[r] + pf_l[r] + pf_u[r] +
+                                ((pf_fwd && fin[r] != -9) ? fin[r] : pf_d[r]);
                     }
-                    sign_bytes<KW>(sg, lo, hi);
-                    const float lim = mag_word((thi - tlo) + (thi - tlo));
-                    const bool amb = FP64 ? emin <= lim : emin < lim;
-                    if (__builtin_amdgcn_ballot_w64(amb)) {   // rare: a diff within the band
-                        if (amb) {
-                            const T tlog =
-                                (T)(float)acclog_u01_double_tab(r1, logtab, logtab + 128);
+                } else {
+                    const int8_t *up = row_at((y + 1 == L) ? 0 : y + 1);
+                    const int8_t *dn = row_at((y == 0) ? L - 1 : y - 1);
 #pragma unroll
-                            for (int k = 0; k < KW; k++) sg[k] = tlog < diff[k] ? 0x80000000u : 0u;
-                            sign_bytes<KW>(sg, lo, hi);
-                        }
+                    for (int r = 0; r < NR; r++) {
+                        old_s[r] = row[sx[r]];
+                        nb[r] = row[sxr[r]] + row[sxl[r]] + up[sx[r]] + dn[sx[r]];
                     }
-                };
-                // Branch-free over the rounds so that the loads of all rounds
-                // can be in flight together: a lane past the end of the
-                // chunk works on a clamped (in-bounds) attempt and keeps
-                // nothing of it.
+                }
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
-                    const uint32_t j = 16 * r + tl;
-                    const bool valid = j < cnt;
-                    const uint32_t jc = valid ? j : cnt - 1;
-                    const uint32_t x = 2 * (jb + jc) + h;
-                    const uint32_t xr = (x + 1 == L) ? 0 : x + 1;
-                    const uint32_t xl = (x == 0) ? L - 1 : x - 1;
-                    int32_t old_s, nb;
-                    if (PF && pf_have) {
-                        old_s = pf_s[r];
-                        nb = pf_r[r] + pf_l[r] + pf_u[r] + ((pf_fwd && fin[r] != -9) ? fin[r] : pf_d[r]);
-                    } else {
-                        old_s = sp(y * L + x);
-                        nb = sp(y * L + xr) + sp(y * L + xl) + sp(yu * L + x) + sp(yd * L + x);
-                    }
-                    uint32_t widx = s4 + jc;
+                    uint32_t widx = s4 + 16 * r + tl;
                     widx = widx >= ringw ? widx - ringw : widx;
-                    const uint32_t r1 = rng[widx], r3 = rng[ringw + widx];
-                    int32_t new_s = old_s + (r3 < 0x80000000u ? 1 : -1);
-                    new_s = new_s == 2 ? -1 : (new_s == -2 ? 1 : new_s);
-                    const int32_t ds = new_s - old_s;
-                    const int32_t dE = -ds * nb;
-                    const int32_t ddel = new_s * new_s - old_s * old_s;
-                    // (T)(-dE * beta) by arithmetic (the same operations as
-                    // the table in LDS, without a dependent LDS load)
-                    const T fde = (T)(-(double)dE * a.beta);
-                    accept_bytes(wfrom, wcen, r1, valid ? fde : -(T)INFINITY, ddel, alo[r], ahi[r]);
-                    info[r] = (ddel + 1) | ((dE + 8) << 2) | ((ds + 2) << 7) | ((new_s + 1) << 10);
+                    r1[r] = rng[widx];
+                    r3[r] = rng[ringw + widx];
+                }
+                T fde[NR];
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    uint32_t pr;
+                    int32_t mds;
+                    proposal_bytes(old_s[r], r3[r], pr, mds);
+                    thi[r] = acclog_screen(r1[r]);
+                    const int32_t dE = __mul24(mds, nb[r]);
+                    info[r] = (int32_t)pr | ((dE + 8) << 8);
+                    // past the chunk's end: -inf accepts nowhere
+                    fde[r] = 16 * r + (uint32_t)tl < cnt ? (T)(-(double)dE * a.beta) : -(T)INFINITY;
+                    // made here, not where the round uses them: that would put
+                    // their latency into the chain
+                    asm volatile("" : "+v"(info[r]), "+v"(fde[r]), "+v"(thi[r]));
                 }
                 wave_sync();
                 if (PF) {
@@ -525,115 +548,115 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     pf_have = have;
                     pf_fwd = fwd;
                     if (have) {
+                        if (h_n != sx_h || jb_n != sx_jb) sites(h_n, jb_n);
+                        const int8_t *row_n = row_at(y_n), *up_n = row_at(yu_n),
+                                     *dn_n = row_at(yd_n);
 #pragma unroll
                         for (int r = 0; r < NR; r++) {
-                            const uint32_t jn = min(16u * r + tl, cnt_n - 1);
-                            const uint32_t x = 2 * (jb_n + jn) + h_n;
-                            const uint32_t xr = (x + 1 == L) ? 0 : x + 1;
-                            const uint32_t xl = (x == 0) ? L - 1 : x - 1;
-                            pf_s[r] = sp(y_n * L + x);
-                            pf_r[r] = sp(y_n * L + xr);
-                            pf_l[r] = sp(y_n * L + xl);
-                            pf_u[r] = sp(yu_n * L + x);
-                            pf_d[r] = sp(yd_n * L + x);
+                            pf_s[r] = row_n[sx[r]];
+                            pf_r[r] = row_n[sxr[r]];
+                            pf_l[r] = row_n[sxl[r]];
+                            pf_u[r] = up_n[sx[r]];
+                            pf_d[r] = dn_n[sx[r]];
                         }
                     }
                 }
-                // ---- B: the D chain.  Attempt j maps the window position k =
-                // D - dlo before it to the one after it: k + dDel where byte k
-                // of its accept bytes is set, else k; a position outside the
-                // window is 0xff and stays so.  A map is eight bytes, and
-                // v_perm_b32 looks up four of them at once (a selector of 0xff
-                // gives 0xff), so that two maps compose in two instructions
-                // and sixteen lanes' maps in a prefix scan of four levels.  The
-                // scans of all rounds are independent of D and of each other;
-                // only one lookup per round depends on the D the round before
-                // ended at.
+                // ---- B: the D chain, round by round.  A window of KW values
+                // of D around the one the round starts at, dlo .. dlo + KW - 1:
+                // attempt j maps the window position k = D - dlo before it to
+                // the one after it, k + dDel where it accepts at dlo + k and
+                // else k; a position outside the window is 0xff and stays so.
+                // A map is eight bytes, and v_perm_b32 looks up four of them
+                // at once (a selector of 0xff gives 0xff), so that two maps
+                // compose in two instructions and sixteen lanes' maps in a
+                // prefix scan of four levels.
                 const uint32_t sh = (uint32_t)(tid & 48);    // this team's 16 lanes of a ballot
                 const uint32_t upto = (2u << tl) - 1u;       // steps 0..tl of a round
-                // made ahead of the rounds where registers allow
-                constexpr bool AHEAD = !LNWG;
-                auto scan = [&](uint32_t lo, uint32_t hi, int32_t inf, uint32_t &plo,
-                                uint32_t &phi) {
-                    window_map<KW>(lo, hi, (uint32_t)inf, plo, phi);
-                    if (!AHEAD)
-#pragma unroll
-                        for (int k = 0; k < 4; k++) {
-                            ql[k] = window_id<KW>(0);
-                            qh[k] = window_id<KW>(1);
-                        }
-                    scan_level<KW, 0x111>(plo, phi, ql[0], qh[0]);
-                    scan_level<KW, 0x112>(plo, phi, ql[1], qh[1]);
-                    scan_level<KW, 0x114>(plo, phi, ql[2], qh[2]);
-                    scan_level<KW, 0x118>(plo, phi, ql[3], qh[3]);
-                };
-                // the maps of steps 0..tl of each round
-                uint32_t plo[NR], phi[NR];
-                if (AHEAD)
-#pragma unroll
-                    for (int r = 0; r < NR; r++) scan(alo[r], ahi[r], info[r], plo[r], phi[r]);
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
                     const uint32_t j0 = 16 * r;
                     if (PF) fin[r] = -9;
                     if (j0 >= cnt) continue;
-                    if (!AHEAD) scan(alo[r], ahi[r], info[r], plo[r], phi[r]);
                     const bool valid = j0 + tl < cnt;
-                    // the window's accept bytes recomputed around dlo by all
-                    // lanes of the team; steps below `from` are decided and
-                    // become identities
-                    auto remask = [&](uint32_t from) {
-                        const T *wc = window();
-                        T wf[KW];
+                    // The window around D = dc before step `from` of the round;
+                    // the steps before it are identities (fde = -inf accepts
+                    // nowhere).  Byte k of (lo, hi): accept at dlo + k, i.e.
+                    // acclog(r1) < ((fde + lnW[dlo + k + dDel]) - lnW[dlo + k]),
+                    // screened: the sign of e = thi - diff (e is -0 never); a
+                    // diff with 0 <= e < lim needs the exact log -- flagged by
+                    // min |e| < lim, the minimum taken over mag_word (exact in
+                    // FP32, the high words in FP64, compared there with <=).
+                    // o: the window position after this lane's step; before:
+                    // the one before it; ok: accepted there.
+                    auto pass = [&](int32_t dc, uint32_t from, uint32_t &o, uint32_t &before,
+                                    bool &ok) {
+                        const T *wc = window(dc);
+                        const T *wto = wc + i_ddel(info[r]);
+                        const T fd = (uint32_t)tl >= from ? fde[r] : -(T)INFINITY;
+                        T diff[KW];
 #pragma unroll
-                        for (int k = 0; k < KW; k++) wf[k] = wc[k];
-                        uint32_t w1 = s4 + min(j0 + tl, cnt - 1);
-                        w1 = w1 >= ringw ? w1 - ringw : w1;
-                        const T fde = fdet[((info[r] >> 2) & 31) - 8];
-                        accept_bytes(wf, wc, rng[w1], valid && tl >= from ? fde : -(T)INFINITY,
-                                     (info[r] & 3) - 1, alo[r], ahi[r]);
-                        scan(alo[r], ahi[r], info[r], plo[r], phi[r]);
-                    };
-                    // the window follows D from round to round: a round that
-                    // starts outside the masks' window gets its masks
-                    // recomputed around the current D (only this round's: the
-                    // later rounds' stay relative to dlo_a)
-                    dlo = dlo_a;
-                    uint32_t off = (uint32_t)(d - dlo_a);
-                    const bool shift = off >= (uint32_t)KW;
-                    if (__builtin_amdgcn_ballot_w64(shift)) {
-                        if (shift) {
-                            dlo = d - KW / 2;
-                            off = KW / 2;
-                            remask(0);
+                        for (int k = 0; k < KW; k++) {
+                            diff[k] = fd + wto[k];
+                            diff[k] = diff[k] - wc[k];
                         }
-                    }
-                    uint32_t o = window_at(plo[r], phi[r], off);
-                    uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(
-                        (int)off, (int)o, 0x111, 0xf, 0xf, false);
-                    // this lane's attempt: accepted, and D (and M) after it
-                    bool acc = window_at(alo[r], ahi[r], before) != 0;
-                    int32_t dv = dlo + (int32_t)o, mv = 0;
-                    // Rare: D left the window at step k.  Steps 0..k stand (step
-                    // k is accepted and moved D by its dDel); the masks of the
-                    // later ones are recomputed around D there, and so on until
-                    // the round is done.  k grows by KW / 2 at least each time.
+                        uint32_t sg[8], lo, hi;
+                        float emin = 1e30f;
+                        const T th = (T)thi[r];
+#pragma unroll
+                        for (int k = 0; k < KW; k++) {
+                            const T e = th - diff[k];
+                            sg[k] = sign_word(e);
+                            emin = fminf(emin, fabsf(mag_word(e)));
+                        }
+                        sign_bytes<KW>(sg, lo, hi);
+                        const float lim = mag_word((T)acclog_screen_lim(thi[r]));
+                        const bool amb = FP64 ? emin <= lim : emin < lim;
+                        if (__builtin_amdgcn_ballot_w64(amb)) {   // rare
+                            if (amb) {
+                                uint32_t w1 = s4 + j0 + tl;
+                                w1 = w1 >= ringw ? w1 - ringw : w1;
+                                const T tlog = (T)(float)acclog_u01_double_tab(rng[w1], logtab,
+                                                                               logtab + 128);
+#pragma unroll
+                                for (int k = 0; k < KW; k++)
+                                    sg[k] = tlog < diff[k] ? 0x80000000u : 0u;
+                                sign_bytes<KW>(sg, lo, hi);
+                            }
+                        }
+                        uint32_t plo, phi;   // the map of steps 0..tl
+                        window_map<KW>(lo, hi, (uint32_t)info[r], plo, phi);
+                        scan_level<KW, 0x111>(plo, phi, ql[0], qh[0]);
+                        scan_level<KW, 0x112>(plo, phi, ql[1], qh[1]);
+                        scan_level<KW, 0x114>(plo, phi, ql[2], qh[2]);
+                        scan_level<KW, 0x118>(plo, phi, ql[3], qh[3]);
+                        o = window_at(plo, phi, KW / 2);
+                        before = (uint32_t)__builtin_amdgcn_update_dpp(KW / 2, (int)o, 0x111, 0xf,
+                                                                       0xf, false);
+                        ok = window_at(lo, hi, before) != 0;
+                    };
+                    uint32_t o, before;
+                    bool acc;   // this lane's attempt: accepted, and D (and M) after it
+                    pass(d, 0, o, before, acc);
+                    int32_t dlo = d - KW / 2, dv = dlo + (int32_t)o, mv = 0;
+                    // D left the window at step k: steps 0..k stand (step k is
+                    // accepted and moved D by its dDel), and the window moves
+                    // to D after it for the later ones, until the round is
+                    // done.  k grows by KW / 2 at least each time.
                     uint64_t outs;
                     bool out = o == 0xffu;
                     while ((outs = __builtin_amdgcn_ballot_w64(out)) != 0) {
                         const uint32_t mine = (uint32_t)(outs >> sh) & 0xffffu;
                         if (mine) {
                             const uint32_t k = (uint32_t)__builtin_ctz(mine);
-                            const int32_t dk = dlo + (int32_t)before + (info[r] & 3) - 1;
+                            const int32_t dk = dlo + (int32_t)before + i_ddel(info[r]);
                             if ((uint32_t)tl == k) dv = dk;
-                            dlo = __shfl(dk, (int)k, kTeam) - KW / 2;
-                            remask(k + 1);
-                            o = window_at(plo[r], phi[r], KW / 2);
-                            before = (uint32_t)__builtin_amdgcn_update_dpp(
-                                KW / 2, (int)o, 0x111, 0xf, 0xf, false);
+                            const int32_t dc = __shfl(dk, (int)k, kTeam);
+                            dlo = dc - KW / 2;
+                            bool ok;
+                            pass(dc, k + 1, o, before, ok);
                             out = o == 0xffu;
                             if ((uint32_t)tl > k) {
-                                acc = window_at(alo[r], ahi[r], before) != 0;
+                                acc = ok;
                                 dv = dlo + (int32_t)o;
                             }
                         }
@@ -642,7 +665,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     if (TRACKM) {
                         // M after this lane's step: an inclusive scan over the
                         // team of the accepted spin changes
-                        int32_t x = acc ? ((info[r] >> 7) & 7) - 2 : 0;
+                        int32_t x = acc ? i_ds(info[r]) : 0;
                         x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
                         x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
                         x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
@@ -652,15 +675,14 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     }
                     // ---- C: accepted spins, dE / dM sums, histogram of the round
                     const uint32_t j = j0 + tl, left = min(cnt - j0, 16u);
-                    const int32_t ns = ((info[r] >> 10) & 3) - 1;    // the proposed spin
-                    const int32_t ds = ((info[r] >> 7) & 7) - 2;
+                    const int32_t ns = i_new(info[r]), ds = i_ds(info[r]);   // the proposal
                     // the site's spin after this chunk
                     if (PF) fin[r] = valid ? (acc ? ns : ns - ds) : -9;
                     if (acc) {
                         // the new spin is known from phase A: no site of
                         // the chunk is written between its read and here
-                        sp(y * L + 2 * (jb + j) + h) = (int8_t)ns;
-                        de_lane += ((info[r] >> 2) & 31) - 8;
+                        row[cx[r]] = (int8_t)ns;
+                        de_lane += i_dE(info[r]);
                         dm_lane += ds;
                     }
                     if (JOINT && phase && valid) {
@@ -689,7 +711,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                         // starting at step 0 and at every accepted step that
                         // changed D; the first lane of a run adds its length (one
                         // atomic per run instead of sixteen on the same bin)
-                        const bool moved = acc && (info[r] & 3) != 1;
+                        const bool moved = acc && i_ddel(info[r]) != 0;
                         const uint32_t starts =
                             ((uint32_t)(__builtin_amdgcn_ballot_w64(moved) >> sh) & 0xffffu) | 1u;
                         const uint32_t later = starts & ~upto;
