@@ -44,7 +44,7 @@ extern "C" {
  * compute unit and the layout; muca_autotune chooses by measurement) */
 #define MUCA_KERNEL_AUTO 0
 #define MUCA_KERNEL_GENERIC 1  /* one lane per walker, reference site order from tables */
-#define MUCA_KERNEL_TEAM 2     /* sixteen lanes per walker (L % 8 == 0, L <= 256; lattices and
+#define MUCA_KERNEL_TEAM 2     /* sixteen lanes per walker (even L, 8 <= L <= 256; lattices and
                                   ln W in LDS when they fit) */
 #define MUCA_KERNEL_LANE 3     /* one lane per walker, even L, table-free, screened acceptance */
 
@@ -241,8 +241,8 @@ typedef struct muca_instance_status {
 } muca_instance_status;
 
 const char *muca_batch_last_error(void);
-/* tiles: MUCA_KERNEL_AUTO, MUCA_KERNEL_TEAM (every L % 8 == 0, L <= 128) or
- * MUCA_KERNEL_LANE; precision: MUCA_REF32 | MUCA_FP64.  Lane tiles hold
+/* tiles: MUCA_KERNEL_AUTO (team tiles for few walkers where every L is in
+ * [8, 128]), MUCA_KERNEL_TEAM (every L % 8 == 0, L <= 128) or MUCA_KERNEL_LANE; precision: MUCA_REF32 | MUCA_FP64.  Lane tiles hold
  * 256 walkers, or 512 / 1024 when the largest instance's ln W and histogram
  * leave LDS room for only a few workgroups per compute unit (the autotuner
  * may choose otherwise). */

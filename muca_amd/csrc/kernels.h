@@ -63,7 +63,7 @@ struct TeamLayout {
     bool lds_hist, lat_lds;
     bool lnw_global;      // ln W too large for LDS: read from HBM (L2) per window
 };
-// false when the team kernel cannot run this launch (L % 8 != 0 or L > 256)
+// false when the team kernel cannot run this launch (odd L, L < 8 or L > 256)
 bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay);
 hipError_t launch_mcs_team(hipStream_t st, const Launch &cfg, const McsArgs &a,
                            const TeamLayout &lay);

@@ -466,7 +466,7 @@ int muca_batch_create(int32_t device, const muca_instance *ins, uint32_t n, int3
     b->device = device;
     b->fp64 = precision == MUCA_FP64;
     b->cus = (uint32_t)cu;
-    bool team_ok = true, lane_ok = true;
+    bool team_ok = true, team_ask = true, lane_ok = true;
     uint64_t lat = 0, st = 0, wo = 0;
     for (uint32_t i = 0; i < n; i++) {
         const muca_instance &q = ins[i];
@@ -490,9 +490,10 @@ int muca_batch_create(int32_t device, const muca_instance *ins, uint32_t n, int3
         a.L = I.L;
         a.W = I.W;
         a.nup = 1;
-        if (!(I.L % 8 == 0 && I.L <= 128 && muca::team_layout(a, b->fp64, lds_budget, I.lay) &&
+        if (!(I.L <= 128 && muca::team_layout(a, b->fp64, lds_budget, I.lay) &&
               !I.lay.lnw_global))
             team_ok = false;
+        if (I.L % 8 != 0) team_ask = false;   // team tiles on request: multiples of 8 only
         const size_t tsz = b->fp64 ? 8 : 4;
         I.lane_lds_w = (uint32_t)(((I.N + 1) * tsz + 15) & ~(size_t)15);
         I.lane_hist = I.lane_lds_w + (size_t)(I.N + 1) * 4 <= lds_budget;
@@ -506,7 +507,7 @@ int muca_batch_create(int32_t device, const muca_instance *ins, uint32_t n, int3
     b->team_ok = team_ok;
     b->lane_ok = lane_ok;
     b->lds_device = (size_t)lds;
-    if (tiles == MUCA_KERNEL_TEAM && !team_ok) {
+    if (tiles == MUCA_KERNEL_TEAM && !(team_ok && team_ask)) {
         batch_free(b);
         return bfail(MUCA_E_ARG, "team tiles need every L % 8 == 0 and L <= 128");
     }

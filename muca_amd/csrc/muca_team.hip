@@ -21,15 +21,16 @@ MUCA_TEAM_EXTERN(10, true, 1)
 
 bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
 {
-    if (a.L % 8 != 0 || a.L > 256) return false;
+    if (a.L % 2 != 0 || a.L < 8 || a.L > 256) return false;
     const size_t tsz = fp64 ? 8 : 4;
     const size_t row = a.L / 2;
     auto al = [](size_t x) { return (x + 15) & ~(size_t)15; };
     lay.row = (uint32_t)row;
-    // Philox ring: a chunk of a half-row (at most 64 attempts) needs chunk/4
-    // blocks per key and a generation pass may run up to 7 blocks ahead of
-    // them; then the team's ln W window
-    lay.ring = (uint32_t)((row < 64 ? row : 64) / 4 + 8);
+    // Philox ring: a chunk of a half-row (at most 64 attempts, starting at any
+    // of a block's four words) touches (chunk + 6) / 4 blocks per key at most
+    // and a generation pass may run up to 7 blocks ahead of them; then the
+    // team's ln W window
+    lay.ring = (uint32_t)(((row < 64 ? row : 64) + 6) / 4 + 8);
     lay.off_win = (uint32_t)al(2 * (size_t)lay.ring * 16);
     // per-D moments (produce path, FP64): the team's window of moment slots;
     // they replace the D histogram

@@ -34,9 +34,10 @@
 //   diff = ((T)(-dE*beta) + lnW[D+dDel]) - lnW[D];  accept iff diff >= 0 or
 //   acclog(r1) < diff.  Because acclog(r1) < 0 always, that is exactly
 //   acclog(r1) < diff.  Results are bit-identical to the one-lane kernel.
-// Requires L % 8 == 0 (whole Philox blocks per half-row) and L <= 256.
+// Requires even L, 8 <= L <= 256.  A half-row need not be a whole number of
+// Philox blocks: a chunk starts at word rs % 4 of its first block.
 //
-// LDS (dynamic): per team a ring of Philox blocks [2 keys][min(L/2, 64)/4 + 8][4]; the
+// LDS (dynamic): per team a ring of Philox blocks [2 keys][(min(L/2, 64) + 6)/4 + 8][4]; the
 // acceptance-log table; (T)(-dE*beta) for dE = -8..8; ln W with guard entries
 // on each side; the D histogram (u32, when it fits); the workgroup's lattices
 // [N][16] int8 (when they fit).
@@ -276,7 +277,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     // walker); a lane's four loads are all in flight before the first is
     // used.  Otherwise one byte per lane and step.
     const bool lat_vec = LATLDS && W % kTeams == 0 && wbase + kTeams <= W &&
-                         ((uintptr_t)a.lat & 15) == 0;   // N % 64 == 0 (L % 8 == 0)
+                         ((uintptr_t)a.lat & 15) == 0;   // N % 4 == 0 (even L)
     if (LATLDS) {
         if (lat_vec) {
             for (uint32_t q = tid; q < N / 4; q += blockDim.x) {
@@ -431,7 +432,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 // multiple of eight.  Blocks [blk0, blk0 + nblk) serve this
                 // chunk; a pass may run up to 7 blocks ahead, and RB >= nblk + 8
                 // keeps those from overwriting blocks still in use.
-                const uint32_t nblk = (cnt + 3) / 4;
+                const uint32_t wo = (uint32_t)rs & 3u, nblk = (wo + cnt + 3) / 4;
                 const uint32_t blk0 = c0base + (uint32_t)(rs / 4);
                 while (gen < blk0 + nblk) {
                     const uint32_t b = gen + (uint32_t)(tl >> 1), key = tl & 1;
@@ -447,14 +448,17 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     gen += 8;
                     gen_slot = gen_slot + 8 >= RB ? gen_slot + 8 - RB : gen_slot + 8;
                 }
-                // ring slot of this chunk's first block (blocks are contiguous
-                // from one chunk to the next, across the phase change too)
+                // ring slot of this chunk's first block; the next chunk starts
+                // in this one's last block unless that is used up or the
+                // phase ends (a phase starts with a block of its own)
                 const uint32_t slot0 = cur_slot;
-                cur_slot = cur_slot + nblk >= RB ? cur_slot + nblk - RB : cur_slot + nblk;
+                cur_slot += rs + cnt == n ? nblk : (wo + cnt) / 4;
+                cur_slot = cur_slot >= RB ? cur_slot - RB : cur_slot;
                 wave_sync();
                 // ---- A2: attempt j = 16 r + tl on this lane, everything in registers
                 int8_t *const row = row_at(y);
-                const uint32_t s4 = slot0 * 4, ringw = RB * 4;   // ring word of attempt j: s4 + j (mod ringw)
+                // ring word of attempt j: s4 + j (mod ringw)
+                const uint32_t s4 = slot0 * 4 + wo, ringw = RB * 4;
                 // the proposal: kDdel, kDs, kNew (proposal_bytes) and dE + 8
                 // in bits 8..12
                 int32_t info[NR];
