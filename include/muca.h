@@ -44,8 +44,8 @@ extern "C" {
  * compute unit and the layout; muca_autotune chooses by measurement) */
 #define MUCA_KERNEL_AUTO 0
 #define MUCA_KERNEL_GENERIC 1  /* one lane per walker, reference site order from tables */
-#define MUCA_KERNEL_TEAM 2     /* sixteen lanes per walker (even L, 8 <= L <= 256; lattices and
-                                  ln W in LDS when they fit) */
+#define MUCA_KERNEL_TEAM 2     /* sixteen lanes per walker (8 <= L <= 256; lattices and ln W in
+                                  LDS when they fit, for odd L only then) */
 #define MUCA_KERNEL_LANE 3     /* one lane per walker, even L, table-free, screened acceptance */
 
 /* what the produce path accumulates per walker block */

@@ -52,7 +52,7 @@ hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a);
 
 // team kernel (muca_team.hip): LDS layout of one workgroup of 16 walkers
 struct TeamLayout {
-    uint32_t row;         // L/2 attempts per half-row
+    uint32_t row;         // attempts per half-row: L/2, for odd L up to (L+1)/2
     uint32_t team_bytes;  // per-team Philox ring and ln W window
     uint32_t ring;        // Philox blocks per key held in a team's ring
     uint32_t off_win;     // inside a team's area: its ln W window (ln W in HBM)
@@ -63,7 +63,8 @@ struct TeamLayout {
     bool lds_hist, lat_lds;
     bool lnw_global;      // ln W too large for LDS: read from HBM (L2) per window
 };
-// false when the team kernel cannot run this launch (odd L, L < 8 or L > 256)
+// false when the team kernel cannot run this launch (L < 8 or L > 256, or odd L
+// whose lattices do not fit in LDS)
 bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay);
 hipError_t launch_mcs_team(hipStream_t st, const Launch &cfg, const McsArgs &a,
                            const TeamLayout &lay);

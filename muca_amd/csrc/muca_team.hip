@@ -21,9 +21,9 @@ MUCA_TEAM_EXTERN(10, true, 1)
 
 bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
 {
-    if (a.L % 2 != 0 || a.L < 8 || a.L > 256) return false;
+    if (a.L < 8 || a.L > 256) return false;
     const size_t tsz = fp64 ? 8 : 4;
-    const size_t row = a.L / 2;
+    const size_t row = (a.L + 1) / 2;   // the longest chunk
     auto al = [](size_t x) { return (x + 15) & ~(size_t)15; };
     lay.row = (uint32_t)row;
     // Philox ring: a chunk of a half-row (at most 64 attempts, starting at any
@@ -65,6 +65,7 @@ bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
     lay.lat_lds = off + al((size_t)stride * kTeams) <= lds_max;
     if (lay.lat_lds) off += al((size_t)stride * kTeams);
     lay.bytes = off;
+    if (a.L % 2 && !lay.lat_lds) return false;   // odd L: lattices in LDS only
     // lattices in HBM are addressed by a 32-bit offset within a row
     if (!lay.lat_lds && (uint64_t)a.L * a.W > 0xffffffffull) return false;
     return off <= lds_max;

@@ -34,8 +34,13 @@
 //   diff = ((T)(-dE*beta) + lnW[D+dDel]) - lnW[D];  accept iff diff >= 0 or
 //   acclog(r1) < diff.  Because acclog(r1) < 0 always, that is exactly
 //   acclog(r1) < diff.  Results are bit-identical to the one-lane kernel.
-// Requires even L, 8 <= L <= 256.  A half-row need not be a whole number of
-// Philox blocks: a chunk starts at word rs % 4 of its first block.
+// Requires 8 <= L <= 256.  A half-row need not be a whole number of Philox
+// blocks: a chunk starts at word rs % 4 of its first block.  Odd L (ODD, while
+// the lattices fit in LDS): the reference's order visits the even linear
+// indices 0, 2, .., N-3 twice and then N-2 (muca_delta_multigpu.cu:173).  Two
+// of them are neighbours only across a wrap: x = 0 and L-1 of an even row, and
+// rows 0 and L-1.  Chunks end at x = L-3 of an even row and at x = L-2 of an
+// odd one, which separates both.
 //
 // LDS (dynamic): per team a ring of Philox blocks [2 keys][(min(L/2, 64) + 6)/4 + 8][4]; the
 // acceptance-log table; (T)(-dE*beta) for dE = -8..8; ln W with guard entries
@@ -223,7 +228,8 @@ using namespace team_detail;
 // LNWG: ln W read from HBM (it does not fit in LDS), one window per team.
 // One workgroup's sixteen walkers wbase .. wbase+15 of the launch described
 // by a (all 256 lanes of the workgroup call it together).
-template <int R, bool FP64, int KEYING, bool LATLDS, bool LDSHIST, int OBS, bool LNWG, int NR>
+template <int R, bool FP64, int KEYING, bool LATLDS, bool LDSHIST, int OBS, bool LNWG, int NR,
+          bool ODD = false>
 __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay, uint64_t wbase,
                                          unsigned char *lds)
 {
@@ -275,9 +281,10 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     // 16-byte global accesses (one per site: the tile's walkers), a 4x4 byte
     // transpose per four walkers, sixteen dword LDS accesses (one per
     // walker); a lane's four loads are all in flight before the first is
-    // used.  Otherwise one byte per lane and step.
+    // used.  Otherwise, and for the last N % 4 sites, one byte per lane and
+    // step.
     const bool lat_vec = LATLDS && W % kTeams == 0 && wbase + kTeams <= W &&
-                         ((uintptr_t)a.lat & 15) == 0;   // N % 4 == 0 (even L)
+                         ((uintptr_t)a.lat & 15) == 0;
     if (LATLDS) {
         if (lat_vec) {
             for (uint32_t q = tid; q < N / 4; q += blockDim.x) {
@@ -298,12 +305,12 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                         (((s4[2][c] >> sh) & 0xffu) << 16) | (((s4[3][c] >> sh) & 0xffu) << 24);
                 }
             }
-        } else {
-            for (uint32_t e = tid; e < N * kTeams; e += blockDim.x) {
-                const uint32_t site = e >> 4, t = e & 15;
-                latl[t * lay.lat_stride + site] =
-                    (wbase + t < W) ? a.lat[(uint64_t)site * W + wbase + t] : (int8_t)0;
-            }
+        }
+        for (uint32_t e = (lat_vec ? (N & ~3u) : 0) * kTeams + tid; e < N * kTeams;
+             e += blockDim.x) {
+            const uint32_t site = e >> 4, t = e & 15;
+            latl[t * lay.lat_stride + site] =
+                (wbase + t < W) ? a.lat[(uint64_t)site * W + wbase + t] : (int8_t)0;
         }
     }
     __syncthreads();
@@ -398,7 +405,6 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
             ql[k] = window_id<KW>(0);
             qh[k] = window_id<KW>(1);
         }
-        // a workgroup adds at most 16 NUPDATES counts to one u32 bin
         // this lane's sites in a row for a chunk of half h from jb on, and
         // their right and left neighbours; they stay from row to row
         uint32_t sx[NR], sxr[NR], sxl[NR], sx_h = ~0u, sx_jb = ~0u;
@@ -414,6 +420,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
             sx_h = sh;
             sx_jb = sj;
         };
+        // a workgroup adds at most 16 NUPDATES counts to one u32 bin
         const bool may_wrap = a.hist_preload != 0 || (uint64_t)kTeams * a.nup >= (1ull << 32);
         for (int phase = 0; phase < 2; phase++) {
             const uint64_t n = phase ? a.nup : a.therm;
@@ -423,8 +430,15 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
             // (x parity), row y, place jb in the half-row -- advanced chunk by
             // chunk from 0, without divisions.
             uint32_t h = 0, y = 0, jb = 0;
+            // ODD: the next site (ox, oy), its place ot in its pair of rows
+            // (L sites: (L - 1) / 2, then the even row's last and the odd
+            // row's), and op: first or second visit of the even indices, or N-2
+            uint32_t ox = 0, oy = 0, ot = 0, op = 0;
+            const uint32_t hw = (L - 1) / 2;
             for (uint64_t rs = 0; rs < n;) {
-                const uint32_t cnt = (uint32_t)min((uint64_t)min(Rw - jb, 16u * NR), n - rs);
+                const uint32_t most = ODD ? (op == 2 ? 1u : ot < hw ? hw - ot : L - ot) : Rw - jb;
+                const uint32_t cmax = min(most, 16u * NR);
+                const uint32_t cnt = (uint32_t)min((uint64_t)cmax, n - rs);
                 // ---- A1: the walker's Philox stream (block b uses counter b + 1;
                 // the stream runs on across chunks and phases) is generated
                 // eight blocks x two keys per pass into a ring of `RB` blocks per
@@ -456,7 +470,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 cur_slot = cur_slot >= RB ? cur_slot - RB : cur_slot;
                 wave_sync();
                 // ---- A2: attempt j = 16 r + tl on this lane, everything in registers
-                int8_t *const row = row_at(y);
+                int8_t *const row = ODD ? latl : row_at(y);
                 // ring word of attempt j: s4 + j (mod ringw)
                 const uint32_t s4 = slot0 * 4 + wo, ringw = RB * 4;
                 // the proposal: kDdel, kDs, kNew (proposal_bytes) and dE + 8
@@ -467,14 +481,30 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 // wavefront per SIMD hides no latency of its own.
                 // A lane past the end of the chunk works on an in-bounds
                 // attempt and keeps nothing of it.
-                if (LNWG || h != sx_h || jb != sx_jb) sites(h, jb);
+                if (!ODD && (LNWG || h != sx_h || jb != sx_jb)) sites(h, jb);
                 uint32_t cx[NR];   // this chunk's sites (sx may move on to the next one's)
 #pragma unroll
                 for (int r = 0; r < NR; r++) cx[r] = sx[r];
                 int32_t old_s[NR], nb[NR];
                 uint32_t r1[NR], r3[NR];
                 float thi[NR];   // the screened log of r1 (acclog_screen)
-                if (PF && pf_have) {
+                if (ODD) {
+#pragma unroll
+                    for (int r = 0; r < NR; r++) {
+                        uint32_t x = ox + 2 * min(16u * r + tl, cmax - 1), yy = oy;
+                        if (x >= L) {
+                            x -= L;
+                            yy++;
+                        }
+                        const uint32_t c = x0 + yy * L + x;
+                        cx[r] = c;
+                        old_s[r] = row[c];
+                        nb[r] = row[x + 1 == L ? c + 1 - L : c + 1] +
+                                row[x == 0 ? c + L - 1 : c - 1] +
+                                row[yy + 1 == L ? c + L - N : c + L] +
+                                row[yy == 0 ? c + N - L : c - L];
+                    }
+                } else if (PF && pf_have) {
 #pragma unroll
                     for (int r = 0; r < NR; r++) {
                         old_s[r] = pf_s[r];
@@ -790,12 +820,30 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 if (!LATLDS) __threadfence_block();
                 wave_sync();
                 rs += cnt;
-                jb += cnt;
-                if (jb == Rw) {
-                    jb = 0;
-                    if (++y == L) {
-                        y = 0;
-                        h ^= 1u;
+                if (ODD) {
+                    ox += 2 * cnt;
+                    ot += cnt;
+                    while (ox >= L) {
+                        ox -= L;
+                        oy++;
+                    }
+                    if (ot == L) ot = 0;
+                    if (op == 2) {
+                        ox = oy = ot = op = 0;
+                    } else if (oy == L - 1 && ox == L - 1) {   // N-1 is not visited
+                        ox = op == 0 ? 0 : L - 2;
+                        oy = op == 0 ? 0 : L - 1;
+                        ot = 0;
+                        op++;
+                    }
+                } else {
+                    jb += cnt;
+                    if (jb == Rw) {
+                        jb = 0;
+                        if (++y == L) {
+                            y = 0;
+                            h ^= 1u;
+                        }
                     }
                 }
             }
@@ -848,18 +896,19 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                         make_uint4(d[0], d[1], d[2], d[3]);
                 }
             }
-        } else {
-            for (uint32_t e2 = tid; e2 < N * kTeams; e2 += blockDim.x) {
-                const uint32_t site = e2 >> 4, t = e2 & 15;
-                if (wbase + t < W) a.lat[(uint64_t)site * W + wbase + t] = latl[t * lay.lat_stride + site];
-            }
+        }
+        for (uint32_t e2 = (lat_vec ? (N & ~3u) : 0) * kTeams + tid; e2 < N * kTeams;
+             e2 += blockDim.x) {
+            const uint32_t site = e2 >> 4, t = e2 & 15;
+            if (wbase + t < W) a.lat[(uint64_t)site * W + wbase + t] = latl[t * lay.lat_stride + site];
         }
     }
 }
 
 // LNWG launches are the large lattices (L >= 136) with many walkers: they
 // are held to 128 VGPRs, four wavefronts per SIMD
-template <int R, bool FP64, int KEYING, bool LATLDS, bool LDSHIST, int OBS, bool LNWG, int NR>
+template <int R, bool FP64, int KEYING, bool LATLDS, bool LDSHIST, int OBS, bool LNWG, int NR,
+          bool ODD = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LNWG ? 4 : 1))) void
 k_mcs_team(McsArgs a, TeamLayout lay)
 {
@@ -872,7 +921,7 @@ k_mcs_team(McsArgs a, TeamLayout lay)
     const uint32_t G = gridDim.x;
     uint32_t g = blockIdx.x;
     if (G % kXcds == 0) g = (g % kXcds) * (G / kXcds) + g / kXcds;
-    team_run<R, FP64, KEYING, LATLDS, LDSHIST, OBS, LNWG, NR>(a, lay, (uint64_t)g * kTeams, lds);
+    team_run<R, FP64, KEYING, LATLDS, LDSHIST, OBS, LNWG, NR, ODD>(a, lay, (uint64_t)g * kTeams, lds);
 }
 
 template <int R, bool FP64, int KEYING, int NR>
@@ -884,7 +933,15 @@ hipError_t launch_team_nr(hipStream_t st, const McsArgs &a, const TeamLayout &la
     const bool moms = FP64 && a.moms != nullptr && !joint;
     constexpr int MO = FP64 ? 2 : 0;
     void (*k)(McsArgs, TeamLayout) = nullptr;
-    if (lay.lnw_global) {
+    if (a.L % 2) {
+        // odd L: lattices in LDS
+        k = moms ? k_mcs_team<R, FP64, KEYING, true, false, MO, false, NR, true>
+            : lay.lds_hist
+                ? joint ? k_mcs_team<R, FP64, KEYING, true, true, 1, false, NR, true>
+                        : k_mcs_team<R, FP64, KEYING, true, true, 0, false, NR, true>
+            : joint ? k_mcs_team<R, FP64, KEYING, true, false, 1, false, NR, true>
+                    : k_mcs_team<R, FP64, KEYING, true, false, 0, false, NR, true>;
+    } else if (lay.lnw_global) {
         // ln W too large for LDS (L >= 136): lattices and histogram stay in
         // HBM as well
         if constexpr (NR == kLnwgRounds) {
