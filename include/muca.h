@@ -243,9 +243,11 @@ typedef struct muca_instance_status {
 const char *muca_batch_last_error(void);
 /* tiles: MUCA_KERNEL_AUTO (team tiles for few walkers where every L is in
  * [8, 128]), MUCA_KERNEL_TEAM (every L % 8 == 0, L <= 128) or MUCA_KERNEL_LANE; precision: MUCA_REF32 | MUCA_FP64.  Lane tiles hold
- * 256 walkers, or 512 / 1024 when the largest instance's ln W and histogram
- * leave LDS room for only a few workgroups per compute unit (the autotuner
- * may choose otherwise). */
+ * 1024 or 512 walkers (four or two per lane) when every L > 8, every walker
+ * count is a multiple of 4 and there are 1024 walkers per compute unit, else
+ * 256, or 512 / 1024 when the largest instance's ln W and histogram leave LDS
+ * room for only a few workgroups per compute unit (the autotuner may choose
+ * otherwise). */
 int muca_batch_create(int32_t device, const muca_instance *instances, uint32_t n,
                       int32_t precision, int32_t tiles, muca_batch **batch);
 int muca_batch_destroy(muca_batch *batch);

@@ -36,6 +36,23 @@ __host__ __device__ static inline uint64_t acclog_double_to_bits(double d)
     return b;
 }
 
+// A constant of the exact log.  On the device it is put into registers where
+// it is used: the exact log is a rare branch of the update kernels' loops, and
+// ten hoisted double constants would hold 20 VGPRs through them.
+template <uint64_t BITS>
+__host__ __device__ static inline double acclog_k()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    uint32_t lo, hi;
+    asm volatile("v_mov_b32 %0, %1" : "=v"(lo) : "i"((uint32_t)BITS));
+    asm volatile("v_mov_b32 %0, %1" : "=v"(hi) : "i"((uint32_t)(BITS >> 32)));
+    return acclog_bits_to_double((uint64_t)hi << 32 | lo);
+#else
+    return acclog_bits_to_double(BITS);
+#endif
+}
+#define ACCLOG_K(c) acclog_k<__builtin_bit_cast(uint64_t, (double)(c))>()
+
 // log(u) in double-double precision, u = m * 2^-24 with m odd in [1, 2^24),
 // with the table at (invc_tab, logc_tab) (device constant memory, host
 // memory, or a copy in LDS).
@@ -54,22 +71,22 @@ __host__ __device__ static inline double acclog_u01_double_tab(uint32_t r,
     const double logc = logc_tab[i];
     const double rr = fma(z, invc, -1.0);           // |rr| <= 2^-7
     const double kf = (double)k;
-    const double kh = kf * ACCLOG_LN2HI;             // exact: |k| <= 24
+    const double kh = kf * ACCLOG_K(ACCLOG_LN2HI);             // exact: |k| <= 24
     const double t1 = kh + logc;
     const double e1 = (kh - t1) + logc;              // |kh| >= |logc| or kh == 0
     const double t2 = t1 + rr;
     const double e2 = (t1 - t2) + rr;                // |t1| >= |rr| or t1 == 0
     // log1p(rr) - rr = rr^2 * P(rr), Taylor series to rr^9
-    double p = 1.0 / 9.0;
-    p = fma(p, rr, -1.0 / 8.0);
-    p = fma(p, rr, 1.0 / 7.0);
-    p = fma(p, rr, -1.0 / 6.0);
-    p = fma(p, rr, 1.0 / 5.0);
-    p = fma(p, rr, -1.0 / 4.0);
-    p = fma(p, rr, 1.0 / 3.0);
+    double p = ACCLOG_K(1.0 / 9.0);
+    p = fma(p, rr, ACCLOG_K(-1.0 / 8.0));
+    p = fma(p, rr, ACCLOG_K(1.0 / 7.0));
+    p = fma(p, rr, ACCLOG_K(-1.0 / 6.0));
+    p = fma(p, rr, ACCLOG_K(1.0 / 5.0));
+    p = fma(p, rr, ACCLOG_K(-1.0 / 4.0));
+    p = fma(p, rr, ACCLOG_K(1.0 / 3.0));
     p = fma(p, rr, -0.5);
     const double r2 = rr * rr;
-    const double lo = fma(r2, p, fma(kf, ACCLOG_LN2LO, e1 + e2));
+    const double lo = fma(r2, p, fma(kf, ACCLOG_K(ACCLOG_LN2LO), e1 + e2));
     return t2 + lo;
 }
 
@@ -119,7 +136,9 @@ __device__ static inline float acclog_fast_band(float la)
 // and only 0 <= thi - diff < lim needs the exact log.
 __device__ static inline float acclog_screen(uint32_t r)
 {
-    const float u = (float)(1u | (r >> 8)) * 0x1p-24f;
+    // u = (k + 1/2) 2^-23, k = r >> 9: 1 + k 2^-23 from its bits, less
+    // 1 - 2^-24 (exact: both are multiples of 2^-24 within a factor of two)
+    const float u = __uint_as_float(__builtin_amdgcn_alignbit(0x7fu, r, 9)) - 0x1.fffffep-1f;
     return __builtin_fmaf(__builtin_amdgcn_logf(u), 0x1.62e430p-1f * (1.0f - ACCLOG_FAST_REL),
                           ACCLOG_FAST_ABS);
 }

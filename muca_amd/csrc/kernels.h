@@ -40,6 +40,7 @@ struct Launch {
     int kernel;      // MUCA_KERNEL_*
     int block;       // threads per block
     size_t lds_max;  // bytes of LDS available per block
+    uint32_t cus;    // compute units of the device
 };
 
 // strat_W = 0: the reference's uniform start; > 0: stratified over strat_W walkers
@@ -71,6 +72,9 @@ hipError_t launch_mcs_team(hipStream_t st, const Launch &cfg, const McsArgs &a,
 
 // lane kernel (muca_lane.hip): even L >= 4 and ln W fits in LDS
 bool lane_eligible(const McsArgs &a, int fp64, size_t lds_max);
+// walkers per lane of a lane launch: 4 where W walkers still make one and a half
+// wavefronts per SIMD, else 1
+int lane_walkers(uint32_t L, uint64_t W, uint32_t cus);
 hipError_t launch_mcs_lane(hipStream_t st, const Launch &cfg, const McsArgs &a);
 
 // ---- batched engine (muca_batch.hip) ----
@@ -88,6 +92,7 @@ struct BatchInst {
     uint64_t nup_max;      // schedule cap
     uint32_t lane_lds_w;   // lane tiles: LDS bytes of ln W
     uint32_t lane_hist;    // lane tiles: histogram in LDS
+    uint32_t lane_vec;     // lane tiles: walkers per lane
     TeamLayout lay;        // team tiles
     // advanced on the device
     uint32_t iter, width, reach, converged, reach_iter, done_iter;
@@ -177,11 +182,11 @@ __device__ __forceinline__ uint32_t batch_take(const BatchArgs &b)
 // every instance has, else 0.  The kernel built for just those is launched.
 hipError_t launch_batch_team(hipStream_t st, int fp64, const BatchArgs &b, uint32_t grid,
                              size_t lds_bytes, int lat_modes, int nrs);
-hipError_t launch_batch_lane(hipStream_t st, int fp64, const BatchArgs &b, uint32_t grid,
+hipError_t launch_batch_lane(hipStream_t st, int fp64, int vecs, const BatchArgs &b, uint32_t grid,
                              uint32_t block, size_t lds_bytes);
 // the kernels' dynamic-LDS limit, set once outside any graph capture
 hipError_t prepare_batch_team(int fp64, size_t lds_bytes, int lat_modes, int nrs);
-hipError_t prepare_batch_lane(int fp64, size_t lds_bytes);
+hipError_t prepare_batch_lane(int fp64, int vecs, size_t lds_bytes);
 // one workgroup per instance: histogram bookkeeping, convergence, ln W update
 hipError_t launch_batch_update(hipStream_t st, const BatchArgs &b);
 hipError_t launch_acclog(hipStream_t st, uint32_t k0, uint32_t n, float *out);

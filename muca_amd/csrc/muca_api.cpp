@@ -133,6 +133,7 @@ int muca_create(const muca_params *params, muca_ctx **out)
     c->cfg.rounds = (int)p.rounds;
     c->cfg.fp64 = p.precision == MUCA_FP64;
     c->cfg.keying = p.keying;
+    c->cfg.cus = c->cus;
     // Kernel choice (measured on MI355X, L = 72): the team kernel keeps every
     // SIMD busy when walkers are few (31 attempts/ns at 4096 walkers against
     // 6.7 for one lane per walker); one lane per walker wins once there are
@@ -182,16 +183,24 @@ int muca_create(const muca_params *params, muca_ctx **out)
         while (c->cfg.block > 64 && (uint64_t)W < (uint64_t)c->cfg.block * ncu)
             c->cfg.block /= 2;
     }
-    if (p.block == 0 && c->cfg.kernel == MUCA_KERNEL_LANE && (uint64_t)W >= 1024ull * ncu) {
-        // Enough walkers for two 512-lane workgroups per compute unit; when
-        // the lane kernel's LDS (ln W and the histogram) admits only one
-        // workgroup per compute unit, 1024 lanes keep twice the wavefronts
-        // resident (measured at L = 128, 262 144 walkers: 273 attempts/ns
-        // against 158 with 512; at L = 72, 524 288 walkers, 512 leads: 279).
+    if (p.block == 0 && c->cfg.kernel == MUCA_KERNEL_LANE) {
+        // Four walkers per lane (lane_walkers): 256 lanes, or 512 where the
+        // lane kernel's LDS (ln W and the histogram) admits one workgroup per
+        // compute unit (524 288 walkers, L = 72: 570 attempts/ns either way).
+        // One walker per lane: with room for several workgroups 512 lanes once
+        // they fill the device (L = 72, 262 144 walkers: 335 attempts/ns
+        // against 195 with 256 lanes); with room for one the walkers of a
+        // compute unit in one workgroup (L = 128, 131 072 walkers: 186 with
+        // 512 lanes against 103 with 256; 262 144: 324 with 1024).
         const size_t tsz = p.precision == MUCA_FP64 ? 8 : 4;
         const size_t lds_lane = (size_t)(p.L * p.L + 1) * (tsz + 4);
-        const size_t lds_cu = (size_t)(lds > 0 ? lds : 65536);
-        c->cfg.block = lds_lane * 2 > lds_cu ? 1024 : 512;
+        const bool one = lds_lane * 2 > (size_t)(lds > 0 ? lds : 65536);
+        if (muca::lane_walkers(p.L, W, (uint32_t)ncu) == 4)
+            c->cfg.block = one ? 512 : 256;
+        else if (one)
+            c->cfg.block = W > 512ull * ncu ? 1024 : W > 256ull * ncu ? 512 : 256;
+        else
+            c->cfg.block = W >= 1024ull * ncu ? 512 : 256;
     }
     c->cfg.lds_max = (size_t)(lds > 0 ? lds : 65536);
     const uint64_t N = c->N;

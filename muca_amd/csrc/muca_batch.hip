@@ -270,6 +270,7 @@ int bfail(int code, const std::string &m)
 struct muca_batch {
     int device = 0, fp64 = 0, kind = 0;   // kind: MUCA_KERNEL_TEAM | MUCA_KERNEL_LANE
     uint32_t block = 256, grid = 0, cus = 0;
+    int vecs = 0;        // lane tiles: several walkers per lane (BatchInst::lane_vec)
     size_t lds_bytes = 0;
     int lat_modes = 3;   // team tiles: lattices in LDS (bit 0) / in HBM (bit 1)
     int nrs = 0;         // team tiles: rounds per chunk common to all instances, else 0
@@ -352,8 +353,8 @@ hipError_t launch_iteration(muca_batch *b)
     hipError_t e = b->kind == MUCA_KERNEL_TEAM
                        ? muca::launch_batch_team(b->st, b->fp64, b->a, b->grid, b->lds_bytes,
                                                  b->lat_modes, b->nrs)
-                       : muca::launch_batch_lane(b->st, b->fp64, b->a, b->grid, b->block,
-                                                 b->lds_bytes);
+                       : muca::launch_batch_lane(b->st, b->fp64, b->vecs, b->a, b->grid,
+                                                 b->block, b->lds_bytes);
     if (e != hipSuccess) return e;
     return muca::launch_batch_update(b->st, b->a);
 }
@@ -371,33 +372,55 @@ hipError_t configure(muca_batch *b, int kind, uint32_t block)
                                   ? I.lay.bytes
                                   : (size_t)I.lane_lds_w + (I.lane_hist ? (size_t)(I.N + 1) * 4 : 0));
     const uint32_t per_cu_lds = (uint32_t)std::max<size_t>(1, b->lds_device / (need + 256));
+    const uint32_t n = (uint32_t)b->inst.size();
+    // Lane tiles, automatic: with enough walkers for a wavefront of four per
+    // lane on every SIMD, 256-lane tiles of four walkers per lane, or of two
+    // for lattices whose tile would take longer than an even share of the
+    // work (their tiles, alone on their compute units, would be what the
+    // launch lasts).  96 problems of L = 32 to 128 with 4096 walkers each:
+    // 8.5 ms per iteration, 11.6 with four throughout, 12.4 with one walker
+    // per lane in 1024-lane tiles.
+    b->vecs = kind == MUCA_KERNEL_LANE && block == 0 && b->walkers >= 1024ull * b->cus;
+    double work = 0;   // site visits per sweep
+    for (const auto &I : b->inst) {
+        if (I.W % 4 || I.L <= 8) b->vecs = 0;
+        work += (double)I.W * I.N;
+    }
+    const double share = work / (1024.0 * b->cus * std::min(per_cu_lds, 2u));
+    for (auto &I : b->inst)
+        I.lane_vec = !b->vecs ? 1 : I.N > 1.2 * share || I.W <= 512 ? 2 : 4;
+    if (b->vecs) block = 256;
     if (kind == MUCA_KERNEL_LANE && block == 0) {
-        // one lane per walker hides latency with many wavefronts: when LDS
+        // one walker per lane hides latency with many wavefronts: when LDS
         // admits few workgroups per compute unit, make them larger (L = 128:
         // ln W and the histogram take 128 KB, one 1024-lane workgroup per CU)
         block = 256;
         while (block < 1024 && per_cu_lds * block < 2048) block *= 2;
     }
     b->block = kind == MUCA_KERNEL_TEAM ? 256 : block;
-    const uint32_t per = kind == MUCA_KERNEL_TEAM ? 16 : b->block;
-    const uint32_t n = (uint32_t)b->inst.size();
-    std::vector<uint32_t> order(n);   // largest lattices first
+    auto per = [&](const muca::BatchInst &I) {   // walkers per tile
+        return kind == MUCA_KERNEL_TEAM ? 16u : b->block * I.lane_vec;
+    };
+    auto cost = [&](const muca::BatchInst &I) { return (uint64_t)I.N * I.lane_vec; };
+    std::vector<uint32_t> order(n);   // longest tiles first
     for (uint32_t i = 0; i < n; i++) order[i] = i;
     std::stable_sort(order.begin(), order.end(),
-                     [&](uint32_t x, uint32_t y) { return b->inst[x].N > b->inst[y].N; });
+                     [&](uint32_t x, uint32_t y) { return cost(b->inst[x]) > cost(b->inst[y]); });
     // groups of tiles that share lattice lines (eight team tiles of 16
     // walkers make 128 bytes; a lane tile fills whole lines by itself) are
-    // dealt to the XCD queues in turn, each queue keeping the largest-first
+    // dealt to the XCD queues in turn, each queue keeping the longest-first
     // order
     const uint32_t group = kind == MUCA_KERNEL_TEAM ? 8 : 1;
     std::vector<muca::BatchTile> q[muca::kBatchQueues];
     uint32_t next = 0;
-    for (uint32_t i : order)
-        for (uint32_t w = 0; w < b->inst[i].W; w += per) {
-            q[next].push_back({i, w});
-            if ((w / per) % group == group - 1 || w + per >= b->inst[i].W)
+    for (uint32_t i : order) {
+        const uint32_t pw = per(b->inst[i]);
+        for (uint64_t w = 0; w < b->inst[i].W; w += pw) {
+            q[next].push_back({i, (uint32_t)w});
+            if ((w / pw) % group == group - 1 || w + pw >= b->inst[i].W)
                 next = (next + 1) % muca::kBatchQueues;
         }
+    }
     b->tiles.clear();
     for (uint32_t x = 0; x < muca::kBatchQueues; x++) {
         b->a.qstart[x] = (uint32_t)b->tiles.size();
@@ -422,7 +445,7 @@ hipError_t configure(muca_batch *b, int kind, uint32_t block)
     if (e != hipSuccess) return e;
     return kind == MUCA_KERNEL_TEAM
                ? muca::prepare_batch_team(b->fp64, b->lds_bytes, b->lat_modes, b->nrs)
-               : muca::prepare_batch_lane(b->fp64, b->lds_bytes);
+               : muca::prepare_batch_lane(b->fp64, b->vecs, b->lds_bytes);
 }
 
 }  // namespace
@@ -736,7 +759,8 @@ int muca_batch_iterate_profiled(muca_batch *b, uint32_t iterations, float *updat
         BHIP(b->kind == MUCA_KERNEL_TEAM
                  ? muca::launch_batch_team(b->st, b->fp64, b->a, b->grid, b->lds_bytes,
                                            b->lat_modes, b->nrs)
-                 : muca::launch_batch_lane(b->st, b->fp64, b->a, b->grid, b->block, b->lds_bytes));
+                 : muca::launch_batch_lane(b->st, b->fp64, b->vecs, b->a, b->grid, b->block,
+                                           b->lds_bytes));
         BHIP(hipEventRecord(ev[1], b->st));
         BHIP(muca::launch_batch_update(b->st, b->a));
         BHIP(hipEventRecord(ev[2], b->st));
@@ -763,7 +787,7 @@ int muca_batch_autotune(muca_batch *b, uint32_t mm, int32_t *kind, uint32_t *blo
     std::vector<Cand> cands;
     if (b->team_ok) cands.push_back({MUCA_KERNEL_TEAM, 256});
     if (b->lane_ok)
-        for (uint32_t blk : {256u, 512u, 1024u}) cands.push_back({MUCA_KERNEL_LANE, blk});
+        for (uint32_t blk : {0u, 256u, 512u, 1024u}) cands.push_back({MUCA_KERNEL_LANE, blk});
     // ln W of an initialised batch (a surrogate seed, say) survives the
     // tuning: each candidate re-initialises the batch, which zeroes ln W
     BHIP(hipStreamSynchronize(b->st));
@@ -775,7 +799,7 @@ int muca_batch_autotune(muca_batch *b, uint32_t mm, int32_t *kind, uint32_t *blo
         BHIP(hipMemcpy(keep32.data(), b->a.lnw32, b->bins * 4, hipMemcpyDeviceToHost));
     }
     float best = 0;
-    Cand pick{b->kind, b->block};
+    Cand pick = cands[0];
     for (const Cand &c : cands) {
         BHIP(configure(b, c.kind, c.block));
         int rc = batch_init(b, mm, b->stratified);

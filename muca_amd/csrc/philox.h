@@ -16,6 +16,16 @@ struct philox4 {
 #define MUCA_PHILOX_W0 0x9E3779B9u
 #define MUCA_PHILOX_W1 0xBB67AE85u
 
+// one v_bitop3_b32 on the device (two v_xor_b32 otherwise)
+__host__ __device__ static inline uint32_t muca_xor3(uint32_t a, uint32_t b, uint32_t c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+    return a ^ b ^ c;
+#endif
+}
+
 template <int R>
 __host__ __device__ static inline philox4 philox4x32(uint32_t c0, uint32_t c1, uint32_t c2,
                                                      uint32_t c3, uint32_t k0, uint32_t k1)
@@ -28,8 +38,8 @@ __host__ __device__ static inline philox4 philox4x32(uint32_t c0, uint32_t c1, u
         }
         const uint64_t p0 = (uint64_t)MUCA_PHILOX_M0 * c0;
         const uint64_t p1 = (uint64_t)MUCA_PHILOX_M1 * c2;
-        const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
-        const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+        const uint32_t n0 = muca_xor3((uint32_t)(p1 >> 32), c1, k0);
+        const uint32_t n2 = muca_xor3((uint32_t)(p0 >> 32), c3, k1);
         c1 = (uint32_t)p1;
         c3 = (uint32_t)p0;
         c0 = n0;

@@ -52,6 +52,7 @@
 #include "acclog.h"
 #include "moments.h"
 #include "philox.h"
+#include "proposal.h"
 
 namespace muca {
 
@@ -116,17 +117,11 @@ __device__ __forceinline__ float mag_word(double x)
     return __uint_as_float((uint32_t)(__double_as_longlong(x) >> 32));
 }
 
-// ---- proposals: new spin from the old one (-1, 0, 1) and the step's random
-// word (+1 below 2^31, else -1, wrapped into -1..1).  Bits 0-1 of a proposal
-// byte hold dDel + 1, 2-4 the spin change + 2, 5-6 the new spin + 1; the six
-// cases are the bytes of two dwords, indexed by old + 1 (+ 4 for a step down).
-// mds: minus the spin change.
-__device__ __forceinline__ void proposal_bytes(int32_t old_s, uint32_t r3, uint32_t &pr,
-                                               int32_t &mds)
+// The proposal byte of an attempt: bits 0-1 hold dDel + 1, 2-4 the spin change
+// + 2, 5-6 the new spin + 1 (the six cases of proposal_index)
+__device__ __forceinline__ uint32_t proposal_byte(uint32_t at)
 {
-    const uint32_t at = (uint32_t)old_s + 0x0c0c0c01u + ((r3 >> 29) & 4u);
-    pr = __builtin_amdgcn_perm(0x00240651u, 0x00014e2cu, at);
-    mds = (int32_t)(int8_t)__builtin_amdgcn_perm(0x000101feu, 0x0002ffffu, at);
+    return __builtin_amdgcn_perm(0x00240651u, 0x00014e2cu, at);
 }
 // fields of an attempt's info word: a proposal byte and (dE + 8) << 8
 __device__ __forceinline__ int32_t i_ddel(int32_t i)
@@ -473,7 +468,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 int8_t *const row = ODD ? latl : row_at(y);
                 // ring word of attempt j: s4 + j (mod ringw)
                 const uint32_t s4 = slot0 * 4 + wo, ringw = RB * 4;
-                // the proposal: kDdel, kDs, kNew (proposal_bytes) and dE + 8
+                // the proposal byte and dE + 8
                 // in bits 8..12
                 int32_t info[NR];
                 // Every load of the chunk's spins and random words first, then
@@ -530,9 +525,9 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 T fde[NR];
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
-                    uint32_t pr;
-                    int32_t mds;
-                    proposal_bytes(old_s[r], r3[r], pr, mds);
+                    const uint32_t at = proposal_index(old_s[r], r3[r]);
+                    const uint32_t pr = proposal_byte(at);
+                    const int32_t mds = proposal_mds(at);
                     thi[r] = acclog_screen(r1[r]);
                     const int32_t dE = __mul24(mds, nb[r]);
                     info[r] = (int32_t)pr | ((dE + 8) << 8);
