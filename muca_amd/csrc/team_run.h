@@ -358,11 +358,6 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 for (int k = 0; k < kMomLdsWords; k++) msl[k * kMomSlots + tl] = 0;
             }
         };
-        // joint-histogram entries of this lane's attempts, counted for the bin
-        // in use and the one before it and added with one atomic when a third
-        // bin comes up (a walker stepping back and forth adds nothing)
-        uint64_t jrun = 0, jprun = 0;
-        int64_t jbin = -1, jpbin = -1;
         uint32_t c0base = 0;
         const uint32_t RB = lay.ring;
         uint32_t gen = 0, gen_slot = 0, cur_slot = 0;   // next block to make, its slot, block blk0's slot
@@ -714,26 +709,24 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                         de_lane += i_dE(info[r]);
                         dm_lane += ds;
                     }
-                    if (JOINT && phase && valid) {
-                        const int64_t dd = dv;
-                        const int64_t mm = min(max((int64_t)mv, -dd), dd);
-                        const int64_t jbn = (mm + dd * dd + 2 * dd) / 2;
-                        if (jbn != jbin) {
-                            if (jbn == jpbin) {
-                                const uint64_t t = jrun;
-                                jrun = jprun;
-                                jprun = t;
-                                jpbin = jbin;
-                            } else {
-                                if (jprun)
-                                    atomicAdd((unsigned long long *)&jbase[jpbin], jprun);
-                                jprun = jrun;
-                                jpbin = jbin;
-                                jrun = 0;
-                            }
-                            jbin = jbn;
-                        }
-                        jrun++;
+                    // Attempt j records the (D, M) after its step.  Steps that are
+                    // not accepted keep the state, so a round splits into
+                    // segments that start at step 0 and at every accepted step
+                    // and share one (D, M); the first lane of each adds its
+                    // length.
+                    bool lead = false;
+                    uint32_t slen = 0;
+                    if (TRACKM && phase) {
+                        const uint32_t ab =
+                            (uint32_t)(__builtin_amdgcn_ballot_w64(acc) >> sh) & 0xffffu;
+                        const uint32_t later = ab & ~upto;
+                        lead = tl < left && (tl == 0 || acc);
+                        slen = (later ? (uint32_t)__builtin_ctz(later) : left) - (uint32_t)tl;
+                    }
+                    if (JOINT && lead) {
+                        const int64_t mm = min(max(mv, -dv), dv);
+                        atomicAdd((unsigned long long *)&jbase[(mm + (int64_t)dv * (dv + 2)) >> 1],
+                                  (unsigned long long)slen);
                     }
                     if (phase && !MOMS) {
                         // The D histogram: a round's steps split into runs at one D,
@@ -762,17 +755,8 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                         }
                     }
                     if (MOMS && phase) {
-                        // Attempt j records the (D, M) after its step.  Steps that
-                        // are not accepted keep the state, so a round splits into
-                        // segments that start at step 0 and at every accepted step
-                        // and share one (D, M); the first lane of each segment adds
-                        // len x (1, |M|, M^2, M^4) to the slot of its D.
-                        const uint32_t ab =
-                            (uint32_t)(__builtin_amdgcn_ballot_w64(acc) >> sh) & 0xffffu;
-                        const bool lead = tl < left && (tl == 0 || acc);
-                        const uint32_t later = ab & ~upto;
-                        const uint32_t len =
-                            (later ? (uint32_t)__builtin_ctz(later) : left) - (uint32_t)tl;
+                        // a segment adds len x (1, |M|, M^2, M^4) to the slot of its D
+                        const uint32_t len = slen;
                         const int32_t dd = dv;
                         int32_t slot = dd - mwb;
                         const bool past = lead && (uint32_t)slot >= (uint32_t)kMomSlots;
@@ -843,10 +827,6 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 }
             }
             c0base += (uint32_t)((n + 3) / 4);
-        }
-        if (JOINT) {
-            if (jrun) atomicAdd((unsigned long long *)&jbase[jbin], jrun);
-            if (jprun) atomicAdd((unsigned long long *)&jbase[jpbin], jprun);
         }
         if (MOMS) flush_slot();
         // dE and dM of accepted moves were summed per lane; one reduction
