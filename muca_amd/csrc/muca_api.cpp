@@ -241,12 +241,16 @@ int muca_create(const muca_params *params, muca_ctx **out)
         e = hipMemcpy(c->naver, naver.data(), naver.size() * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpy(c->order, order.data(), order.size() * 4, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(c->lat, 0, N * W);
-    if (e == hipSuccess) e = hipMemset(c->E, 0, W * 4);
-    if (e == hipSuccess) e = hipMemset(c->D, 0, W * 4);
-    if (e == hipSuccess) e = hipMemset(c->M, 0, W * 4);
+    // on the context's stream: one of the null stream would not be ordered
+    // before the launches that follow
+    if (e == hipSuccess) e = hipMemsetAsync(c->lat, 0, N * W, c->st);
+    if (e == hipSuccess) e = hipMemsetAsync(c->E, 0, W * 4, c->st);
+    if (e == hipSuccess) e = hipMemsetAsync(c->D, 0, W * 4, c->st);
+    if (e == hipSuccess) e = hipMemsetAsync(c->M, 0, W * 4, c->st);
     if (e == hipSuccess && c->moms)
-        e = hipMemset(c->moms, 0, (uint64_t)muca::kMomWords * (N + 1) * p.joint_blocks * 8);
+        e = hipMemsetAsync(c->moms, 0, (uint64_t)muca::kMomWords * (N + 1) * p.joint_blocks * 8,
+                           c->st);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     if (e != hipSuccess) {
         free_ctx(c);
         return fail(MUCA_E_HIP, std::string("context setup: ") + hipGetErrorString(e));

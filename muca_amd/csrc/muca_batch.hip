@@ -631,12 +631,15 @@ int batch_init(muca_batch *b, uint32_t mm, int stratified)
     BHIP(hipStreamSynchronize(b->st));
     BHIP(hipMemcpy(A.inst, b->inst.data(), b->inst.size() * sizeof(muca::BatchInst),
                    hipMemcpyHostToDevice));
-    BHIP(hipMemset(A.queue, 0, 4 * muca::kBatchQueues));
-    BHIP(hipMemset(A.lnw32, 0, b->bins * 4));
-    BHIP(hipMemset(A.lnw64, 0, b->bins * 8));
-    BHIP(hipMemset(A.hist, 0, b->bins * 8));
-    BHIP(hipMemset(A.hist_last, 0, b->bins * 8));
-    BHIP(hipMemset(A.p_acc, 0, b->bins * 8));
+    // on the batch's stream: one of the null stream would not be ordered
+    // before the launches that follow
+    BHIP(hipMemsetAsync(A.queue, 0, 4 * muca::kBatchQueues, b->st));
+    BHIP(hipMemsetAsync(A.lnw32, 0, b->bins * 4, b->st));
+    BHIP(hipMemsetAsync(A.lnw64, 0, b->bins * 8, b->st));
+    BHIP(hipMemsetAsync(A.hist, 0, b->bins * 8, b->st));
+    BHIP(hipMemsetAsync(A.hist_last, 0, b->bins * 8, b->st));
+    BHIP(hipMemsetAsync(A.p_acc, 0, b->bins * 8, b->st));
+    BHIP(hipStreamSynchronize(b->st));
     b->inited = true;
     return MUCA_OK;
 }

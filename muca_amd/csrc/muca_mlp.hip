@@ -674,8 +674,8 @@ int muca_mlp_set_params(muca_mlp *g, const float *params, uint32_t n)
         if (!std::isfinite(params[i])) return mfail(MUCA_E_ARG, "parameters must be finite");
     MHIP(hipSetDevice(g->device));
     MHIP(hipMemcpy(g->p, params, kParams * sizeof(float), hipMemcpyHostToDevice));
-    MHIP(hipMemset(g->m, 0, kParams * sizeof(float)));
-    MHIP(hipMemset(g->v, 0, kParams * sizeof(float)));
+    MHIP(hipMemsetAsync(g->m, 0, kParams * sizeof(float), g->st));
+    MHIP(hipMemsetAsync(g->v, 0, kParams * sizeof(float), g->st));
     g->step = 0;
     hipLaunchKernelGGL(k_mlp_refresh_bf16, dim3((kParams + 255) / 256), dim3(256), 0, g->st, g->p,
                        g->wb);
