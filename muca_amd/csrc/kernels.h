@@ -54,6 +54,8 @@ hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a);
 // team kernel (muca_team.hip): LDS layout of one workgroup of 16 walkers
 struct TeamLayout {
     uint32_t row;         // attempts per half-row: L/2, for odd L up to (L+1)/2
+    uint32_t rounds;      // rounds of sixteen attempts per chunk
+    uint32_t order;       // 0: chunks end with their row; 1: odd L; 2: they run on
     uint32_t team_bytes;  // per-team Philox ring and ln W window
     uint32_t ring;        // Philox blocks per key held in a team's ring
     uint32_t off_win;     // inside a team's area: its ln W window (ln W in HBM)

@@ -432,7 +432,7 @@ hipError_t configure(muca_batch *b, int kind, uint32_t block)
     b->nrs = -1;
     for (const auto &I : b->inst) {
         b->lat_modes |= I.lay.lat_lds ? 1 : 2;
-        const int nr = (int)std::min<uint32_t>((I.lay.row + 15) / 16, 4);
+        const int nr = (int)(I.lay.rounds + (I.lay.order == 2 ? 8 : 0));
         b->nrs = b->nrs == -1 || b->nrs == nr ? nr : 0;
     }
     if (b->nrs < 0) b->nrs = 0;

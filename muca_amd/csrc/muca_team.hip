@@ -65,6 +65,15 @@ bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
     lay.lat_lds = off + al((size_t)stride * kTeams) <= lds_max;
     if (lay.lat_lds) off += al((size_t)stride * kTeams);
     lay.bytes = off;
+    // Where the last round of a half-row would be at most half full, chunks of
+    // whole rounds run on into the next row (lattices in LDS: those in HBM are
+    // read a chunk ahead, row by row).
+    const uint32_t hw = a.L / 2, rem = hw % 16;   // attempts from a site to its upper neighbour
+    const bool flow = lay.lat_lds && hw >= 16 && rem <= 8 && (rem != 0 || a.L % 2);
+    lay.order = a.L % 2 ? 1 : flow ? 2 : 0;
+    const uint32_t nr = flow ? hw / 16 : (uint32_t)(row + 15) / 16;
+    const uint32_t cap = lay.lnw_global ? (uint32_t)kLnwgRounds : 4u;
+    lay.rounds = nr < cap ? nr : cap;
     if (a.L % 2 && !lay.lat_lds) return false;   // odd L: lattices in LDS only
     // lattices in HBM are addressed by a 32-bit offset within a row
     if (!lay.lat_lds && (uint64_t)a.L * a.W > 0xffffffffull) return false;
@@ -96,7 +105,8 @@ hipError_t launch_mcs_team(hipStream_t st, const Launch &cfg, const McsArgs &a,
 // Philox4x32-7, walker ids 0..W-1 within each instance, seed = instance seed.
 // ---------------------------------------------------------------------------
 // LM: the lattice placements this build of the kernel handles (1: LDS,
-// 2: HBM, 3: both); NRS: the rounds per chunk of every instance (0: any).
+// 2: HBM, 3: both); NRS: the rounds per chunk of every instance (0: any), 8
+// more where chunks run on from row to row.
 // A batch of one placement (and one chunk size) launches the build for it
 // alone, whose registers and schedule the other variants' code does not
 // constrain.
@@ -116,39 +126,41 @@ __global__ __launch_bounds__(256) void k_batch_team(BatchArgs b)
         if (I->converged) continue;
         const McsArgs a = batch_mcs_args(b, *I);
         const TeamLayout lay = I->lay;
-        const uint32_t nr = (lay.row + 15) / 16;
-        const int v = (lay.lat_lds ? 1 : 0) | (lay.lds_hist ? 2 : 0);
-#define MUCA_BT(NR)                                                                            \
-    switch (v) {                                                                               \
-    case 0:                                                                                    \
-        if constexpr ((LM & 2) != 0)                                                           \
-            team_run<7, FP64, 0, false, false, 0, false, NR>(a, lay, tile.wbase, lds);         \
-        break;                                                                                 \
-    case 1:                                                                                    \
-        if constexpr ((LM & 1) != 0)                                                           \
-            team_run<7, FP64, 0, true, false, 0, false, NR>(a, lay, tile.wbase, lds);          \
-        break;                                                                                 \
-    case 2:                                                                                    \
-        if constexpr ((LM & 2) != 0)                                                           \
-            team_run<7, FP64, 0, false, true, 0, false, NR>(a, lay, tile.wbase, lds);          \
-        break;                                                                                 \
-    default:                                                                                   \
-        if constexpr ((LM & 1) != 0)                                                           \
-            team_run<7, FP64, 0, true, true, 0, false, NR>(a, lay, tile.wbase, lds);           \
-        break;                                                                                 \
-    }
-        if constexpr (NRS != 0) {
-            MUCA_BT(NRS)
-        } else if (nr <= 1) {
-            MUCA_BT(1)
-        } else if (nr <= 2) {
-            MUCA_BT(2)
-        } else if (nr <= 3) {
-            MUCA_BT(3)
+        auto run = [&](auto nr, auto ord) {
+            constexpr int NR = decltype(nr)::value, ORD = decltype(ord)::value;
+            if (lay.lat_lds) {
+                if constexpr ((LM & 1) != 0) {
+                    if (lay.lds_hist)
+                        team_run<7, FP64, 0, true, true, 0, false, NR, ORD>(a, lay, tile.wbase, lds);
+                    else
+                        team_run<7, FP64, 0, true, false, 0, false, NR, ORD>(a, lay, tile.wbase, lds);
+                }
+            } else if constexpr ((LM & 2) != 0 && ORD == 0) {
+                if (lay.lds_hist)
+                    team_run<7, FP64, 0, false, true, 0, false, NR, ORD>(a, lay, tile.wbase, lds);
+                else
+                    team_run<7, FP64, 0, false, false, 0, false, NR, ORD>(a, lay, tile.wbase, lds);
+            }
+        };
+        std::integral_constant<int, 0> rows;
+        std::integral_constant<int, 2> flow;
+        if constexpr (NRS > 8) {
+            run(std::integral_constant<int, NRS - 8>{}, flow);
+        } else if constexpr (NRS != 0) {
+            run(std::integral_constant<int, NRS>{}, rows);
+        } else if (lay.order == 2) {
+            if (lay.rounds == 1)
+                run(std::integral_constant<int, 1>{}, flow);
+            else
+                run(std::integral_constant<int, 2>{}, flow);
         } else {
-            MUCA_BT(4)
+            switch (lay.rounds) {
+            case 1: run(std::integral_constant<int, 1>{}, rows); break;
+            case 2: run(std::integral_constant<int, 2>{}, rows); break;
+            case 3: run(std::integral_constant<int, 3>{}, rows); break;
+            default: run(std::integral_constant<int, 4>{}, rows); break;
+            }
         }
-#undef MUCA_BT
     }
 }
 
@@ -161,6 +173,8 @@ static void (*batch_team_kernel(int lat_modes, int nrs))(BatchArgs)
         case 2: return k_batch_team<FP64, 1, 2>;
         case 3: return k_batch_team<FP64, 1, 3>;
         case 4: return k_batch_team<FP64, 1, 4>;
+        case 9: return k_batch_team<FP64, 1, 9>;
+        case 10: return k_batch_team<FP64, 1, 10>;
         default: return k_batch_team<FP64, 1, 0>;
         }
     }

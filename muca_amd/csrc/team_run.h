@@ -224,12 +224,13 @@ using namespace team_detail;
 // One workgroup's sixteen walkers wbase .. wbase+15 of the launch described
 // by a (all 256 lanes of the workgroup call it together).
 template <int R, bool FP64, int KEYING, bool LATLDS, bool LDSHIST, int OBS, bool LNWG, int NR,
-          bool ODD = false>
+          int ORD = 0>
 __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay, uint64_t wbase,
                                          unsigned char *lds)
 {
     typedef typename std::conditional<FP64, double, float>::type T;
     constexpr int KW = kWinFor<KEYING>;   // this launch's mask width (<= kWin)
+    constexpr bool ODD = ORD == 1, FLOW = ORD == 2;
     constexpr bool JOINT = OBS == 1, MOMS = OBS == 2, TRACKM = OBS >= 1;
     __syncthreads();   // LDS may still be read by a previous call's flush
     T *wt = (T *)(lds + lay.off_w) + kGuard;   // valid for [-kGuard, N + kGuard]
@@ -416,6 +417,13 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
             const uint64_t n = phase ? a.nup : a.therm;
             // A half-row is worked in chunks of up to 16 NR attempts (no two
             // sites of a half-row are neighbours, so any split of it is exact).
+            // FLOW: chunks of 16 NR <= Rw attempts run on into the next row
+            // (the lower neighbour of an attempt is Rw attempts back, every
+            // other one of its half further): half-rows of 16 k + 1 .. 16 k + 8
+            // attempts would leave half or more of their last round idle.
+            // L = 72, 4096 walkers: 74 -> 82 attempts/ns (FP64 67 -> 76), with
+            // 36 = 32 + 4 attempts in a row; at 16 k + 10 and more the shorter
+            // chunks cost more than the lanes (L = 60: 81 -> 75).
             // Attempt rs of a phase is at sweep position rs mod N: half h
             // (x parity), row y, place jb in the half-row -- advanced chunk by
             // chunk from 0, without divisions.
@@ -424,9 +432,17 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
             // (L sites: (L - 1) / 2, then the even row's last and the odd
             // row's), and op: first or second visit of the even indices, or N-2
             uint32_t ox = 0, oy = 0, ot = 0, op = 0;
+            // (of two neighbouring sites visited in one pass over the even indices
+            // the later one comes hw attempts after the other or more: with
+            // 16 NR <= hw a chunk may run on over the ends of rows)
             const uint32_t hw = (L - 1) / 2;
             for (uint64_t rs = 0; rs < n;) {
-                const uint32_t most = ODD ? (op == 2 ? 1u : ot < hw ? hw - ot : L - ot) : Rw - jb;
+                const uint32_t odd_left = hw >= 16u * NR ? (N - 1 - oy * L - ox) / 2
+                                          : ot < hw      ? hw - ot
+                                                         : L - ot;
+                const uint32_t most = ODD    ? (op == 2 ? 1u : odd_left)
+                                      : FLOW ? Rw
+                                             : Rw - jb;
                 const uint32_t cmax = min(most, 16u * NR);
                 const uint32_t cnt = (uint32_t)min((uint64_t)cmax, n - rs);
                 // ---- A1: the walker's Philox stream (block b uses counter b + 1;
@@ -460,7 +476,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 cur_slot = cur_slot >= RB ? cur_slot - RB : cur_slot;
                 wave_sync();
                 // ---- A2: attempt j = 16 r + tl on this lane, everything in registers
-                int8_t *const row = ODD ? latl : row_at(y);
+                int8_t *const row = ODD || FLOW ? latl : row_at(y);
                 // ring word of attempt j: s4 + j (mod ringw)
                 const uint32_t s4 = slot0 * 4 + wo, ringw = RB * 4;
                 // the proposal byte and dE + 8
@@ -471,7 +487,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 // wavefront per SIMD hides no latency of its own.
                 // A lane past the end of the chunk works on an in-bounds
                 // attempt and keeps nothing of it.
-                if (!ODD && (LNWG || h != sx_h || jb != sx_jb)) sites(h, jb);
+                if (!ODD && !FLOW && (LNWG || h != sx_h || jb != sx_jb)) sites(h, jb);
                 uint32_t cx[NR];   // this chunk's sites (sx may move on to the next one's)
 #pragma unroll
                 for (int r = 0; r < NR; r++) cx[r] = sx[r];
@@ -493,6 +509,24 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                                 row[x == 0 ? c + L - 1 : c - 1] +
                                 row[yy + 1 == L ? c + L - N : c + L] +
                                 row[yy == 0 ? c + N - L : c - L];
+                    }
+                } else if (FLOW) {
+                    // row y from jb on, then the next row (of the next half
+                    // after the last) from its start
+                    const uint32_t y1 = y + 1 == L ? 0 : y + 1, h1 = y + 1 == L ? h ^ 1u : h;
+                    const uint32_t c0 = x0 + y * L + h, c1 = x0 + y1 * L + h1 - L;
+                    const uint32_t up0 = y + 1 == L ? L - N : L, up1 = y1 + 1 == L ? L - N : L;
+                    const uint32_t dn0 = y == 0 ? N - L : 0u - L, dn1 = y1 == 0 ? N - L : 0u - L;
+#pragma unroll
+                    for (int r = 0; r < NR; r++) {
+                        const uint32_t j2 = 2 * (jb + min(16u * r + tl, cmax - 1));
+                        const bool nxt = j2 >= L;
+                        const uint32_t c = j2 + (nxt ? c1 : c0), x = j2 + (nxt ? h1 - L : h);
+                        cx[r] = c;
+                        old_s[r] = row[c];
+                        nb[r] = row[x + 1 == L ? c + 1 - L : c + 1] +
+                                row[x == 0 ? c + L - 1 : c - 1] + row[c + (nxt ? up1 : up0)] +
+                                row[c + (nxt ? dn1 : dn0)];
                     }
                 } else if (PF && pf_have) {
 #pragma unroll
@@ -817,8 +851,8 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     }
                 } else {
                     jb += cnt;
-                    if (jb == Rw) {
-                        jb = 0;
+                    if (jb >= Rw) {
+                        jb -= Rw;
                         if (++y == L) {
                             y = 0;
                             h ^= 1u;
@@ -883,7 +917,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
 // LNWG launches are the large lattices (L >= 136) with many walkers: they
 // are held to 128 VGPRs, four wavefronts per SIMD
 template <int R, bool FP64, int KEYING, bool LATLDS, bool LDSHIST, int OBS, bool LNWG, int NR,
-          bool ODD = false>
+          int ORD = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LNWG ? 4 : 1))) void
 k_mcs_team(McsArgs a, TeamLayout lay)
 {
@@ -896,10 +930,10 @@ k_mcs_team(McsArgs a, TeamLayout lay)
     const uint32_t G = gridDim.x;
     uint32_t g = blockIdx.x;
     if (G % kXcds == 0) g = (g % kXcds) * (G / kXcds) + g / kXcds;
-    team_run<R, FP64, KEYING, LATLDS, LDSHIST, OBS, LNWG, NR, ODD>(a, lay, (uint64_t)g * kTeams, lds);
+    team_run<R, FP64, KEYING, LATLDS, LDSHIST, OBS, LNWG, NR, ORD>(a, lay, (uint64_t)g * kTeams, lds);
 }
 
-template <int R, bool FP64, int KEYING, int NR>
+template <int R, bool FP64, int KEYING, int NR, int ORD>
 hipError_t launch_team_nr(hipStream_t st, const McsArgs &a, const TeamLayout &lay)
 {
     const dim3 grid((unsigned)((a.W + kTeams - 1) / kTeams)), block(kTeams * kTeam);
@@ -908,14 +942,14 @@ hipError_t launch_team_nr(hipStream_t st, const McsArgs &a, const TeamLayout &la
     const bool moms = FP64 && a.moms != nullptr && !joint;
     constexpr int MO = FP64 ? 2 : 0;
     void (*k)(McsArgs, TeamLayout) = nullptr;
-    if (a.L % 2) {
-        // odd L: lattices in LDS
-        k = moms ? k_mcs_team<R, FP64, KEYING, true, false, MO, false, NR, true>
+    if constexpr (ORD != 0) {
+        // lattices in LDS
+        k = moms ? k_mcs_team<R, FP64, KEYING, true, false, MO, false, NR, ORD>
             : lay.lds_hist
-                ? joint ? k_mcs_team<R, FP64, KEYING, true, true, 1, false, NR, true>
-                        : k_mcs_team<R, FP64, KEYING, true, true, 0, false, NR, true>
-            : joint ? k_mcs_team<R, FP64, KEYING, true, false, 1, false, NR, true>
-                    : k_mcs_team<R, FP64, KEYING, true, false, 0, false, NR, true>;
+                ? joint ? k_mcs_team<R, FP64, KEYING, true, true, 1, false, NR, ORD>
+                        : k_mcs_team<R, FP64, KEYING, true, true, 0, false, NR, ORD>
+            : joint ? k_mcs_team<R, FP64, KEYING, true, false, 1, false, NR, ORD>
+                    : k_mcs_team<R, FP64, KEYING, true, false, 0, false, NR, ORD>;
     } else if (lay.lnw_global) {
         // ln W too large for LDS (L >= 136): lattices and histogram stay in
         // HBM as well
@@ -957,12 +991,20 @@ hipError_t launch_team_nr(hipStream_t st, const McsArgs &a, const TeamLayout &la
 template <int R, bool FP64, int KEYING>
 hipError_t launch_team_r(hipStream_t st, const McsArgs &a, const TeamLayout &lay)
 {
-    const uint32_t rounds = (lay.row + 15) / 16;
-    if (lay.lnw_global) return launch_team_nr<R, FP64, KEYING, kLnwgRounds>(st, a, lay);
-    if (rounds <= 1) return launch_team_nr<R, FP64, KEYING, 1>(st, a, lay);
-    if (rounds <= 2) return launch_team_nr<R, FP64, KEYING, 2>(st, a, lay);
-    if (rounds <= 3) return launch_team_nr<R, FP64, KEYING, 3>(st, a, lay);
-    return launch_team_nr<R, FP64, KEYING, 4>(st, a, lay);   // longer half-rows in chunks of 64
+    if (lay.lnw_global) return launch_team_nr<R, FP64, KEYING, kLnwgRounds, 0>(st, a, lay);
+    if (lay.order == 1) {
+        if (lay.rounds == 1) return launch_team_nr<R, FP64, KEYING, 1, 1>(st, a, lay);
+        if (lay.rounds == 2) return launch_team_nr<R, FP64, KEYING, 2, 1>(st, a, lay);
+        return launch_team_nr<R, FP64, KEYING, 3, 1>(st, a, lay);
+    }
+    if (lay.order == 2) {
+        if (lay.rounds == 1) return launch_team_nr<R, FP64, KEYING, 1, 2>(st, a, lay);
+        return launch_team_nr<R, FP64, KEYING, 2, 2>(st, a, lay);
+    }
+    if (lay.rounds == 1) return launch_team_nr<R, FP64, KEYING, 1, 0>(st, a, lay);
+    if (lay.rounds == 2) return launch_team_nr<R, FP64, KEYING, 2, 0>(st, a, lay);
+    if (lay.rounds == 3) return launch_team_nr<R, FP64, KEYING, 3, 0>(st, a, lay);
+    return launch_team_nr<R, FP64, KEYING, 4, 0>(st, a, lay);
 }
 
 }  // namespace muca
