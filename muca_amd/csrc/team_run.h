@@ -62,12 +62,10 @@ constexpr int kTeam = 16;
 constexpr int kTeams = 16;   // per workgroup of 256 lanes
 constexpr uint32_t kXcds = 8;   // accelerator dies of an MI355X, one L2 each
 // D values per window (at most 8).  Narrower ones cut the mask work per pass and
-// make D leave them more often.  The weight path uses 8: L = 128, seeded 1.85
-// ms per launch against 1.90 with 6 and 2.03 with 4; L = 72 from ln W = 0 293,
-// 294 and 300 us.  The produce path (FP64 masks) uses 6: L = 256 with moments
-// 15.0 ms against 18.6 with 8, which spills; without 13.2 against 13.0.
-template <int KEYING>
-constexpr int kWinFor = KEYING == 1 ? 6 : 8;
+// make D leave them more often: L = 128, seeded 1.85 ms per launch against 1.90
+// with 6 and 2.03 with 4; FP64 production, L = 256, 12.9 against 13.4 with 6
+// (with moments 14.3 and 14.2), L = 72 0.43 against 0.46.
+constexpr int kWin = 8;
 // Rounds per chunk where ln W is in HBM: those launches have 128 VGPRs (four
 // wavefronts per SIMD), which two rounds' state fits without spills.  L = 256,
 // 16 384 walkers, 65 536 attempts each, with moments / without: 15.8 / 15.5 ms
@@ -229,7 +227,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                                          unsigned char *lds)
 {
     typedef typename std::conditional<FP64, double, float>::type T;
-    constexpr int KW = kWinFor<KEYING>;   // this launch's mask width (<= kWin)
+    constexpr int KW = kWin;
     constexpr bool ODD = ORD == 1, FLOW = ORD == 2;
     constexpr bool JOINT = OBS == 1, MOMS = OBS == 2, TRACKM = OBS >= 1;
     __syncthreads();   // LDS may still be read by a previous call's flush
