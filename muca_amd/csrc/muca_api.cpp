@@ -45,11 +45,12 @@ void free_ctx(muca_ctx *c)
 {
     if (!c) return;
     if (c->p.device >= 0) hipSetDevice(c->p.device);
-    void *bufs[] = {c->lat, c->E, c->D, c->M, c->lnw32, c->lnw64, c->order, c->naver,
+    void *bufs[] = {c->lat, c->E, c->D, c->M, c->lnw64, c->order, c->naver,
                     c->hist, c->joint, c->moms, c->mom, c->deltas, c->rw_out,
                     c->rw_flag};
     for (void *b : bufs)
         if (b) hipFree(b);
+    if (c->pin) hipHostFree(c->pin);
     if (c->ev0) hipEventDestroy(c->ev0);
     if (c->ev1) hipEventDestroy(c->ev1);
     if (c->st) hipStreamDestroy(c->st);
@@ -134,19 +135,20 @@ int muca_create(const muca_params *params, muca_ctx **out)
     c->cfg.fp64 = p.precision == MUCA_FP64;
     c->cfg.keying = p.keying;
     c->cfg.cus = c->cus;
-    // Kernel choice (measured on MI355X, L = 72): the team kernel keeps every
-    // SIMD busy when walkers are few (31 attempts/ns at 4096 walkers against
-    // 6.7 for one lane per walker); one lane per walker wins once there are
-    // enough wavefronts to hide its memory latency (58/ns at 65536 walkers
-    // against 28).  The crossover sits near 128 walkers per compute unit.
-    // Beyond that the lane kernel leads (213 against 147 at 524288 walkers),
-    // with 512-lane workgroups once there are enough of them to fill every
-    // compute unit twice (279 at 524288 walkers; 256 lanes stay ahead at
-    // 65536).  Even L that are no multiple of 8 follow the same rule (L = 100,
-    // 4100 walkers, FP32: 1.2 ms per launch against 6.7 ms for one lane per
-    // walker), and so do odd L while their lattices fit in LDS (L = 45, 2000
-    // walkers: 28 attempts/ns against 3.3 for the generic kernel; 65 536
-    // walkers 106 against 75).  muca_autotune replaces this rule by measurement.
+    // Kernel choice (attempts/ns on MI355X).  The team kernel keeps every SIMD
+    // busy when walkers are few (L = 72: 82 at 4096 walkers; 76 at 16 384
+    // against 37 for one lane per walker); the lane kernel wins once there
+    // are enough wavefronts to hide its memory latency.  They meet near 128
+    // walkers per compute unit (L = 64, 32 768 walkers: 80 against 73; 65 536:
+    // 80 against 149; L = 128 the same).  Where several workgroups of teams
+    // share a compute unit's LDS and half-rows fill a round the teams lead
+    // to twice that (L = 32, 65 536 walkers: 185 against 142; 131 072: 198
+    // against 243), and so they do at odd L against the generic kernel
+    // (L = 33, 65 536: 162 against 73; L = 63: 72 against 74).  With per-D
+    // moments the alternative is the generic kernel too: L = 72, 65 536 walkers
+    // 49 against 25, 131 072 42 against 57; below L = 64, where its atomics
+    // collide, at any number (L = 48, 262 144 walkers: 67 against 43; L = 32:
+    // 62 against 11).  muca_autotune replaces this rule by measurement.
     const uint64_t ncu = (uint64_t)(cu > 0 ? cu : 256);
     if (p.kernel == MUCA_KERNEL_AUTO) {
         // eligibility as the launch decides it (layout in this device's LDS)
@@ -156,14 +158,18 @@ int muca_create(const muca_params *params, muca_ctx **out)
         probe.W = W;
         probe.nup = 1;
         const size_t lds_probe = (size_t)(lds > 0 ? lds : 65536);
-        muca::TeamLayout lay_probe;
+        muca::TeamLayout lay_probe{};
         const bool team_ok = muca::team_layout(probe, p.precision == MUCA_FP64, lds_probe, lay_probe);
         const bool lane_ok = muca::lane_eligible(probe, p.precision == MUCA_FP64, lds_probe);
-        if (moments)
-            c->cfg.kernel = team_ok && (uint64_t)W <= 128ull * ncu ? MUCA_KERNEL_TEAM
-                                                                   : MUCA_KERNEL_GENERIC;
-        else if (team_ok && (uint64_t)W <= 128ull * ncu)
+        const uint64_t per_cu = moments ? (p.L < 64 ? UINT64_MAX / ncu : 256)
+                                : p.L >= 32 && (p.L % 2 || lay_probe.bytes * 3 <= lds_probe) &&
+                                        p.joint_blocks == 0
+                                    ? 256
+                                    : 128;
+        if (team_ok && (uint64_t)W <= per_cu * ncu)
             c->cfg.kernel = MUCA_KERNEL_TEAM;
+        else if (moments)
+            c->cfg.kernel = MUCA_KERNEL_GENERIC;
         else if (lane_ok)
             c->cfg.kernel = MUCA_KERNEL_LANE;
         else
@@ -209,8 +215,9 @@ int muca_create(const muca_params *params, muca_ctx **out)
     if (!rc) rc = dev_alloc(&c->E, W, "E");
     if (!rc) rc = dev_alloc(&c->D, W, "D");
     if (!rc) rc = dev_alloc(&c->M, W, "M");
-    if (!rc) rc = dev_alloc(&c->lnw32, N + 1, "lnw32");
-    if (!rc) rc = dev_alloc(&c->lnw64, N + 1, "lnw64");
+    // ln W in both precisions, one copy per set
+    if (!rc) rc = dev_alloc(&c->lnw64, (N + 1) * 3 / 2 + 1, "lnw");
+    if (!rc) c->lnw32 = (float *)(c->lnw64 + N + 1);
     if (!rc) rc = dev_alloc(&c->order, N, "order");
     if (!rc) rc = dev_alloc(&c->naver, 4 * N, "naver");
     if (!rc) rc = dev_alloc(&c->hist, N + 1, "hist");
@@ -235,6 +242,7 @@ int muca_create(const muca_params *params, muca_ctx **out)
     std::vector<uint32_t> naver, order;
     make_tables(p.L, naver, order);
     hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->pin, (N + 1) * 12, hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
     if (e == hipSuccess)
@@ -368,14 +376,15 @@ int muca_set_log_weight(muca_ctx *c, const double *lnw, uint32_t nbins)
 {
     if (!c || !lnw) return fail(MUCA_E_ARG, "NULL argument");
     if (nbins != c->N + 1) return fail(MUCA_E_ARG, "nbins must be N+1");
-    std::vector<float> f(nbins);
-    for (uint32_t i = 0; i < nbins; i++) {
+    for (uint32_t i = 0; i < nbins; i++)
         if (!std::isfinite(lnw[i])) return fail(MUCA_E_ARG, "ln W must be finite");
-        f[i] = (float)lnw[i];
-    }
+    double *w64 = (double *)c->pin;
+    float *w32 = (float *)(w64 + nbins);
+    memcpy(w64, lnw, nbins * sizeof(double));
+    for (uint32_t i = 0; i < nbins; i++) w32[i] = (float)lnw[i];
     HIP_TRY(hipSetDevice(c->p.device));
-    HIP_TRY(hipMemcpy(c->lnw64, lnw, nbins * sizeof(double), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(c->lnw32, f.data(), nbins * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(muca::launch_copy(c->st, c->lnw64, c->pin, nbins * 12ull));
+    HIP_TRY(hipStreamSynchronize(c->st));
     c->have_weights = true;
     return MUCA_OK;
 }
@@ -425,10 +434,10 @@ int muca_run(muca_ctx *c, uint32_t iter, uint32_t seed, uint64_t therm, uint64_t
     HIP_TRY(hipEventRecord(c->ev0, c->st));
     HIP_TRY(muca::launch_mcs(c->st, c->cfg, a));
     HIP_TRY(hipEventRecord(c->ev1, c->st));
-    HIP_TRY(hipEventSynchronize(c->ev1));
+    if (hist_out) HIP_TRY(muca::launch_copy(c->st, c->pin, c->hist, (N + 1) * sizeof(uint64_t)));
+    HIP_TRY(hipStreamSynchronize(c->st));
     if (kernel_ms) HIP_TRY(hipEventElapsedTime(kernel_ms, c->ev0, c->ev1));
-    if (hist_out)
-        HIP_TRY(hipMemcpy(hist_out, c->hist, (N + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost));
+    if (hist_out) memcpy(hist_out, c->pin, (N + 1) * sizeof(uint64_t));
     return MUCA_OK;
 }
 
