@@ -36,7 +36,7 @@ struct muca_ctx {
     float *lnw32 = nullptr;
     double *lnw64 = nullptr;
     uint32_t *order = nullptr, *naver = nullptr;
-    void *pin = nullptr;        // pinned, 12 (N + 1) bytes: ln W in, histogram out
+    void *pin = nullptr;        // pinned, 20 N + 12 bytes: site tables and ln W in, histogram out
     uint64_t *hist = nullptr;
     uint64_t *joint = nullptr;
     uint64_t *moms = nullptr;   // MUCA_OBS_MOMENTS: blocks * kMomWords * (N+1)

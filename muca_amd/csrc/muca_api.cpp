@@ -45,7 +45,7 @@ void free_ctx(muca_ctx *c)
 {
     if (!c) return;
     if (c->p.device >= 0) hipSetDevice(c->p.device);
-    void *bufs[] = {c->lat, c->E, c->D, c->M, c->lnw64, c->order, c->naver,
+    void *bufs[] = {c->lat, c->E, c->D, c->M, c->lnw64, c->naver,
                     c->hist, c->joint, c->moms, c->mom, c->deltas, c->rw_out,
                     c->rw_flag};
     for (void *b : bufs)
@@ -218,8 +218,8 @@ int muca_create(const muca_params *params, muca_ctx **out)
     // ln W in both precisions, one copy per set
     if (!rc) rc = dev_alloc(&c->lnw64, (N + 1) * 3 / 2 + 1, "lnw");
     if (!rc) c->lnw32 = (float *)(c->lnw64 + N + 1);
-    if (!rc) rc = dev_alloc(&c->order, N, "order");
-    if (!rc) rc = dev_alloc(&c->naver, 4 * N, "naver");
+    if (!rc) rc = dev_alloc(&c->naver, 5 * N, "site tables");   // naver, then order
+    if (!rc) c->order = c->naver + 4 * N;
     if (!rc) rc = dev_alloc(&c->hist, N + 1, "hist");
     if (!rc && p.joint_blocks > 0) {
         if (p.joint_blocks > W) {
@@ -242,13 +242,14 @@ int muca_create(const muca_params *params, muca_ctx **out)
     std::vector<uint32_t> naver, order;
     make_tables(p.L, naver, order);
     hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->pin, (N + 1) * 12, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->pin, N * 20 + 12, hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
-    if (e == hipSuccess)
-        e = hipMemcpy(c->naver, naver.data(), naver.size() * 4, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(c->order, order.data(), order.size() * 4, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        memcpy(c->pin, naver.data(), 16 * N);
+        memcpy((char *)c->pin + 16 * N, order.data(), 4 * N);
+        e = muca::launch_copy(c->st, c->naver, c->pin, 20 * N);
+    }
     // on the context's stream: one of the null stream would not be ordered
     // before the launches that follow
     if (e == hipSuccess) e = hipMemsetAsync(c->lat, 0, N * W, c->st);

@@ -211,9 +211,8 @@ __global__ __launch_bounds__(kStateParts *kStateLanes) void k_state(const int8_t
 }
 
 // A few kilobytes between pinned host memory and the device as part of the
-// stream's work: a copy of its own engine costs more than the data does (a
-// histogram of 257 bins back to the host: run call 42 us with a blocking copy
-// after it, @@ us with this one before its synchronization).
+// stream's work: a blocking copy of its own costs more than the data does (257
+// bins: a run that returns the histogram 42 -> 32 us, setting ln W 30 -> 15 us).
 __global__ __launch_bounds__(256) void k_copy(uint32_t *dst, const uint32_t *src, uint32_t words)
 {
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) dst[i] = src[i];

@@ -178,6 +178,7 @@ static void (*batch_team_kernel(int lat_modes, int nrs))(BatchArgs)
         default: return k_batch_team<FP64, 1, 0>;
         }
     }
+    if (lat_modes == 2 && nrs == 4) return k_batch_team<FP64, 2, 4>;
     return lat_modes == 2 ? k_batch_team<FP64, 2, 0> : k_batch_team<FP64, 3, 0>;
 }
 
