@@ -22,7 +22,6 @@ MUCA_TEAM_EXTERN(10, true, 1)
 bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
 {
     if (a.L < 8 || a.L > 256) return false;
-    const size_t tsz = fp64 ? 8 : 4;
     const size_t row = (a.L + 1) / 2;   // the longest chunk
     auto al = [](size_t x) { return (x + 15) & ~(size_t)15; };
     lay.row = (uint32_t)row;
@@ -36,12 +35,16 @@ bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
     // they replace the D histogram
     const bool moms = fp64 && a.moms != nullptr && a.joint == nullptr;
     const size_t mbytes = moms ? kMomLdsWords * kMomSlots * sizeof(uint64_t) : 0;
-    const size_t fixed = 256 * sizeof(double);   // the acceptance-log table
-    // ln W in LDS when it fits (with the guards), else read from HBM, where it
-    // stays in L2 (512 KB at L = 256 in FP64), one window per team at a time
-    const size_t wbytes = al((a.N + 1 + 2 * kGuard) * tsz);
-    lay.lnw_global = al((lay.off_win + mbytes) * kTeams) + fixed + wbytes > lds_max;
-    lay.off_mom = (uint32_t)(lay.off_win + (lay.lnw_global ? al(kWinCache * tsz) : 0));
+    const size_t fixed = 256 * sizeof(double) + 16;   // the acceptance-log table, FP64 bounds
+    // ln W (FP64: its differences in FP32) in LDS when it fits (with the
+    // guards), else read from HBM, where it stays in L2 (512 KB at L = 256 in
+    // FP64), one window per team at a time.  FP64 differences would fit to
+    // L = 192, but one workgroup per compute unit then does less than four
+    // whose windows come from L2.
+    const size_t wbytes = al((a.N + 1 + 2 * kGuard) * sizeof(float));
+    lay.lnw_global =
+        al((lay.off_win + mbytes) * kTeams) + fixed + wbytes * (fp64 ? 2 : 1) > lds_max;
+    lay.off_mom = (uint32_t)(lay.off_win + (lay.lnw_global ? al(kWinCache * sizeof(float)) : 0));
     lay.team_bytes = (uint32_t)(lay.off_mom + mbytes);
     size_t off = 0;
     lay.off_team = 0;

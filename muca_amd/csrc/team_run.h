@@ -71,7 +71,10 @@ constexpr int kWin = 8;
 // 16 384 walkers, 65 536 attempts each, with moments / without: 15.8 / 15.5 ms
 // with two rounds, 16.8 / 16.1 with three, 18.5 / 16.0 with four.
 constexpr int kLnwgRounds = 2;
-constexpr int kWinCache = 64;   // ln W values per team in LDS where ln W is in HBM
+// ln W values (FP64: differences) per team in LDS where ln W is in HBM: 64 are
+// loaded again more often (L = 256, 16 384 walkers 13.3 ms against 12.9), 256
+// cost more per load (with moments 15.7 against 14.2)
+constexpr int kWinCache = 128;
 constexpr int kGuard = 24;   // ln W guard entries on each side (> kWin / 2 + 2)
 
 __device__ __forceinline__ void wave_sync()
@@ -91,10 +94,6 @@ __device__ __forceinline__ uint32_t sign_word(float x)
 {
     return __float_as_uint(x);
 }
-__device__ __forceinline__ uint32_t sign_word(double x)
-{
-    return (uint32_t)(__double_as_longlong(x) >> 32);
-}
 
 // value of lane L of this lane's 16-lane row (v_mov_b32_dpp row_newbcast:L;
 // every lane of the row reads a valid source, so no old value is needed)
@@ -102,17 +101,6 @@ template <int L>
 __device__ __forceinline__ int32_t row_bcast(int32_t v)
 {
     return __builtin_amdgcn_mov_dpp(v, 0x150 + L, 0xf, 0xf, false);
-}
-
-// a monotone FP32 image of |x|'s order: x itself, or the high word of a double
-// read as a float (magnitudes above 2^1016 read as NaN, which a minimum skips)
-__device__ __forceinline__ float mag_word(float x)
-{
-    return x;
-}
-__device__ __forceinline__ float mag_word(double x)
-{
-    return __uint_as_float((uint32_t)(__double_as_longlong(x) >> 32));
 }
 
 // The proposal byte of an attempt: bits 0-1 hold dDel + 1, 2-4 the spin change
@@ -226,12 +214,13 @@ template <int R, bool FP64, int KEYING, bool LATLDS, bool LDSHIST, int OBS, bool
 __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay, uint64_t wbase,
                                          unsigned char *lds)
 {
-    typedef typename std::conditional<FP64, double, float>::type T;
     constexpr int KW = kWin;
     constexpr bool ODD = ORD == 1, FLOW = ORD == 2;
     constexpr bool JOINT = OBS == 1, MOMS = OBS == 2, TRACKM = OBS >= 1;
     __syncthreads();   // LDS may still be read by a previous call's flush
-    T *wt = (T *)(lds + lay.off_w) + kGuard;   // valid for [-kGuard, N + kGuard]
+    // FP32: ln W.  FP64: ln W[D + 1] - ln W[D] in FP32, for the screening of
+    // `pass`; its exact test reads ln W from HBM.  Valid for [-kGuard, N + kGuard]
+    float *wt = (float *)(lds + lay.off_w) + kGuard;
     uint32_t *hist = (uint32_t *)(lds + lay.off_hist);
     int8_t *latl = (int8_t *)(lds + lay.off_lat);
     double *logtab = (double *)(lds + lay.off_tab);
@@ -239,16 +228,21 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     const uint32_t N = a.N, L = a.L, Rw = lay.row;
     unsigned char *tbase = lds + lay.off_team + (size_t)team * lay.team_bytes;
     uint32_t *rng = (uint32_t *)tbase;                          // [2][ring][4]
-    T *winb = (T *)(tbase + lay.off_win);                       // LNWG: lnW[wb .. wb + kWinCache - 1]
-    // ln W at any D: from LDS, or from HBM (clamped into [0, N]; only
-    // positions a walker cannot be at read a clamped value)
-    auto lnw_at = [&](int32_t i) -> T {
-        if (LNWG) {
-            const int32_t c = min(max(i, 0), (int32_t)a.N);
-            return FP64 ? (T)a.lnw64[c] : (T)a.lnw32[c];
-        }
-        return wt[i];
+    float *winb = (float *)(tbase + lay.off_win);               // LNWG: wt[wb .. wb + kWinCache - 1]
+    // wt's value at any D from HBM (only positions a walker cannot be at read
+    // one from outside [0, N]); FP64: `bound` grows to the error that the
+    // screening has to allow for it, 2^-22 |value| for the FP32 arithmetic and
+    // 2^-50 |ln W| for the rounding of the exact FP64 difference
+    auto lnw_at = [&](int32_t i, float &bound) -> float {
+        const int32_t c = min(max(i, 0), (int32_t)a.N - (FP64 ? 1 : 0));
+        if (!FP64) return a.lnw32[c];
+        const double from = a.lnw64[c], to = a.lnw64[c + 1];
+        const float g = (float)(to - from);
+        bound = fmaxf(bound, fabsf(g) * 0x1p-22f + (float)(fabs(from) + fabs(to)) * 0x1p-50f);
+        return g;
     };
+    float gbound = 0.0f;   // FP64: the largest bound of wt (LNWG: of the team's window)
+    float *const wave_bound = (float *)(lds + lay.off_tab + 256 * sizeof(double));
 
     const uint64_t W = a.W;
     const uint64_t w = wbase + team;
@@ -256,10 +250,12 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
 
     if (!LNWG) {
 #pragma unroll 4
-        for (int i = (int)tid - kGuard; i <= (int)N + kGuard; i += blockDim.x) {
-            T v = (T)0;
-            if (i >= 0 && i <= (int)N) v = FP64 ? (T)a.lnw64[i] : (T)a.lnw32[i];
-            wt[i] = v;
+        for (int i = (int)tid - kGuard; i <= (int)N + kGuard; i += blockDim.x)
+            wt[i] = lnw_at(i, gbound);
+        if (FP64) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) gbound = fmaxf(gbound, __shfl_xor(gbound, off));
+            if ((tid & 63) == 0) wave_bound[tid >> 6] = gbound;
         }
     }
     // MOMS: this team's moment slots, word k of slot s at msl[k * kMomSlots + s]
@@ -308,6 +304,8 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
         }
     }
     __syncthreads();
+    if (FP64 && !LNWG)
+        gbound = fmaxf(fmaxf(wave_bound[0], wave_bound[1]), fmaxf(wave_bound[2], wave_bound[3]));
 
     if (active) {
         // The walker's spin at x of a row: the row's address is the same in
@@ -357,6 +355,9 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 for (int k = 0; k < kMomLdsWords; k++) msl[k * kMomSlots + tl] = 0;
             }
         };
+        // FP64: the part of the screening's limit that is the same for all
+        // attempts (|beta dE| <= 8 |beta|)
+        const float limc = (8.0f * fabsf((float)a.beta) + 1.0f) * 0x1p-22f;
         uint32_t c0base = 0;
         const uint32_t RB = lay.ring;
         uint32_t gen = 0, gen_slot = 0, cur_slot = 0;   // next block to make, its slot, block blk0's slot
@@ -371,17 +372,22 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
         int32_t pf_s[NR], pf_r[NR], pf_l[NR], pf_u[NR], pf_d[NR], fin[NR];
         bool pf_have = false, pf_fwd = false;
         int32_t de_lane = 0, dm_lane = 0;
-        // lnW[dc - KW/2 + k] at [k], k = -1 .. KW.  LNWG: from the team's
+        // wt[dc - KW/2 + k] at [k], k = -1 .. KW.  LNWG: from the team's
         // window of kWinCache values in LDS, staged again around dc when it
         // does not hold them
         int32_t wb = -(1 << 30);
-        auto window = [&](int32_t dc) -> const T * {
+        auto window = [&](int32_t dc) -> const float * {
             if (!LNWG) return wt + dc - KW / 2;
             if (dc - KW / 2 - 1 < wb || dc + KW / 2 >= wb + kWinCache) {
                 wb = dc - kWinCache / 2;
-#pragma unroll
+                gbound = 0.0f;
+#pragma unroll 4
                 for (int i = 0; i < kWinCache / kTeam; i++)
-                    winb[kTeam * i + tl] = lnw_at(wb + kTeam * i + (int32_t)tl);
+                    winb[kTeam * i + tl] = lnw_at(wb + kTeam * i + (int32_t)tl, gbound);
+                if (FP64)
+#pragma unroll
+                    for (int off = 8; off > 0; off >>= 1)
+                        gbound = fmaxf(gbound, __shfl_xor(gbound, off, kTeam));
                 wave_sync();
             }
             return winb + (dc - KW / 2 - wb);
@@ -549,7 +555,8 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     r1[r] = rng[widx];
                     r3[r] = rng[ringw + widx];
                 }
-                T fde[NR];
+                // FP32: -beta dE; FP64: the screened log less it
+                float fde[NR];
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
                     const uint32_t at = proposal_index(old_s[r], r3[r]);
@@ -558,8 +565,10 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     thi[r] = acclog_screen(r1[r]);
                     const int32_t dE = __mul24(mds, nb[r]);
                     info[r] = (int32_t)pr | ((dE + 8) << 8);
-                    // past the chunk's end: -inf accepts nowhere
-                    fde[r] = 16 * r + (uint32_t)tl < cnt ? (T)(-(double)dE * a.beta) : -(T)INFINITY;
+                    // past the chunk's end: accepted nowhere
+                    const float f = (float)(-(double)dE * a.beta);
+                    const bool in = 16 * r + (uint32_t)tl < cnt;
+                    fde[r] = FP64 ? (in ? thi[r] - f : INFINITY) : (in ? f : -INFINITY);
                     // made here, not where the round uses them: that would put
                     // their latency into the chain
                     asm volatile("" : "+v"(info[r]), "+v"(fde[r]), "+v"(thi[r]));
@@ -635,48 +644,78 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     if (j0 >= cnt) continue;
                     const bool valid = j0 + tl < cnt;
                     // The window around D = dc before step `from` of the round;
-                    // the steps before it are identities (fde = -inf accepts
-                    // nowhere).  Byte k of (lo, hi): accept at dlo + k, i.e.
+                    // the steps before it are identities (accepted nowhere).
+                    // Byte k of (lo, hi): accept at dlo + k, i.e.
                     // acclog(r1) < ((fde + lnW[dlo + k + dDel]) - lnW[dlo + k]),
-                    // screened: the sign of e = thi - diff (e is -0 never); a
-                    // diff with 0 <= e < lim needs the exact log -- flagged by
-                    // min |e| < lim, the minimum taken over mag_word (exact in
-                    // FP32, the high words in FP64, compared there with <=).
+                    // screened: the sign of e = thi - diff; |e| < lim needs the
+                    // exact test.  FP64 screens with FP32 differences of ln W
+                    // (lim allows for them): one load and one fma per position
+                    // and half the LDS, against two loads and three additions of
+                    // doubles (L = 72, 4096 walkers: thermalization launch 432 ->
+                    // 380 us, joint 728 -> 673; L = 256 waits for memory: the same).
                     // o: the window position after this lane's step; before:
                     // the one before it; ok: accepted there.
                     auto pass = [&](int32_t dc, uint32_t from, uint32_t &o, uint32_t &before,
                                     bool &ok) {
-                        const T *wc = window(dc);
-                        const T *wto = wc + i_ddel(info[r]);
-                        const T fd = (uint32_t)tl >= from ? fde[r] : -(T)INFINITY;
-                        T diff[KW];
-#pragma unroll
-                        for (int k = 0; k < KW; k++) {
-                            diff[k] = fd + wto[k];
-                            diff[k] = diff[k] - wc[k];
-                        }
+                        const float *wc = window(dc);
+                        const int32_t dd = i_ddel(info[r]);
                         uint32_t sg[8], lo, hi;
-                        float emin = 1e30f;
-                        const T th = (T)thi[r];
+                        float emin = 1e30f, diff[KW];
+                        float lim = acclog_screen_lim(thi[r]);
+                        if constexpr (FP64) {
+                            // thi - diff = (thi + beta dE) -+ the step's difference
+                            const float *wq = wc + min(dd, 0), step = -(float)dd;
+                            const float base = (uint32_t)tl >= from ? fde[r] : INFINITY;
+                            lim += (limc - thi[r] * 0x1p-22f) + gbound;
 #pragma unroll
-                        for (int k = 0; k < KW; k++) {
-                            const T e = th - diff[k];
-                            sg[k] = sign_word(e);
-                            emin = fminf(emin, fabsf(mag_word(e)));
+                            for (int k = 0; k < KW; k++) {
+                                const float e = __builtin_fmaf(step, wq[k], base);
+                                sg[k] = sign_word(e);
+                                emin = fminf(emin, fabsf(e));
+                            }
+                        } else {
+                            const float *wto = wc + dd;
+                            const float fd = (uint32_t)tl >= from ? fde[r] : -INFINITY;
+#pragma unroll
+                            for (int k = 0; k < KW; k++) {
+                                diff[k] = fd + wto[k];
+                                diff[k] = diff[k] - wc[k];
+                            }
+#pragma unroll
+                            for (int k = 0; k < KW; k++) {
+                                const float e = thi[r] - diff[k];
+                                sg[k] = sign_word(e);
+                                emin = fminf(emin, fabsf(e));
+                            }
                         }
                         sign_bytes<KW>(sg, lo, hi);
-                        const float lim = mag_word((T)acclog_screen_lim(thi[r]));
-                        const bool amb = FP64 ? emin <= lim : emin < lim;
+                        const bool amb = !(emin >= lim);
                         if (__builtin_amdgcn_ballot_w64(amb)) {   // rare
                             if (amb) {
                                 uint32_t w1 = s4 + j0 + tl;
                                 w1 = w1 >= ringw ? w1 - ringw : w1;
-                                const T tlog = (T)(float)acclog_u01_double_tab(rng[w1], logtab,
-                                                                               logtab + 128);
+                                const float tlog = (float)acclog_u01_double_tab(rng[w1], logtab,
+                                                                                logtab + 128);
+                                if constexpr (FP64) {
+                                    const double f = -(double)i_dE(info[r]) * a.beta;
+                                    const bool live = (uint32_t)tl >= from && fde[r] < INFINITY;
+                                    uint64_t bytes = 0;
+#pragma unroll 1
+                                    for (int k = 0; k < KW; k++) {
+                                        const int32_t at = dc - KW / 2 + k;
+                                        const double x = f + a.lnw64[min(max(at + dd, 0), (int32_t)N)];
+                                        if (live &&
+                                            (double)tlog < x - a.lnw64[min(max(at, 0), (int32_t)N)])
+                                            bytes |= 0xffull << (8 * k);
+                                    }
+                                    lo = (uint32_t)bytes;
+                                    hi = (uint32_t)(bytes >> 32);
+                                } else {
 #pragma unroll
-                                for (int k = 0; k < KW; k++)
-                                    sg[k] = tlog < diff[k] ? 0x80000000u : 0u;
-                                sign_bytes<KW>(sg, lo, hi);
+                                    for (int k = 0; k < KW; k++)
+                                        sg[k] = tlog < diff[k] ? 0x80000000u : 0u;
+                                    sign_bytes<KW>(sg, lo, hi);
+                                }
                             }
                         }
                         uint32_t plo, phi;   // the map of steps 0..tl
