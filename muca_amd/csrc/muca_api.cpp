@@ -145,10 +145,11 @@ int muca_create(const muca_params *params, muca_ctx **out)
     // to twice that (L = 32, 65 536 walkers: 185 against 142; 131 072: 198
     // against 243), and so they do at odd L against the generic kernel
     // (L = 33, 65 536: 162 against 73; L = 63: 72 against 74).  With per-D
-    // moments the alternative is the generic kernel too: L = 72, 65 536 walkers
-    // 49 against 25, 131 072 42 against 57; below L = 64, where its atomics
-    // collide, at any number (L = 48, 262 144 walkers: 67 against 43; L = 32:
-    // 62 against 11).  muca_autotune replaces this rule by measurement.
+    // moments the alternative is the generic kernel, whose atomics collide: at
+    // even L and below L = 64 teams lead at any number (L = 72, 65 536 walkers:
+    // 85 against 25; L = 128: 97 against 45; L = 48, 262 144: 67 against 43),
+    // at larger odd L as without.  muca_autotune replaces this rule by
+    // measurement.
     const uint64_t ncu = (uint64_t)(cu > 0 ? cu : 256);
     if (p.kernel == MUCA_KERNEL_AUTO) {
         // eligibility as the launch decides it (layout in this device's LDS)
@@ -161,7 +162,7 @@ int muca_create(const muca_params *params, muca_ctx **out)
         muca::TeamLayout lay_probe{};
         const bool team_ok = muca::team_layout(probe, p.precision == MUCA_FP64, lds_probe, lay_probe);
         const bool lane_ok = muca::lane_eligible(probe, p.precision == MUCA_FP64, lds_probe);
-        const uint64_t per_cu = moments ? (p.L < 64 ? UINT64_MAX / ncu : 256)
+        const uint64_t per_cu = moments ? (p.L % 2 == 0 || p.L < 64 ? UINT64_MAX / ncu : 256)
                                 : p.L >= 32 && (p.L % 2 || lay_probe.bytes * 3 <= lds_probe) &&
                                         p.joint_blocks == 0
                                     ? 256

@@ -19,7 +19,8 @@ MUCA_TEAM_EXTERN(10, true, 0)
 MUCA_TEAM_EXTERN(10, true, 1)
 #undef MUCA_TEAM_EXTERN
 
-bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
+// windows: ln W read from HBM and lattices left there whether or not they fit
+static bool place(const McsArgs &a, int fp64, size_t lds_max, bool windows, TeamLayout &lay)
 {
     if (a.L < 8 || a.L > 256) return false;
     const size_t row = (a.L + 1) / 2;   // the longest chunk
@@ -43,7 +44,7 @@ bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
     // whose windows come from L2.
     const size_t wbytes = al((a.N + 1 + 2 * kGuard) * sizeof(float));
     lay.lnw_global =
-        al((lay.off_win + mbytes) * kTeams) + fixed + wbytes * (fp64 ? 2 : 1) > lds_max;
+        windows || al((lay.off_win + mbytes) * kTeams) + fixed + wbytes * (fp64 ? 2 : 1) > lds_max;
     lay.off_mom = (uint32_t)(lay.off_win + (lay.lnw_global ? al(kWinCache * sizeof(float)) : 0));
     lay.team_bytes = (uint32_t)(lay.off_mom + mbytes);
     size_t off = 0;
@@ -65,7 +66,7 @@ bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
     uint32_t stride = (uint32_t)((a.N + 3) & ~3u);
     while ((stride / 4) % 32 != 8) stride += 4;
     lay.lat_stride = stride;
-    lay.lat_lds = off + al((size_t)stride * kTeams) <= lds_max;
+    lay.lat_lds = !windows && off + al((size_t)stride * kTeams) <= lds_max;
     if (lay.lat_lds) off += al((size_t)stride * kTeams);
     lay.bytes = off;
     // Where the last round of a half-row would be at most half full, chunks of
@@ -81,6 +82,26 @@ bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
     // lattices in HBM are addressed by a 32-bit offset within a row
     if (!lay.lat_lds && (uint64_t)a.L * a.W > 0xffffffffull) return false;
     return off <= lds_max;
+}
+
+bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
+{
+    if (!place(a, fp64, lds_max, false, lay)) return false;
+    // Per-D moments need no histogram, so with windows of ln W from HBM four
+    // workgroups share a compute unit (128 VGPRs).  That leads as soon as there
+    // are more walkers than the LDS layout keeps resident (attempts/ns; L = 128:
+    // 8192 walkers 55 -> 80, 65 536 54 -> 97; 4096 55 against 49; L = 72: 16 384
+    // 57 -> 76; L = 96, three workgroups per compute unit: 16 384 82 -> 90, 8192
+    // 78 against 75), but not where two workgroups with their lattices fit
+    // (L = 48, 16 384: 89 against 80).  Odd L need their lattices in LDS.
+    const uint64_t per_cu = lds_max / lay.bytes;
+    const bool moms = fp64 && a.moms != nullptr && a.joint == nullptr;
+    TeamLayout win;
+    if (moms && a.L % 2 == 0 && !lay.lnw_global &&
+        (per_cu == 1 || (!lay.lat_lds && per_cu < 4)) && a.W > kTeams * kCus * per_cu &&
+        place(a, fp64, lds_max, true, win))
+        lay = win;
+    return true;
 }
 
 hipError_t launch_mcs_team(hipStream_t st, const Launch &cfg, const McsArgs &a,

@@ -60,6 +60,7 @@ namespace team_detail {
 
 constexpr int kTeam = 16;
 constexpr int kTeams = 16;   // per workgroup of 256 lanes
+constexpr uint64_t kCus = 256;   // compute units
 constexpr uint32_t kXcds = 8;   // accelerator dies of an MI355X, one L2 each
 // D values per window (at most 8).  Narrower ones cut the mask work per pass and
 // make D leave them more often: L = 128, seeded 1.85 ms per launch against 1.90
@@ -769,7 +770,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                         m += row_bcast<15>(x);
                     }
                     // ---- C: accepted spins, dE / dM sums, histogram of the round
-                    const uint32_t j = j0 + tl, left = min(cnt - j0, 16u);
+                    const uint32_t left = min(cnt - j0, 16u);
                     const int32_t ns = i_new(info[r]), ds = i_ds(info[r]);   // the proposal
                     // the site's spin after this chunk
                     if (PF) fin[r] = valid ? (acc ? ns : ns - ds) : -9;
