@@ -9,28 +9,28 @@
 // neighbour of a half-row was last written by an earlier half-row.  So per
 // chunk of a half-row (up to 64 attempts) the team
 //   A. computes in parallel, attempt j on lane j % 16 of round j / 16: the
-//      Philox blocks, the proposed spin, dE, dDel, (T)(-dE*beta) and the
-//      screened log of r1, for all rounds of the chunk at once;
-//   B. resolves the D chain round by round: for each of a window of 8 (weight
-//      path) or 6 (produce path) D values around the one the round starts at,
-//      whether the attempt accepts there (one byte each; the exact log only
-//      where the screen is inconclusive).  An attempt is then a map of window
-//      positions, eight bytes wide; v_perm_b32 looks four of them up at once,
-//      so sixteen lanes' maps compose in a prefix scan of four DPP steps.
-//      Where D leaves the window, the steps after that are done again around
-//      the D reached;
+//      Philox blocks, the proposed spin, dE, dDel, -dE*beta and the screened
+//      log of r1, for all rounds of the chunk at once;
+//   B. resolves the D chain round by round: for each of a window of 8 D values
+//      around the one the round starts at, whether the attempt accepts there
+//      (one byte each; the exact test only where the screen is inconclusive).
+//      An attempt is then a map of window positions, eight bytes wide;
+//      v_perm_b32 looks four of them up at once, so sixteen lanes' maps compose
+//      in a prefix scan of four DPP steps.  Where D leaves the window, the steps
+//      after that are done again around the D reached;
 //   C. writes the accepted spins, sums dE and dM and fills the histogram.
 // Bound by one wavefront's issue and latency (a dependent VALU instruction
-// takes 8.6 cycles, an independent one 5.2, a branch 21 to 37).  Measured
-// against a serial chain of one DPP broadcast, bit extract and add per attempt
-// over masks made once per chunk: L = 72, 4096 walkers, from ln W = 0: 293 us
-// per launch against 381; L = 128, seeded, NUPDATES = N: 1.85 against 2.51 ms;
-// L = 72 thermalisation in FP64: 0.48 against 0.96 ms; L = 256, 16 384
-// walkers: 13.3 against 26.1 ms, with moments 15.0 against 19.5.  The scan
-// alone, over masks per chunk: 341 us, 2.19, 0.63, 15.5 and 15.8 ms: D leaves
-// a window of 8 around a chunk's start 0.2 to 1.3 times a round (L = 72 from
-// ln W = 0; seeded L = 128), one around the round's start 0.03 to 0.6 times.
-// Every acceptance is computed with the reference's operations and rounding:
+// takes 8.6 cycles, an independent one 5.2, a branch 21 to 37; L = 72: 22 % of
+// the cycles in the Philox passes, 13 in A, 50 in B, 8 in C).  Measured against
+// a serial chain of one DPP broadcast, bit extract and add per attempt over
+// masks made once per chunk, one chunk per half-row: L = 72, 4096 walkers, from
+// ln W = 0: 255 us per launch against 381; L = 128, seeded, NUPDATES = N: 1.86
+// against 2.51 ms; L = 72 thermalization in FP64: 0.38 against 0.96 ms; L = 256,
+// 16 384 walkers: 12.9 against 26.1 ms, with moments 14.2 against 19.5.  The
+// scan alone, over masks per chunk, gave 341 us, 2.19, 0.63, 15.5 and 15.8 ms:
+// D leaves a window of 8 around a chunk's start 0.2 to 1.3 times a round (L = 72
+// from ln W = 0; seeded L = 128), one around the round's start 0.03 to 0.6 times.
+// Every acceptance is decided by the reference's operations and rounding:
 //   diff = ((T)(-dE*beta) + lnW[D+dDel]) - lnW[D];  accept iff diff >= 0 or
 //   acclog(r1) < diff.  Because acclog(r1) < 0 always, that is exactly
 //   acclog(r1) < diff.  Results are bit-identical to the one-lane kernel.
@@ -40,12 +40,13 @@
 // indices 0, 2, .., N-3 twice and then N-2 (muca_delta_multigpu.cu:173).  Two
 // of them are neighbours only across a wrap: x = 0 and L-1 of an even row, and
 // rows 0 and L-1.  Chunks end at x = L-3 of an even row and at x = L-2 of an
-// odd one, which separates both.
+// odd one, which separates both, or are no longer than the (L - 1) / 2 attempts
+// that lie between such neighbours.
 //
-// LDS (dynamic): per team a ring of Philox blocks [2 keys][(min(L/2, 64) + 6)/4 + 8][4]; the
-// acceptance-log table; (T)(-dE*beta) for dE = -8..8; ln W with guard entries
-// on each side; the D histogram (u32, when it fits); the workgroup's lattices
-// [N][16] int8 (when they fit).
+// LDS (dynamic): per team a ring of Philox blocks [2 keys][(min(L/2, 64) + 6)/4 + 8][4]
+// and, where ln W stays in HBM, a window of it; the acceptance-log table; ln W
+// (FP64: its differences) with guard entries on each side; the D histogram (u32,
+// when it fits); the workgroup's lattices [N][16] int8 (when they fit).
 #pragma once
 #include "kernels.h"
 
