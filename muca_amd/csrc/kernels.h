@@ -47,6 +47,12 @@ struct Launch {
 hipError_t launch_init_lattice(hipStream_t st, int8_t *lat, uint64_t W, uint32_t N,
                                int keying, int rounds, uint32_t mm, uint32_t gpu,
                                uint32_t seed, uint32_t w_offset, uint32_t strat_W = 0);
+// the state of every instance of a batch (inst: device memory); tiles: the
+// largest state_tiles of them
+uint32_t state_tiles(uint64_t W, const int8_t *lat);
+struct BatchInst;
+hipError_t launch_state_batch(hipStream_t st, const BatchInst *inst, uint32_t n, uint32_t tiles,
+                              const int8_t *lat, int32_t *E, int32_t *D, int32_t *M);
 // dst, src: device or pinned host memory; bytes a multiple of four
 hipError_t launch_copy(hipStream_t st, void *dst, const void *src, uint64_t bytes);
 hipError_t launch_state(hipStream_t st, const int8_t *lat, uint64_t W, uint32_t L, int32_t *E,

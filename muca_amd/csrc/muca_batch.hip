@@ -614,12 +614,12 @@ int batch_init(muca_batch *b, uint32_t mm, int stratified)
     b->stratified = stratified;
     BHIP(hipSetDevice(b->device));
     muca::BatchArgs &A = b->a;
+    uint32_t tiles = 0;
     for (size_t i = 0; i < b->inst.size(); i++) {
         muca::BatchInst &I = b->inst[i];
         BHIP(muca::launch_init_lattice(b->st, A.lat + I.lat_off, I.W, I.N, MUCA_KEYING_WEIGHT, 7,
                                        mm, 0, I.seed, 0, stratified ? I.W : 0));
-        BHIP(muca::launch_state(b->st, A.lat + I.lat_off, I.W, I.L, A.E + I.st_off,
-                                A.D + I.st_off, A.M + I.st_off));
+        tiles = std::max(tiles, muca::state_tiles(I.W, A.lat + I.lat_off));
         I.iter = 0;
         I.nup = b->init_nup[i];
         I.width = 10;   // :314
@@ -631,6 +631,8 @@ int batch_init(muca_batch *b, uint32_t mm, int stratified)
     BHIP(hipStreamSynchronize(b->st));
     BHIP(hipMemcpy(A.inst, b->inst.data(), b->inst.size() * sizeof(muca::BatchInst),
                    hipMemcpyHostToDevice));
+    BHIP(muca::launch_state_batch(b->st, A.inst, (uint32_t)b->inst.size(), tiles, A.lat, A.E, A.D,
+                                  A.M));
     // on the batch's stream: one of the null stream would not be ordered
     // before the launches that follow
     BHIP(hipMemsetAsync(A.queue, 0, 4 * muca::kBatchQueues, b->st));
