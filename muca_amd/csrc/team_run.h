@@ -97,6 +97,12 @@ __device__ __forceinline__ uint32_t sign_word(float x)
     return __float_as_uint(x);
 }
 
+// the smaller of two, NaN where either is (v_minimum3_f32)
+__device__ __forceinline__ float min_or_nan(float x, float y)
+{
+    return __builtin_elementwise_minimum(x, y);
+}
+
 // value of lane L of this lane's 16-lane row (v_mov_b32_dpp row_newbcast:L;
 // every lane of the row reads a valid source, so no old value is needed)
 template <int L>
@@ -234,14 +240,25 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     // wt's value at any D from HBM (only positions a walker cannot be at read
     // one from outside [0, N]); FP64: `bound` grows to the error that the
     // screening has to allow for it, 2^-22 |value| for the FP32 arithmetic and
-    // 2^-50 |ln W| for the rounding of the exact FP64 difference
+    // 2^-50 |ln W| for the rounding of the exact FP64 difference.  Where one bound
+    // serves all D, walls around an excluded range must not set it (L = 64,
+    // 32 768 walkers: 3.6 ms per launch with walls of 10^6 and of 10^300, 9.8 and
+    // 12.1 ms when they did): a value of `plain` or more needs no allowance, since
+    // with |thi| < 17 and |beta dE| <= 8 |beta| it decides the sign of e by 2^22
+    // times its error, and a value between ln W whose rounding would need more than
+    // 2^-16 is NaN, which `pass` takes to the exact test.  A window's own bound
+    // (LNWG) needs neither, and the selects cost its loads 15 % (L = 256, 4096
+    // walkers).
+    const float plain = 2.0f * (8.0f * fabsf((float)a.beta) + 17.0f);
     auto lnw_at = [&](int32_t i, float &bound) -> float {
         const int32_t c = min(max(i, 0), (int32_t)a.N - (FP64 ? 1 : 0));
         if (!FP64) return a.lnw32[c];
         const double from = a.lnw64[c], to = a.lnw64[c + 1];
-        const float g = (float)(to - from);
-        bound = fmaxf(bound, fabsf(g) * 0x1p-22f + (float)(fabs(from) + fabs(to)) * 0x1p-50f);
-        return g;
+        const float g = (float)(to - from), size = (float)(fabs(from) + fabs(to));
+        const bool screened = LNWG || size <= 0x1p34f;
+        const float need = (LNWG || fabsf(g) < plain ? fabsf(g) * 0x1p-22f : 0.0f) + size * 0x1p-50f;
+        bound = fmaxf(bound, screened ? need : 0.0f);
+        return screened ? g : NAN;
     };
     float gbound = 0.0f;   // FP64: the largest bound of wt (LNWG: of the team's window)
     float *const wave_bound = (float *)(lds + lay.off_tab + 256 * sizeof(double));
@@ -649,8 +666,10 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                     // the steps before it are identities (accepted nowhere).
                     // Byte k of (lo, hi): accept at dlo + k, i.e.
                     // acclog(r1) < ((fde + lnW[dlo + k + dDel]) - lnW[dlo + k]),
-                    // screened: the sign of e = thi - diff; |e| < lim needs the
-                    // exact test.  FP64 screens with FP32 differences of ln W
+                    // screened: the sign of e = thi - diff (the difference of two
+                    // infinite floats is a NaN whose sign is clear: rejected);
+                    // |e| < lim, in FP64 also an e that is NaN, needs the exact
+                    // test.  FP64 screens with FP32 differences of ln W
                     // (lim allows for them): one load and one fma per position
                     // and half the LDS, against two loads and three additions of
                     // doubles (L = 72, 4096 walkers: thermalization launch 432 ->
@@ -673,7 +692,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                             for (int k = 0; k < KW; k++) {
                                 const float e = __builtin_fmaf(step, wq[k], base);
                                 sg[k] = sign_word(e);
-                                emin = fminf(emin, fabsf(e));
+                                emin = min_or_nan(emin, fabsf(e));
                             }
                         } else {
                             const float *wto = wc + dd;
@@ -700,7 +719,7 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                                                                                 logtab + 128);
                                 if constexpr (FP64) {
                                     const double f = -(double)i_dE(info[r]) * a.beta;
-                                    const bool live = (uint32_t)tl >= from && fde[r] < INFINITY;
+                                    const bool live = valid && (uint32_t)tl >= from;
                                     uint64_t bytes = 0;
 #pragma unroll 1
                                     for (int k = 0; k < KW; k++) {
