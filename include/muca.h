@@ -109,6 +109,8 @@ int muca_get_lattice(muca_ctx *ctx, int8_t *site_major, uint64_t bytes);
  * computeEnergy/DeltaE/M (produce2_multigpu.cu:66-89). */
 int muca_compute_state(muca_ctx *ctx);
 int muca_get_state(muca_ctx *ctx, int32_t *E, int32_t *D, int32_t *M);
+/* D in [0, N].  Walkers whose D is not their lattice's sum of s^2 run on the
+ * generic kernel, which keeps D in [0, N]. */
 int muca_set_state(muca_ctx *ctx, const int32_t *E, const int32_t *D, const int32_t *M);
 
 /* H2D of ln W (muca_delta_multigpu.cu:386; produce2_multigpu.cu:262).  The

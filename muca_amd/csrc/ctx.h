@@ -45,6 +45,10 @@ struct muca_ctx {
     uint32_t *rw_flag = nullptr;
     uint32_t rw_cap = 0;
     bool have_weights = false;
+    // D is the lattice's: 1 yes (every run keeps it so), -1 no, 0 not known.  The
+    // lane and team kernels index LDS and HBM by D without a bound test and run
+    // only where it is; the generic kernel clamps.
+    int d_state = 1;
     uint32_t hist_preload = 0;   // test hook, see muca_set_test_hist_preload
     muca::Launch cfg{};
     uint32_t cus = 0;

@@ -57,6 +57,9 @@ hipError_t launch_state_batch(hipStream_t st, const BatchInst *inst, uint32_t n,
 hipError_t launch_copy(hipStream_t st, void *dst, const void *src, uint64_t bytes);
 hipError_t launch_state(hipStream_t st, const int8_t *lat, uint64_t W, uint32_t L, int32_t *E,
                         int32_t *D, int32_t *M);
+// *flag = 1 if a and b differ (device memory, n words; flag zeroed by the caller)
+hipError_t launch_differ(hipStream_t st, const int32_t *a, const int32_t *b, uint64_t n,
+                         uint32_t *flag);
 hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a);
 
 // team kernel (muca_team.hip): LDS layout of one workgroup of 16 walkers

@@ -70,6 +70,39 @@ int dev_alloc(T **p, uint64_t count, const char *what)
     return MUCA_OK;
 }
 
+// The launch configuration for the context's walkers as they are: its own where
+// D is the lattice's (looked up once after D or the lattice were set from
+// outside), else the generic kernel, whose accesses stay in bounds for any D.
+int launch_config(muca_ctx *c, muca::Launch &cfg)
+{
+    if (c->d_state == 0) {
+        const uint64_t W = c->W;
+        struct Scratch {
+            int32_t *p = nullptr;   // E, D, flag
+            ~Scratch()
+            {
+                if (p) hipFree(p);
+            }
+        } t;
+        uint32_t differ = 1;
+        if (hipMalloc((void **)&t.p, (2 * W + 1) * 4) == hipSuccess) {
+            uint32_t *flag = (uint32_t *)(t.p + 2 * W);
+            HIP_TRY(hipMemsetAsync(flag, 0, 4, c->st));
+            HIP_TRY(muca::launch_state(c->st, c->lat, W, c->p.L, t.p, t.p + W, nullptr));
+            HIP_TRY(muca::launch_differ(c->st, t.p + W, c->D, W, flag));
+            HIP_TRY(hipMemcpyAsync(&differ, flag, 4, hipMemcpyDeviceToHost, c->st));
+            HIP_TRY(hipStreamSynchronize(c->st));
+        } else {
+            t.p = nullptr;
+            (void)hipGetLastError();
+        }
+        c->d_state = differ ? -1 : 1;
+    }
+    cfg = c->cfg;
+    if (c->d_state < 0) cfg.kernel = MUCA_KERNEL_GENERIC;
+    return MUCA_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -306,6 +339,7 @@ int muca_init_lattice(muca_ctx *c, uint32_t mm, uint32_t gpu_index, uint32_t see
     HIP_TRY(hipSetDevice(c->p.device));
     HIP_TRY(muca::launch_init_lattice(c->st, c->lat, c->W, c->N, c->p.keying, (int)c->p.rounds,
                                       mm, gpu_index, seed, 0));
+    c->d_state = 0;
     HIP_TRY(hipStreamSynchronize(c->st));
     return MUCA_OK;
 }
@@ -316,6 +350,7 @@ int muca_init_lattice_stratified(muca_ctx *c, uint32_t mm, uint32_t gpu_index, u
     HIP_TRY(hipSetDevice(c->p.device));
     HIP_TRY(muca::launch_init_lattice(c->st, c->lat, c->W, c->N, c->p.keying, (int)c->p.rounds,
                                       mm, gpu_index, seed, 0, (uint32_t)c->W));
+    c->d_state = 0;
     HIP_TRY(hipStreamSynchronize(c->st));
     return MUCA_OK;
 }
@@ -327,6 +362,7 @@ int muca_set_lattice(muca_ctx *c, const int8_t *src, uint64_t bytes)
     for (uint64_t i = 0; i < bytes; i++)
         if (src[i] < -1 || src[i] > 1) return fail(MUCA_E_ARG, "spins must be in {-1,0,1}");
     HIP_TRY(hipSetDevice(c->p.device));
+    c->d_state = 0;
     HIP_TRY(hipMemcpy(c->lat, src, bytes, hipMemcpyHostToDevice));
     return MUCA_OK;
 }
@@ -347,6 +383,7 @@ int muca_compute_state(muca_ctx *c)
     HIP_TRY(hipSetDevice(c->p.device));
     HIP_TRY(muca::launch_state(c->st, c->lat, c->W, c->p.L, c->E, c->D, c->M));
     HIP_TRY(hipStreamSynchronize(c->st));
+    c->d_state = 1;
     return MUCA_OK;
 }
 
@@ -368,6 +405,7 @@ int muca_set_state(muca_ctx *c, const int32_t *E, const int32_t *D, const int32_
         for (uint64_t w = 0; w < c->W; w++)
             if (D[w] < 0 || (uint32_t)D[w] > c->N) return fail(MUCA_E_ARG, "D out of [0, N]");
     HIP_TRY(hipSetDevice(c->p.device));
+    if (D) c->d_state = 0;
     if (E) HIP_TRY(hipMemcpy(c->E, E, c->W * 4, hipMemcpyHostToDevice));
     if (D) HIP_TRY(hipMemcpy(c->D, D, c->W * 4, hipMemcpyHostToDevice));
     if (M) HIP_TRY(hipMemcpy(c->M, M, c->W * 4, hipMemcpyHostToDevice));
@@ -433,8 +471,10 @@ int muca_run(muca_ctx *c, uint32_t iter, uint32_t seed, uint64_t therm, uint64_t
     a.block_walkers = c->block_walkers ? c->block_walkers : c->W;
     a.joint_blocks = c->p.joint_blocks;
     a.hist_preload = c->hist_preload;
+    muca::Launch cfg;
+    if (int rc = launch_config(c, cfg)) return rc;
     HIP_TRY(hipEventRecord(c->ev0, c->st));
-    HIP_TRY(muca::launch_mcs(c->st, c->cfg, a));
+    HIP_TRY(muca::launch_mcs(c->st, cfg, a));
     HIP_TRY(hipEventRecord(c->ev1, c->st));
     if (hist_out) HIP_TRY(muca::launch_copy(c->st, c->pin, c->hist, (N + 1) * sizeof(uint64_t)));
     HIP_TRY(hipStreamSynchronize(c->st));
@@ -457,9 +497,12 @@ int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *blo
     if (attempts == 0) return fail(MUCA_E_ARG, "attempts must be > 0");
     HIP_TRY(hipSetDevice(c->p.device));
     const uint64_t N = c->N, W = c->W;
+    muca::Launch cfg0;
+    int rc = launch_config(c, cfg0);
+    if (rc) return rc;
     int8_t *lat0 = nullptr;
     int32_t *st0 = nullptr;
-    int rc = dev_alloc(&lat0, N * W, "autotune lattice copy");
+    rc = dev_alloc(&lat0, N * W, "autotune lattice copy");
     if (rc) return rc;
     rc = dev_alloc(&st0, 3 * W, "autotune state copy");
     if (rc) {
@@ -521,9 +564,10 @@ int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *blo
         a.joint_blocks = c->p.joint_blocks;
         a.block_walkers = c->block_walkers ? c->block_walkers : c->W;
     }
-    if (muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, lay))
+    const bool any = c->d_state > 0;   // D is the lattice's: any kernel may run
+    if (any && muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, lay))
         cands.push_back({MUCA_KERNEL_TEAM, 256});
-    if (!moments && muca::lane_eligible(a, c->cfg.fp64, c->cfg.lds_max))
+    if (any && !moments && muca::lane_eligible(a, c->cfg.fp64, c->cfg.lds_max))
         for (int b : {256, 512, 1024}) cands.push_back({MUCA_KERNEL_LANE, b});
     for (int b : {64, 128, 256}) cands.push_back({MUCA_KERNEL_GENERIC, b});
     hipError_t e = save_restore(true);

@@ -280,6 +280,20 @@ hipError_t launch_state(hipStream_t st, const int8_t *lat, uint64_t W, uint32_t 
     return hipGetLastError();
 }
 
+__global__ __launch_bounds__(256) void k_differ(const int32_t *a, const int32_t *b, uint64_t n,
+                                                uint32_t *flag)
+{
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n && a[i] != b[i]) *flag = 1u;
+}
+
+hipError_t launch_differ(hipStream_t st, const int32_t *a, const int32_t *b, uint64_t n,
+                         uint32_t *flag)
+{
+    hipLaunchKernelGGL(k_differ, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, b, n, flag);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // The update kernel, reference site order from tables (any L).
 // Per walker (muca_delta_multigpu.cu:735-829; produce2_multigpu.cu:401-496):
