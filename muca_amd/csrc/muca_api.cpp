@@ -176,13 +176,20 @@ int muca_create(const muca_params *params, muca_ctx **out)
     // 80 against 149; L = 128 the same).  Where several workgroups of teams
     // share a compute unit's LDS and half-rows fill a round the teams lead
     // to twice that (L = 32, 65 536 walkers: 185 against 142; 131 072: 198
-    // against 243), and so they do at odd L against the generic kernel
-    // (L = 33, 65 536: 162 against 73; L = 63: 72 against 74).  With per-D
-    // moments the alternative is the generic kernel, whose atomics collide: at
-    // even L and below L = 64 teams lead at any number (L = 72, 65 536 walkers:
-    // 85 against 25; L = 128: 97 against 45; L = 48, 262 144: 67 against 43),
-    // at larger odd L as without.  muca_autotune replaces this rule by
-    // measurement.
+    // against 243).  At odd L the alternative is the generic kernel; times of
+    // the teams over its at 24 576, 32 768, 49 152 and 65 536 walkers: L = 9 0.82,
+    // 1.11, 1.45, 1.86; L = 11 0.67, 0.93, 1.18, 1.49 (few of a team's lanes
+    // have work); L = 17 0.46, 0.62, 0.80, 1.01; two workgroups per compute
+    // unit, L = 33 0.22, 0.32, 0.36, 0.47 and L = 51 0.30, 0.44, 0.53, 0.72; one,
+    // L = 57 0.47, 0.72, 0.88, 1.21 and L = 63 0.45, 0.67, 0.83, 1.14.  With the
+    // joint histogram, at 8192, 16 384, 24 576 and 32 768: L = 9 0.77, 1.42, 1.90,
+    // 2.30; L = 11 0.64, 1.18, 1.53, 1.93; L = 13 0.37, 0.72, 0.95, 1.18; L = 17
+    // 0.28, 0.47, 0.58, 0.94.  With per-D moments the alternative is the generic
+    // kernel, whose atomics collide: at even L and below L = 64 teams lead at any
+    // number (L = 9, 98 304 walkers: half its time; L = 72, 65 536: 85 against 25;
+    // L = 128: 97 against 45; L = 48, 262 144: 67 against 43), at larger odd L to
+    // 256 per compute unit (L = 65, 65 536: 0.66 of its time).  muca_autotune
+    // replaces this rule by measurement.
     const uint64_t ncu = (uint64_t)(cu > 0 ? cu : 256);
     if (p.kernel == MUCA_KERNEL_AUTO) {
         // eligibility as the launch decides it (layout in this device's LDS)
@@ -195,11 +202,16 @@ int muca_create(const muca_params *params, muca_ctx **out)
         muca::TeamLayout lay_probe{};
         const bool team_ok = muca::team_layout(probe, p.precision == MUCA_FP64, lds_probe, lay_probe);
         const bool lane_ok = muca::lane_eligible(probe, p.precision == MUCA_FP64, lds_probe);
-        const uint64_t per_cu = moments ? (p.L % 2 == 0 || p.L < 64 ? UINT64_MAX / ncu : 256)
-                                : p.L >= 32 && (p.L % 2 || lay_probe.bytes * 3 <= lds_probe) &&
-                                        p.joint_blocks == 0
-                                    ? 256
-                                    : 128;
+        const bool odd = p.L % 2 != 0, joint = p.joint_blocks > 0;
+        uint64_t per_cu = 128;
+        if (moments)
+            per_cu = !odd || p.L < 64 ? UINT64_MAX / ncu : 256;
+        else if (joint)
+            per_cu = !odd || p.L >= 17 ? 128 : p.L >= 13 ? 96 : 32;
+        else if (odd)
+            per_cu = p.L < 11 ? 96 : p.L < 32 ? 128 : lay_probe.bytes * 2 <= lds_probe ? 256 : 192;
+        else if (p.L >= 32 && lay_probe.bytes * 3 <= lds_probe)
+            per_cu = 256;
         if (team_ok && (uint64_t)W <= per_cu * ncu)
             c->cfg.kernel = MUCA_KERNEL_TEAM;
         else if (moments)

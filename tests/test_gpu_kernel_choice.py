@@ -1,0 +1,42 @@
+"""Which kernel MUCA_KERNEL_AUTO takes, on both sides of each line drawn by the
+measured times (walkers per compute unit, odd L, joint histogram, moments)."""
+import pytest
+
+import muca_amd as M
+
+pytestmark = pytest.mark.gpu
+
+T, G, K = M.KERNEL_TEAM, M.KERNEL_GENERIC, M.KERNEL_LANE
+
+
+@pytest.fixture(scope="module")
+def cus():
+    with M.Context(8, 1) as ctx:
+        return ctx.info.cus
+
+
+def _choice(L, W, prec, blocks=0, obs=M.OBS_JOINT):
+    with M.Context(L, W, precision=prec, joint_blocks=blocks, observables=obs) as ctx:
+        return ctx.info.kernel
+
+
+@pytest.mark.parametrize("prec", [M.REF32, M.FP64])
+@pytest.mark.parametrize("L,per_cu,below,above", [
+    (9, 96, T, G), (11, 128, T, G), (31, 128, T, G), (33, 256, T, G), (51, 256, T, G),
+    (57, 192, T, G), (63, 192, T, G), (79, 192, T, G), (36, 256, T, K), (72, 128, T, K)])
+def test_weights(cus, prec, L, per_cu, below, above):
+    assert _choice(L, per_cu * cus, prec) == below
+    assert _choice(L, per_cu * cus + 1, prec) == above
+
+
+@pytest.mark.parametrize("L,per_cu,above", [(9, 32, G), (11, 32, G), (13, 96, G), (17, 128, G),
+                                            (33, 128, G), (16, 128, K)])
+def test_joint(cus, L, per_cu, above):
+    assert _choice(L, per_cu * cus, M.FP64, 2) == T
+    assert _choice(L, per_cu * cus + 1, M.FP64, 2) == above
+
+
+@pytest.mark.parametrize("L,per_cu,kernel", [(9, 512, T), (16, 512, T), (63, 300, T), (65, 256, T),
+                                             (65, 257, G)])
+def test_moments(cus, L, per_cu, kernel):
+    assert _choice(L, per_cu * cus, M.FP64, 2, M.OBS_MOMENTS) == kernel
