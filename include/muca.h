@@ -244,7 +244,9 @@ typedef struct muca_instance_status {
 
 const char *muca_batch_last_error(void);
 /* tiles: MUCA_KERNEL_AUTO (team tiles for few walkers where every L is in
- * [8, 128]), MUCA_KERNEL_TEAM (every L % 8 == 0, L <= 128) or MUCA_KERNEL_LANE; precision: MUCA_REF32 | MUCA_FP64.  Lane tiles hold
+ * [8, 128], unless the lattices are so small that setting up a tile costs more
+ * than lane tiles do), MUCA_KERNEL_TEAM (every L % 8 == 0, L <= 128) or
+ * MUCA_KERNEL_LANE; precision: MUCA_REF32 | MUCA_FP64.  Lane tiles hold
  * 1024 or 512 walkers (four or two per lane) when every L > 8, every walker
  * count is a multiple of 4 and there are 1024 walkers per compute unit, else
  * 256, or 512 / 1024 when the largest instance's ln W and histogram leave LDS

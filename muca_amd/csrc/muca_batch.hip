@@ -539,10 +539,21 @@ int muca_batch_create(int32_t device, const muca_instance *ins, uint32_t n, int3
         return bfail(MUCA_E_ARG, "lane tiles need ln W of every instance in LDS");
     }
     int kind = tiles;
-    if (tiles != MUCA_KERNEL_TEAM && tiles != MUCA_KERNEL_LANE)
-        // same rule as the single-instance contexts: team while walkers are few
-        kind = (team_ok && (st <= 128ull * (uint64_t)cu || !lane_ok)) ? MUCA_KERNEL_TEAM
-                                                                       : MUCA_KERNEL_LANE;
+    if (tiles != MUCA_KERNEL_TEAM && tiles != MUCA_KERNEL_LANE) {
+        // Same rule as the single-instance contexts: team while walkers are few.
+        // A team tile costs the queue and its tables about 0.12 us whatever its
+        // size (32 768 walkers: 0.25 ms per iteration), so lattices that are not
+        // all multiples of 8 go to lane tiles where a tile has little else to
+        // do.  Time of team over lane tiles at NUPDATES = 1: 32 768 walkers of
+        // L = 12, 18, 22, 26, 30 2.75, 1.68, 1.20, 0.90, 0.69; 16 384 of L = 12,
+        // 14, 18 1.54, 1.27, 0.90; 8192 of L = 10, 12, 14 1.22, 0.99, 0.81; 4096
+        // of L = 10 0.85; at NUPDATES = 4096 all but L = 10 below 1.
+        double sites = 0;   // site visits per sweep
+        for (const auto &I : b->inst) sites += (double)I.W * I.N;
+        const bool few = st <= 128ull * (uint64_t)cu &&
+                         (team_ask || (double)st * (double)st <= 48.0 * sites);
+        kind = team_ok && (few || !lane_ok) ? MUCA_KERNEL_TEAM : MUCA_KERNEL_LANE;
+    }
     if (kind == MUCA_KERNEL_LANE && !lane_ok) {
         batch_free(b);
         return bfail(MUCA_E_ARG, "no tile kind fits every instance");

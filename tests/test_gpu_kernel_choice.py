@@ -40,3 +40,12 @@ def test_joint(cus, L, per_cu, above):
                                              (65, 257, G)])
 def test_moments(cus, L, per_cu, kernel):
     assert _choice(L, per_cu * cus, M.FP64, 2, M.OBS_MOMENTS) == kernel
+
+
+@pytest.mark.parametrize("prec", [M.REF32, M.FP64])
+@pytest.mark.parametrize("L,n,W,tiles", [
+    (12, 8, 4096, K), (22, 2, 16384, K), (28, 2, 16384, T), (14, 4, 4096, K), (20, 4, 4096, T),
+    (10, 8, 1024, K), (14, 8, 1024, T), (10, 1, 2048, T), (16, 8, 4096, T), (100, 4, 4096, T)])
+def test_batch_tiles(cus, prec, L, n, W, tiles):
+    with M.Batch([dict(L=L, walkers=W * cus // 256, seed=i) for i in range(n)], precision=prec) as b:
+        assert b.tiles == tiles
