@@ -25,6 +25,11 @@ inline int fail(int code, const std::string &msg)
             return fail(MUCA_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+// Most that a context pins.  Its copies gain where they are small (see
+// launch_copy); 1 MiB holds ln W to L = 295 and the site tables to L = 228, while 20
+// bytes a site would be 43 GB at the largest L.
+constexpr uint64_t kPinMax = 1ull << 20;
+
 struct muca_ctx {
     muca_params p{};
     uint32_t N = 0;
@@ -36,7 +41,10 @@ struct muca_ctx {
     float *lnw32 = nullptr;
     double *lnw64 = nullptr;
     uint32_t *order = nullptr, *naver = nullptr;
-    void *pin = nullptr;        // pinned, 20 N + 12 bytes: site tables and ln W in, histogram out
+    // pinned, pin_bytes <= kPinMax: what fits of site tables and ln W in, histogram
+    // out (null if none of it does or the host has none to give: pageable copies then)
+    void *pin = nullptr;
+    uint64_t pin_bytes = 0;
     uint64_t *hist = nullptr;
     uint64_t *joint = nullptr;
     uint64_t *moms = nullptr;   // MUCA_OBS_MOMENTS: blocks * kMomWords * (N+1)

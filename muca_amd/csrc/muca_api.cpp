@@ -288,13 +288,23 @@ int muca_create(const muca_params *params, muca_ctx **out)
     std::vector<uint32_t> naver, order;
     make_tables(p.L, naver, order);
     hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->pin, N * 20 + 12, hipHostMallocDefault);
+    // N + 1 values of ln W in both precisions are the least it is for
+    if ((N + 1) * 12 <= kPinMax) c->pin_bytes = N * 20 + 12 < kPinMax ? N * 20 + 12 : kPinMax;
+    if (c->pin_bytes && hipHostMalloc(&c->pin, c->pin_bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->pin = nullptr;
+        c->pin_bytes = 0;
+    }
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
-    if (e == hipSuccess) {
+    if (e == hipSuccess && 20 * N <= c->pin_bytes) {
         memcpy(c->pin, naver.data(), 16 * N);
         memcpy((char *)c->pin + 16 * N, order.data(), 4 * N);
         e = muca::launch_copy(c->st, c->naver, c->pin, 20 * N);
+    } else if (e == hipSuccess) {
+        e = hipMemcpyAsync(c->naver, naver.data(), 16 * N, hipMemcpyHostToDevice, c->st);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(c->order, order.data(), 4 * N, hipMemcpyHostToDevice, c->st);
     }
     // on the context's stream: one of the null stream would not be ordered
     // before the launches that follow
@@ -430,12 +440,16 @@ int muca_set_log_weight(muca_ctx *c, const double *lnw, uint32_t nbins)
     if (nbins != c->N + 1) return fail(MUCA_E_ARG, "nbins must be N+1");
     for (uint32_t i = 0; i < nbins; i++)
         if (!std::isfinite(lnw[i])) return fail(MUCA_E_ARG, "ln W must be finite");
-    double *w64 = (double *)c->pin;
+    std::vector<double> pageable(c->pin ? 0 : (nbins * 12ull + 7) / 8);
+    double *w64 = c->pin ? (double *)c->pin : pageable.data();
     float *w32 = (float *)(w64 + nbins);
     memcpy(w64, lnw, nbins * sizeof(double));
     for (uint32_t i = 0; i < nbins; i++) w32[i] = (float)lnw[i];
     HIP_TRY(hipSetDevice(c->p.device));
-    HIP_TRY(muca::launch_copy(c->st, c->lnw64, c->pin, nbins * 12ull));
+    if (c->pin)
+        HIP_TRY(muca::launch_copy(c->st, c->lnw64, w64, nbins * 12ull));
+    else
+        HIP_TRY(hipMemcpyAsync(c->lnw64, w64, nbins * 12ull, hipMemcpyHostToDevice, c->st));
     HIP_TRY(hipStreamSynchronize(c->st));
     c->have_weights = true;
     return MUCA_OK;
@@ -488,10 +502,14 @@ int muca_run(muca_ctx *c, uint32_t iter, uint32_t seed, uint64_t therm, uint64_t
     HIP_TRY(hipEventRecord(c->ev0, c->st));
     HIP_TRY(muca::launch_mcs(c->st, cfg, a));
     HIP_TRY(hipEventRecord(c->ev1, c->st));
-    if (hist_out) HIP_TRY(muca::launch_copy(c->st, c->pin, c->hist, (N + 1) * sizeof(uint64_t)));
+    if (hist_out && c->pin)
+        HIP_TRY(muca::launch_copy(c->st, c->pin, c->hist, (N + 1) * sizeof(uint64_t)));
+    else if (hist_out)
+        HIP_TRY(hipMemcpyAsync(hist_out, c->hist, (N + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost,
+                               c->st));
     HIP_TRY(hipStreamSynchronize(c->st));
     if (kernel_ms) HIP_TRY(hipEventElapsedTime(kernel_ms, c->ev0, c->ev1));
-    if (hist_out) memcpy(hist_out, c->pin, (N + 1) * sizeof(uint64_t));
+    if (hist_out && c->pin) memcpy(hist_out, c->pin, (N + 1) * sizeof(uint64_t));
     return MUCA_OK;
 }
 
