@@ -46,7 +46,9 @@ extern "C" {
 #define MUCA_KERNEL_GENERIC 1  /* one lane per walker, reference site order from tables */
 #define MUCA_KERNEL_TEAM 2     /* sixteen lanes per walker (8 <= L <= 256; lattices and ln W in
                                   LDS when they fit, for odd L only then) */
-#define MUCA_KERNEL_LANE 3     /* one lane per walker, even L, table-free, screened acceptance */
+#define MUCA_KERNEL_LANE 3     /* one lane per walker, or per four where walkers are many and the
+                                  workgroup has at most 512 lanes; even L, table-free, screened
+                                  acceptance */
 
 /* what the produce path accumulates per walker block */
 #define MUCA_OBS_JOINT 0    /* joint H(D,M), produce2_multigpu.cu:489 */
@@ -65,8 +67,8 @@ typedef struct muca_params {
     uint32_t joint_blocks; /* produce path: 0 = no joint H(D,M); B >= 1 = one joint
                               histogram per contiguous block of walkers (jackknife) */
     int32_t kernel;      /* MUCA_KERNEL_* */
-    uint32_t block;      /* workgroup size of the one-lane kernels (0: chosen from
-                            walkers and compute units; else 64..1024) */
+    uint32_t block;      /* workgroup size of the generic and lane kernels (0: chosen
+                            from walkers and compute units; else 64..1024) */
     int32_t observables; /* produce path with joint_blocks > 0: MUCA_OBS_JOINT keeps
                             the reference's joint H(D,M); MUCA_OBS_MOMENTS keeps
                             exact per-D moments instead (6 (N+1) words per block;
@@ -144,6 +146,10 @@ int muca_autotune(muca_ctx *ctx, uint64_t attempts, int32_t *kernel, uint32_t *b
  * the histogram muca_run returns stays the exact count.  0 (the default)
  * is production behaviour. */
 int muca_set_test_hist_preload(muca_ctx *ctx, uint32_t preload);
+/* Test hook: lanes per workgroup and walkers per lane of a lane launch on a
+ * device of `cus` compute units (no device call). */
+int muca_test_lane_shape(uint32_t L, uint64_t walkers, uint32_t cus, uint32_t block,
+                         uint32_t *lanes, uint32_t *per_lane);
 /* D2H of the last launch's D histogram (muca_delta_multigpu.cu:401-412);
  * copy_ms (nullable) receives the copy's duration */
 int muca_get_hist(muca_ctx *ctx, uint64_t *hist, uint32_t nbins, float *copy_ms);

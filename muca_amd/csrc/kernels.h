@@ -88,6 +88,11 @@ bool lane_eligible(const McsArgs &a, int fp64, size_t lds_max);
 // walkers per lane of a lane launch: 4 where W walkers still make one and a half
 // wavefronts per SIMD, else 1
 int lane_walkers(uint32_t L, uint64_t W, uint32_t cus);
+// lanes per workgroup (the block asked for) and walkers per lane of a lane launch
+struct LaneShape {
+    int lanes, walkers;
+};
+LaneShape lane_shape(uint32_t L, uint64_t W, uint32_t cus, int block);
 hipError_t launch_mcs_lane(hipStream_t st, const Launch &cfg, const McsArgs &a);
 
 // ---- batched engine (muca_batch.hip) ----

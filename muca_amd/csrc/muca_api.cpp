@@ -520,6 +520,16 @@ int muca_set_test_hist_preload(muca_ctx *c, uint32_t preload)
     return MUCA_OK;
 }
 
+int muca_test_lane_shape(uint32_t L, uint64_t walkers, uint32_t cus, uint32_t block,
+                         uint32_t *lanes, uint32_t *per_lane)
+{
+    if (!lanes || !per_lane) return fail(MUCA_E_ARG, "NULL argument");
+    const muca::LaneShape s = muca::lane_shape(L, walkers, cus, (int)block);
+    *lanes = (uint32_t)s.lanes;
+    *per_lane = (uint32_t)s.walkers;
+    return MUCA_OK;
+}
+
 int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *block, float *ms)
 {
     if (!c) return fail(MUCA_E_ARG, "NULL context");

@@ -336,6 +336,13 @@ int lane_walkers(uint32_t L, uint64_t W, uint32_t cus)
     return L > 8 && W % 4 == 0 && W >= 1536ull * cus ? 4 : 1;
 }
 
+// A workgroup has the lanes that were asked for: four walkers per lane are built
+// for up to 512, which leave a lane twice the registers that 1024 do.
+LaneShape lane_shape(uint32_t L, uint64_t W, uint32_t cus, int block)
+{
+    return {block, block <= 512 ? lane_walkers(L, W, cus) : 1};
+}
+
 bool lane_eligible(const McsArgs &a, int fp64, size_t lds_max)
 {
     const size_t tsz = fp64 ? 8 : 4;
@@ -369,11 +376,9 @@ static hipError_t launch_lane_v(hipStream_t st, int block, const Launch &cfg, co
 template <int R, bool FP64, int KEYING>
 static hipError_t launch_lane_r(hipStream_t st, const Launch &cfg, const McsArgs &a)
 {
-    const int V = lane_walkers(a.L, a.W, cfg.cus);
-    const int block = cfg.block;
-    if (V == 4)
-        return launch_lane_v<R, FP64, KEYING, 4, 4>(st, block > 512 ? 512 : block, cfg, a);
-    return launch_lane_v<R, FP64, KEYING, 1, 1>(st, block, cfg, a);
+    const LaneShape sh = lane_shape(a.L, a.W, cfg.cus, cfg.block);
+    return sh.walkers == 4 ? launch_lane_v<R, FP64, KEYING, 4, 4>(st, sh.lanes, cfg, a)
+                           : launch_lane_v<R, FP64, KEYING, 1, 1>(st, sh.lanes, cfg, a);
 }
 
 hipError_t launch_mcs_lane(hipStream_t st, const Launch &cfg, const McsArgs &a)
