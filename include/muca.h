@@ -150,6 +150,12 @@ int muca_set_test_hist_preload(muca_ctx *ctx, uint32_t preload);
  * device of `cus` compute units (no device call). */
 int muca_test_lane_shape(uint32_t L, uint64_t walkers, uint32_t cus, uint32_t block,
                          uint32_t *lanes, uint32_t *per_lane);
+/* Test hook: the team kernel's layout for a launch on a device of `cus` compute
+ * units with `lds` bytes of LDS per workgroup (no device call).  out: eligible,
+ * lattices in LDS, histogram in LDS, ln W in HBM, rounds per chunk, chunk order
+ * (0 rows, 1 odd L, 2 on over row ends), attempts per half-row, LDS bytes. */
+int muca_test_team_layout(uint32_t L, uint64_t walkers, int32_t precision, int32_t moments,
+                          uint32_t lds, uint32_t cus, uint32_t out[8]);
 /* D2H of the last launch's D histogram (muca_delta_multigpu.cu:401-412);
  * copy_ms (nullable) receives the copy's duration */
 int muca_get_hist(muca_ctx *ctx, uint64_t *hist, uint32_t nbins, float *copy_ms);

@@ -78,8 +78,8 @@ struct TeamLayout {
     bool lnw_global;      // ln W too large for LDS: read from HBM (L2) per window
 };
 // false when the team kernel cannot run this launch (L < 8 or L > 256, or odd L
-// whose lattices do not fit in LDS)
-bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay);
+// whose lattices do not fit in LDS); cus: compute units of the device
+bool team_layout(const McsArgs &a, int fp64, size_t lds_max, uint32_t cus, TeamLayout &lay);
 hipError_t launch_mcs_team(hipStream_t st, const Launch &cfg, const McsArgs &a,
                            const TeamLayout &lay);
 

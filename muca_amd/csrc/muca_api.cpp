@@ -200,7 +200,7 @@ int muca_create(const muca_params *params, muca_ctx **out)
         probe.nup = 1;
         const size_t lds_probe = (size_t)(lds > 0 ? lds : 65536);
         muca::TeamLayout lay_probe{};
-        const bool team_ok = muca::team_layout(probe, p.precision == MUCA_FP64, lds_probe, lay_probe);
+        const bool team_ok = muca::team_layout(probe, p.precision == MUCA_FP64, lds_probe, c->cus, lay_probe);
         const bool lane_ok = muca::lane_eligible(probe, p.precision == MUCA_FP64, lds_probe);
         const bool odd = p.L % 2 != 0, joint = p.joint_blocks > 0;
         uint64_t per_cu = 128;
@@ -351,7 +351,7 @@ int muca_query(const muca_ctx *c, muca_info *info)
     a.nup = 1;
     muca::TeamLayout lay{};
     info->lds_lattice = c->cfg.kernel == MUCA_KERNEL_TEAM &&
-                        muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, lay) && lay.lat_lds;
+                        muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, c->cus, lay) && lay.lat_lds;
     return MUCA_OK;
 }
 
@@ -530,6 +530,29 @@ int muca_test_lane_shape(uint32_t L, uint64_t walkers, uint32_t cus, uint32_t bl
     return MUCA_OK;
 }
 
+int muca_test_team_layout(uint32_t L, uint64_t walkers, int32_t precision, int32_t moments,
+                          uint32_t lds, uint32_t cus, uint32_t *out)
+{
+    if (!out) return fail(MUCA_E_ARG, "NULL argument");
+    muca::McsArgs a{};
+    uint64_t mark = 0;   // never read: moments are asked for by a non-null pointer
+    a.N = L * L;
+    a.L = L;
+    a.W = walkers;
+    a.nup = 1;
+    a.moms = moments ? &mark : nullptr;
+    muca::TeamLayout lay{};
+    out[0] = muca::team_layout(a, precision == MUCA_FP64, lds, cus, lay);
+    out[1] = lay.lat_lds;
+    out[2] = lay.lds_hist;
+    out[3] = lay.lnw_global;
+    out[4] = lay.rounds;
+    out[5] = lay.order;
+    out[6] = lay.row;
+    out[7] = (uint32_t)lay.bytes;
+    return MUCA_OK;
+}
+
 int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *block, float *ms)
 {
     if (!c) return fail(MUCA_E_ARG, "NULL context");
@@ -605,7 +628,7 @@ int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *blo
         a.block_walkers = c->block_walkers ? c->block_walkers : c->W;
     }
     const bool any = c->d_state > 0;   // D is the lattice's: any kernel may run
-    if (any && muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, lay))
+    if (any && muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, c->cus, lay))
         cands.push_back({MUCA_KERNEL_TEAM, 256});
     if (any && !moments && muca::lane_eligible(a, c->cfg.fp64, c->cfg.lds_max))
         for (int b : {256, 512, 1024}) cands.push_back({MUCA_KERNEL_LANE, b});

@@ -513,7 +513,7 @@ int muca_batch_create(int32_t device, const muca_instance *ins, uint32_t n, int3
         a.L = I.L;
         a.W = I.W;
         a.nup = 1;
-        if (!(I.L <= 128 && muca::team_layout(a, b->fp64, lds_budget, I.lay) &&
+        if (!(I.L <= 128 && muca::team_layout(a, b->fp64, lds_budget, b->cus, I.lay) &&
               !I.lay.lnw_global))
             team_ok = false;
         if (I.L % 8 != 0) team_ask = false;   // team tiles on request: multiples of 8 only

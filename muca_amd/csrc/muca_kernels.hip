@@ -614,7 +614,7 @@ hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a)
     const bool moments = a.moms != nullptr && a.joint == nullptr;
     if (cfg.kernel == 2 && (!moments || cfg.fp64)) {
         TeamLayout lay{};
-        if (team_layout(a, cfg.fp64, cfg.lds_max, lay)) return launch_mcs_team(st, cfg, a, lay);
+        if (team_layout(a, cfg.fp64, cfg.lds_max, cfg.cus, lay)) return launch_mcs_team(st, cfg, a, lay);
     }
     if (cfg.kernel == 3 && !moments && lane_eligible(a, cfg.fp64, cfg.lds_max))
         return launch_mcs_lane(st, cfg, a);

@@ -84,21 +84,22 @@ static bool place(const McsArgs &a, int fp64, size_t lds_max, bool windows, Team
     return off <= lds_max;
 }
 
-bool team_layout(const McsArgs &a, int fp64, size_t lds_max, TeamLayout &lay)
+bool team_layout(const McsArgs &a, int fp64, size_t lds_max, uint32_t cus, TeamLayout &lay)
 {
     if (!place(a, fp64, lds_max, false, lay)) return false;
     // Per-D moments need no histogram, so with windows of ln W from HBM four
     // workgroups share a compute unit (128 VGPRs).  That leads as soon as there
-    // are more walkers than the LDS layout keeps resident (attempts/ns; L = 128:
+    // are more walkers than the LDS layout keeps resident (attempts/ns on 256
+    // compute units; L = 128:
     // 8192 walkers 55 -> 80, 65 536 54 -> 97; 4096 55 against 49; L = 72: 16 384
-    // 57 -> 76; L = 96, three workgroups per compute unit: 16 384 82 -> 90, 8192
+    // 57 -> 76; L = 96, two workgroups per compute unit: 16 384 82 -> 90, 8192
     // 78 against 75), but not where two workgroups with their lattices fit
     // (L = 48, 16 384: 89 against 80).  Odd L need their lattices in LDS.
     const uint64_t per_cu = lds_max / lay.bytes;
     const bool moms = fp64 && a.moms != nullptr && a.joint == nullptr;
     TeamLayout win;
     if (moms && a.L % 2 == 0 && !lay.lnw_global &&
-        (per_cu == 1 || (!lay.lat_lds && per_cu < 4)) && a.W > kTeams * kCus * per_cu &&
+        (per_cu == 1 || (!lay.lat_lds && per_cu < 4)) && a.W > (uint64_t)kTeams * cus * per_cu &&
         place(a, fp64, lds_max, true, win))
         lay = win;
     return true;

@@ -61,7 +61,6 @@ namespace team_detail {
 
 constexpr int kTeam = 16;
 constexpr int kTeams = 16;   // per workgroup of 256 lanes
-constexpr uint64_t kCus = 256;   // compute units
 constexpr uint32_t kXcds = 8;   // accelerator dies of an MI355X, one L2 each
 // D values per window (at most 8).  Narrower ones cut the mask work per pass and
 // make D leave them more often: L = 128, seeded 1.85 ms per launch against 1.90
