@@ -81,7 +81,8 @@ typedef struct muca_info {
     uint32_t cus, block;          /* compute units, threads per block of the update */
     uint64_t lattice_bytes, joint_bins;
     uint32_t lds_per_block;       /* bytes of LDS one workgroup may use */
-    uint32_t lds_lattice;         /* 1 if the team kernel keeps lattices in LDS */
+    uint32_t lds_lattice;         /* 1 if the team kernel keeps lattices in LDS (in a context
+                                     with per-D moments: in its production launches) */
 } muca_info;
 
 const char *muca_last_error(void);

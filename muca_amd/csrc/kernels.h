@@ -61,6 +61,15 @@ hipError_t launch_state(hipStream_t st, const int8_t *lat, uint64_t W, uint32_t 
 hipError_t launch_differ(hipStream_t st, const int32_t *a, const int32_t *b, uint64_t n,
                          uint32_t *flag);
 hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a);
+// the generic kernel's workgroup for W walkers: with one walker per lane the grid
+// should reach every compute unit before workgroups grow (16 384 walkers at 256
+// lanes would occupy 64 of 256 compute units)
+inline int generic_block(uint64_t W, uint64_t cus)
+{
+    int block = 256;
+    while (block > 64 && W < block * cus) block /= 2;
+    return block;
+}
 
 // team kernel (muca_team.hip): LDS layout of one workgroup of 16 walkers
 struct TeamLayout {

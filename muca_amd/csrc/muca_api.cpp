@@ -70,6 +70,21 @@ int dev_alloc(T **p, uint64_t count, const char *what)
     return MUCA_OK;
 }
 
+// The team kernel's layout for W walkers, with `moments` that of a launch that
+// accumulates per-D moments (production launches of such a context)
+bool probe_team(uint32_t L, uint64_t W, int fp64, bool moments, size_t lds, uint32_t cus,
+                muca::TeamLayout &lay)
+{
+    uint64_t mark = 0;   // never read: a non-null pointer asks for moments
+    muca::McsArgs a{};
+    a.N = L * L;
+    a.L = L;
+    a.W = W;
+    a.nup = 1;
+    a.moms = moments ? &mark : nullptr;
+    return muca::team_layout(a, fp64, lds, cus, lay);
+}
+
 // The launch configuration for the context's walkers as they are: its own where
 // D is the lattice's (looked up once after D or the lattice were set from
 // outside), else the generic kernel, whose accesses stay in bounds for any D.
@@ -99,7 +114,10 @@ int launch_config(muca_ctx *c, muca::Launch &cfg)
         c->d_state = differ ? -1 : 1;
     }
     cfg = c->cfg;
-    if (c->d_state < 0) cfg.kernel = MUCA_KERNEL_GENERIC;
+    if (c->d_state < 0) {
+        cfg.kernel = MUCA_KERNEL_GENERIC;
+        if (c->p.block == 0) cfg.block = muca::generic_block(c->W, c->cus ? c->cus : 256);
+    }
     return MUCA_OK;
 }
 
@@ -193,14 +211,13 @@ int muca_create(const muca_params *params, muca_ctx **out)
     const uint64_t ncu = (uint64_t)(cu > 0 ? cu : 256);
     if (p.kernel == MUCA_KERNEL_AUTO) {
         // eligibility as the launch decides it (layout in this device's LDS)
+        const size_t lds_probe = (size_t)(lds > 0 ? lds : 65536);
+        muca::TeamLayout lay_probe{};
+        const bool team_ok = probe_team(p.L, W, p.precision == MUCA_FP64, moments, lds_probe,
+                                        c->cus, lay_probe);
         muca::McsArgs probe{};
         probe.N = p.L * p.L;
         probe.L = p.L;
-        probe.W = W;
-        probe.nup = 1;
-        const size_t lds_probe = (size_t)(lds > 0 ? lds : 65536);
-        muca::TeamLayout lay_probe{};
-        const bool team_ok = muca::team_layout(probe, p.precision == MUCA_FP64, lds_probe, c->cus, lay_probe);
         const bool lane_ok = muca::lane_eligible(probe, p.precision == MUCA_FP64, lds_probe);
         const bool odd = p.L % 2 != 0, joint = p.joint_blocks > 0;
         uint64_t per_cu = 128;
@@ -228,13 +245,8 @@ int muca_create(const muca_params *params, muca_ctx **out)
         return fail(MUCA_E_ARG, "block must be 0 or a multiple of 64 in [64, 1024]");
     }
     c->cfg.block = p.block ? (int)p.block : 256;
-    if (p.block == 0 && c->cfg.kernel == MUCA_KERNEL_GENERIC) {
-        // one walker per lane and no LDS lattice: the grid should reach every
-        // compute unit before workgroups grow (16 384 walkers at 256 lanes
-        // would occupy 64 of 256 compute units)
-        while (c->cfg.block > 64 && (uint64_t)W < (uint64_t)c->cfg.block * ncu)
-            c->cfg.block /= 2;
-    }
+    if (p.block == 0 && c->cfg.kernel == MUCA_KERNEL_GENERIC)
+        c->cfg.block = muca::generic_block(W, ncu);
     if (p.block == 0 && c->cfg.kernel == MUCA_KERNEL_LANE) {
         // Four walkers per lane (lane_walkers): 256 lanes, or 512 where the
         // lane kernel's LDS (ln W and the histogram) admits one workgroup per
@@ -344,14 +356,11 @@ int muca_query(const muca_ctx *c, muca_info *info)
     info->lattice_bytes = (uint64_t)c->N * c->W;
     info->joint_bins = c->joint_stride * c->p.joint_blocks;
     info->lds_per_block = (uint32_t)c->cfg.lds_max;
-    muca::McsArgs a{};
-    a.N = c->N;
-    a.L = c->p.L;
-    a.W = c->W;
-    a.nup = 1;
     muca::TeamLayout lay{};
     info->lds_lattice = c->cfg.kernel == MUCA_KERNEL_TEAM &&
-                        muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, c->cus, lay) && lay.lat_lds;
+                        probe_team(c->p.L, c->W, c->cfg.fp64, c->moms != nullptr, c->cfg.lds_max,
+                                   c->cus, lay) &&
+                        lay.lat_lds;
     return MUCA_OK;
 }
 
@@ -534,15 +543,8 @@ int muca_test_team_layout(uint32_t L, uint64_t walkers, int32_t precision, int32
                           uint32_t lds, uint32_t cus, uint32_t *out)
 {
     if (!out) return fail(MUCA_E_ARG, "NULL argument");
-    muca::McsArgs a{};
-    uint64_t mark = 0;   // never read: moments are asked for by a non-null pointer
-    a.N = L * L;
-    a.L = L;
-    a.W = walkers;
-    a.nup = 1;
-    a.moms = moments ? &mark : nullptr;
     muca::TeamLayout lay{};
-    out[0] = muca::team_layout(a, precision == MUCA_FP64, lds, cus, lay);
+    out[0] = probe_team(L, walkers, precision == MUCA_FP64, moments != 0, lds, cus, lay);
     out[1] = lay.lat_lds;
     out[2] = lay.lds_hist;
     out[3] = lay.lnw_global;

@@ -607,6 +607,15 @@ static hipError_t launch_generic_k(hipStream_t st, const Launch &cfg, const McsA
                             : launch_generic_r<7, FP64, KEYING>(st, cfg, a);
 }
 
+static hipError_t launch_mcs_generic(hipStream_t st, const Launch &cfg, const McsArgs &a)
+{
+    if (cfg.fp64)
+        return cfg.keying == 0 ? launch_generic_k<true, 0>(st, cfg, a)
+                               : launch_generic_k<true, 1>(st, cfg, a);
+    return cfg.keying == 0 ? launch_generic_k<false, 0>(st, cfg, a)
+                           : launch_generic_k<false, 1>(st, cfg, a);
+}
+
 hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a)
 {
     if (a.W == 0 || (a.therm == 0 && a.nup == 0)) return hipSuccess;
@@ -618,11 +627,12 @@ hipError_t launch_mcs(hipStream_t st, const Launch &cfg, const McsArgs &a)
     }
     if (cfg.kernel == 3 && !moments && lane_eligible(a, cfg.fp64, cfg.lds_max))
         return launch_mcs_lane(st, cfg, a);
-    if (cfg.fp64)
-        return cfg.keying == 0 ? launch_generic_k<true, 0>(st, cfg, a)
-                               : launch_generic_k<true, 1>(st, cfg, a);
-    return cfg.keying == 0 ? launch_generic_k<false, 0>(st, cfg, a)
-                           : launch_generic_k<false, 1>(st, cfg, a);
+    // a context of the team kernel whose launch does not fit it (odd L, a
+    // thermalisation of production with moments: its histogram takes the lattices'
+    // LDS) has no block of its own
+    Launch g = cfg;
+    if (cfg.kernel == 2 && cfg.block == 256 && cfg.cus) g.block = generic_block(a.W, cfg.cus);
+    return launch_mcs_generic(st, g, a);
 }
 
 // ---------------------------------------------------------------------------

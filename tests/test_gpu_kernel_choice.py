@@ -42,6 +42,17 @@ def test_moments(cus, L, per_cu, kernel):
     assert _choice(L, per_cu * cus, M.FP64, 2, M.OBS_MOMENTS) == kernel
 
 
+@pytest.mark.parametrize("L,W,kernel,lds_lattice", [
+    # odd lattices that fit in LDS where no histogram is kept there
+    (81, 4096, T, 1), (83, 4096, T, 1), (85, 4096, G, 0),
+    # even ones: in LDS likewise, and in HBM once walkers outnumber the resident
+    (80, 4096, T, 1), (66, 4096, T, 1), (66, 4100, T, 0)])
+def test_moments_layout_is_the_launch_s(cus, L, W, kernel, lds_lattice):
+    W += 16 * (cus - 256)
+    with M.Context(L, W, precision=M.FP64, joint_blocks=2, observables=M.OBS_MOMENTS) as ctx:
+        assert (ctx.info.kernel, ctx.info.lds_lattice) == (kernel, lds_lattice)
+
+
 @pytest.mark.parametrize("prec", [M.REF32, M.FP64])
 @pytest.mark.parametrize("L,n,W,tiles", [
     (12, 8, 4096, K), (22, 2, 16384, K), (28, 2, 16384, T), (14, 4, 4096, K), (20, 4, 4096, T),
