@@ -268,6 +268,10 @@ const char *muca_batch_last_error(void);
 int muca_batch_create(int32_t device, const muca_instance *instances, uint32_t n,
                       int32_t precision, int32_t tiles, muca_batch **batch);
 int muca_batch_destroy(muca_batch *batch);
+/* Test hook: static LDS of the batch kernel for these tiles (`several` walkers
+ * per lane) and what the library leaves free for it. */
+int muca_test_batch_static_lds(int32_t precision, int32_t tiles, int32_t several,
+                               uint32_t *bytes, uint32_t *reserved);
 /* tile kind, threads per workgroup, tile count, persistent grid, total walkers */
 int muca_batch_query(const muca_batch *batch, int32_t *tiles, uint32_t *block, uint32_t *ntiles,
                      uint32_t *grid, uint64_t *walkers);

@@ -102,6 +102,8 @@ _SIGS = {
                                          ctypes.c_int32, ctypes.c_int32,
                                          ctypes.POINTER(ctypes.c_void_p)]),
     "muca_batch_destroy": (ctypes.c_int, [_vp]),
+    "muca_test_batch_static_lds": (ctypes.c_int, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
+                                                  ctypes.POINTER(_u32), ctypes.POINTER(_u32)]),
     "muca_batch_query": (ctypes.c_int, [_vp, _i32p, ctypes.POINTER(_u32), ctypes.POINTER(_u32),
                                         ctypes.POINTER(_u32), _u64p]),
     "muca_batch_iterate_profiled": (ctypes.c_int, [_vp, _u32, _f32p, _f32p]),

@@ -203,6 +203,14 @@ __device__ __forceinline__ uint32_t batch_take(const BatchArgs &b)
     return b.ntiles;
 }
 
+// LDS that the lane and batch kernels declare statically, at most; the dynamic
+// LDS of a launch leaves it free
+constexpr size_t kStaticLds = 256;
+// bytes of it in the batch kernel (team tiles, else lane tiles; vecs: several
+// walkers per lane)
+hipError_t batch_static_lds(int fp64, int team, int vecs, size_t *bytes);
+const void *batch_team_function(int fp64);   // the build for every kind of instance
+
 // persistent kernels: every workgroup takes tiles (batch_take) until none is left
 // lat_modes: bit 0 set if some instance keeps its tile's lattices in LDS,
 // bit 1 if some reads them from HBM; nrs: the rounds per chunk (1..4) that

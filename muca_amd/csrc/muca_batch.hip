@@ -371,7 +371,7 @@ hipError_t configure(muca_batch *b, int kind, uint32_t block)
         need = std::max(need, kind == MUCA_KERNEL_TEAM
                                   ? I.lay.bytes
                                   : (size_t)I.lane_lds_w + (I.lane_hist ? (size_t)(I.N + 1) * 4 : 0));
-    const uint32_t per_cu_lds = (uint32_t)std::max<size_t>(1, b->lds_device / (need + 256));
+    const uint32_t per_cu_lds = (uint32_t)std::max<size_t>(1, b->lds_device / (need + muca::kStaticLds));
     const uint32_t n = (uint32_t)b->inst.size();
     // Lane tiles, automatic: with enough walkers for a wavefront of four per
     // lane on every SIMD, 256-lane tiles of four walkers per lane, or of two
@@ -484,7 +484,7 @@ int muca_batch_create(int32_t device, const muca_instance *ins, uint32_t n, int3
     int cu = 0, lds = 0;
     BHIP(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, device));
     BHIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
-    const size_t lds_budget = (size_t)lds - 256;   // static LDS of the persistent kernels
+    const size_t lds_budget = (size_t)lds - muca::kStaticLds;
     muca_batch *b = new muca_batch();
     b->device = device;
     b->fp64 = precision == MUCA_FP64;
@@ -591,6 +591,17 @@ int muca_batch_create(int32_t device, const muca_instance *ins, uint32_t n, int3
 int muca_batch_destroy(muca_batch *b)
 {
     batch_free(b);
+    return MUCA_OK;
+}
+
+int muca_test_batch_static_lds(int32_t precision, int32_t tiles, int32_t several,
+                               uint32_t *bytes, uint32_t *reserved)
+{
+    if (!bytes || !reserved) return bfail(MUCA_E_ARG, "NULL argument");
+    size_t n = 0;
+    BHIP(muca::batch_static_lds(precision == MUCA_FP64, tiles == MUCA_KERNEL_TEAM, several, &n));
+    *bytes = (uint32_t)n;
+    *reserved = (uint32_t)muca::kStaticLds;
     return MUCA_OK;
 }
 

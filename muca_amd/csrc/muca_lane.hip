@@ -32,8 +32,9 @@
 
 namespace muca {
 
-// The walkers wbase .. wbase + blockDim.x - 1 of the launch described by a
-// (every lane of the workgroup calls it together).
+template <bool FP64>
+using lane_t = typename std::conditional<FP64, double, float>::type;   // of ln W and diff
+
 // V walkers' spins of one site: a dword, a half-word or a byte
 template <int V>
 __device__ __forceinline__ uint32_t load_spins(const uint8_t *p)
@@ -57,14 +58,15 @@ __device__ __forceinline__ void store_spins(uint8_t *p, uint32_t v)
 // V per lane (every lane of the workgroup calls it together; W % V == 0 and
 // the lattice is V-aligned).
 // OBS: 0 the D histogram; 1 joint H(D,M) per walker block as well.
+// fde_tab: 17 entries in LDS, the kernel's (a variable of this function would
+// be one per variant that a kernel calls).
 template <int R, bool FP64, int KEYING, bool LDSHIST, int OBS, int V, int PD>
 __device__ __forceinline__ void lane_run(const McsArgs &a, uint32_t lds_w, uint64_t wbase,
-                                         unsigned char *lds)
+                                         unsigned char *lds, lane_t<FP64> *fde_tab)
 {
-    typedef typename std::conditional<FP64, double, float>::type T;
+    typedef lane_t<FP64> T;
     constexpr bool JOINT = OBS == 1;
     __syncthreads();   // LDS may still be read by a previous call's flush
-    __shared__ T fde_tab[17];
     T *wt = (T *)lds, *fdet = fde_tab + 8;   // fdet[dE] = (T)(-dE * beta), |dE| <= 8
     uint32_t *hist = (uint32_t *)(lds + lds_w);
     const uint32_t N = a.N, L = a.L, Rw = L / 2;
@@ -323,8 +325,10 @@ template <int R, bool FP64, int KEYING, bool LDSHIST, int OBS, int V, int PD>
 __global__ __launch_bounds__(V > 1 ? 512 : 1024) void k_mcs_lane(McsArgs a, uint32_t lds_w)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    __shared__ lane_t<FP64> fde_tab[17];
+    static_assert(sizeof(fde_tab) <= kStaticLds, "static LDS");
     lane_run<R, FP64, KEYING, LDSHIST, OBS, V, PD>(a, lds_w, (uint64_t)blockIdx.x * blockDim.x * V,
-                                               lds);
+                                               lds, fde_tab);
 }
 
 // Four walkers per lane need one and a half wavefronts per SIMD to lead: 524 288
@@ -346,7 +350,7 @@ LaneShape lane_shape(uint32_t L, uint64_t W, uint32_t cus, int block)
 bool lane_eligible(const McsArgs &a, int fp64, size_t lds_max)
 {
     const size_t tsz = fp64 ? 8 : 4;
-    return a.L % 2 == 0 && a.L >= 4 && (a.N + 1) * tsz <= lds_max;
+    return a.L % 2 == 0 && a.L >= 4 && (a.N + 1) * tsz + kStaticLds <= lds_max;
 }
 
 template <int R, bool FP64, int KEYING, int V, int PD>
@@ -355,7 +359,7 @@ static hipError_t launch_lane_v(hipStream_t st, int block, const Launch &cfg, co
     const size_t tsz = FP64 ? 8 : 4;
     const uint32_t lds_w = (uint32_t)(((a.N + 1) * tsz + 15) & ~(size_t)15);
     const size_t lds_h = (size_t)(a.N + 1) * 4;
-    const bool hist_lds = lds_w + lds_h <= cfg.lds_max;
+    const bool hist_lds = lds_w + lds_h + kStaticLds <= cfg.lds_max;
     const size_t bytes = lds_w + (hist_lds ? lds_h : 0);
     const bool joint = a.joint != nullptr;
     void (*k)(McsArgs, uint32_t);
@@ -408,6 +412,8 @@ __global__ __launch_bounds__(VECS ? 256 : 1024, VECS ? 2 : 4) void k_batch_lane(
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     __shared__ uint32_t s_tile;
+    __shared__ lane_t<FP64> fde_tab[17];
+    static_assert(sizeof(s_tile) + sizeof(fde_tab) + 16 <= kStaticLds, "static LDS");
     for (;;) {
         __syncthreads();
         if (threadIdx.x == 0) s_tile = batch_take(b);
@@ -422,20 +428,20 @@ __global__ __launch_bounds__(VECS ? 256 : 1024, VECS ? 2 : 4) void k_batch_lane(
         if constexpr (VECS) {
             if (I->lane_vec == 4) {
                 if (I->lane_hist)
-                    lane_run<7, FP64, 0, true, 0, 4, 4>(a, lw, tile.wbase, lds);
+                    lane_run<7, FP64, 0, true, 0, 4, 4>(a, lw, tile.wbase, lds, fde_tab);
                 else
-                    lane_run<7, FP64, 0, false, 0, 4, 4>(a, lw, tile.wbase, lds);
+                    lane_run<7, FP64, 0, false, 0, 4, 4>(a, lw, tile.wbase, lds, fde_tab);
             } else {
                 if (I->lane_hist)
-                    lane_run<7, FP64, 0, true, 0, 2, 4>(a, lw, tile.wbase, lds);
+                    lane_run<7, FP64, 0, true, 0, 2, 4>(a, lw, tile.wbase, lds, fde_tab);
                 else
-                    lane_run<7, FP64, 0, false, 0, 2, 4>(a, lw, tile.wbase, lds);
+                    lane_run<7, FP64, 0, false, 0, 2, 4>(a, lw, tile.wbase, lds, fde_tab);
             }
         } else {
             if (I->lane_hist)
-                lane_run<7, FP64, 0, true, 0, 1, 1>(a, lw, tile.wbase, lds);
+                lane_run<7, FP64, 0, true, 0, 1, 1>(a, lw, tile.wbase, lds, fde_tab);
             else
-                lane_run<7, FP64, 0, false, 0, 1, 1>(a, lw, tile.wbase, lds);
+                lane_run<7, FP64, 0, false, 0, 1, 1>(a, lw, tile.wbase, lds, fde_tab);
         }
     }
 }
@@ -451,6 +457,15 @@ hipError_t launch_batch_lane(hipStream_t st, int fp64, int vecs, const BatchArgs
 {
     hipLaunchKernelGGL(batch_lane_kernel(fp64, vecs), dim3(grid), dim3(block), lds_bytes, st, b);
     return hipGetLastError();
+}
+
+hipError_t batch_static_lds(int fp64, int team, int vecs, size_t *bytes)
+{
+    hipFuncAttributes at;
+    const hipError_t e = hipFuncGetAttributes(
+        &at, team ? batch_team_function(fp64) : (const void *)batch_lane_kernel(fp64, vecs));
+    if (e == hipSuccess) *bytes = at.sharedSizeBytes;
+    return e;
 }
 
 hipError_t prepare_batch_lane(int fp64, int vecs, size_t lds_bytes)

@@ -216,6 +216,11 @@ hipError_t launch_batch_team(hipStream_t st, int fp64, const BatchArgs &b, uint3
     return hipGetLastError();
 }
 
+const void *batch_team_function(int fp64)
+{
+    return (const void *)(fp64 ? batch_team_kernel<true>(3, 0) : batch_team_kernel<false>(3, 0));
+}
+
 hipError_t prepare_batch_team(int fp64, size_t lds_bytes, int lat_modes, int nrs)
 {
     void (*k)(BatchArgs) = fp64 ? batch_team_kernel<true>(lat_modes, nrs)
