@@ -331,6 +331,10 @@ const char *muca_mlp_last_error(void);
 uint32_t muca_mlp_param_count(void);
 int muca_mlp_create(int32_t device, muca_mlp **mlp);
 int muca_mlp_destroy(muca_mlp *mlp);
+/* Self-check: the activation of training, its quotients taken from one refined
+ * reciprocal, against divisions at every float; the number of floats where they
+ * differ, and one of them */
+int muca_mlp_silu_check(int32_t device, uint64_t *differing, uint32_t *example);
 /* also resets the Adam moments and step count */
 int muca_mlp_set_params(muca_mlp *mlp, const float *params, uint32_t n);
 int muca_mlp_get_params(muca_mlp *mlp, float *params, uint32_t n);
@@ -359,6 +363,9 @@ int muca_acclog_device(int32_t device, uint32_t k0, uint32_t n, float *out);
 /* the fast screening approximation (hardware log2 * ln 2) the update kernels
  * use before deciding whether the exact log is needed, same inputs */
 int muca_acclog_fast_device(int32_t device, uint32_t k0, uint32_t n, float *out);
+/* The team and lane kernels' screen for draws r = (k0 + t) << 9: log(u) lies below
+ * thi[t], by less than lim[t]. */
+int muca_acclog_screen_device(int32_t device, uint32_t k0, uint32_t n, float *thi, float *lim);
 
 #ifdef __cplusplus
 }

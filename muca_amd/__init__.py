@@ -121,6 +121,7 @@ _SIGS = {
     "muca_mlp_last_error": (ctypes.c_char_p, []),
     "muca_mlp_param_count": (ctypes.c_uint32, []),
     "muca_mlp_create": (ctypes.c_int, [ctypes.c_int32, ctypes.POINTER(ctypes.c_void_p)]),
+    "muca_mlp_silu_check": (ctypes.c_int, [ctypes.c_int32, _u64p, ctypes.POINTER(_u32)]),
     "muca_mlp_destroy": (ctypes.c_int, [_vp]),
     "muca_mlp_set_params": (ctypes.c_int, [_vp, _f32p, _u32]),
     "muca_mlp_get_params": (ctypes.c_int, [_vp, _f32p, _u32]),
@@ -173,6 +174,8 @@ _SIGS = {
                                           _f32p]),
     "muca_acclog_fast_device": (ctypes.c_int, [ctypes.c_int32, ctypes.c_uint32,
                                                ctypes.c_uint32, _f32p]),
+    "muca_acclog_screen_device": (ctypes.c_int, [ctypes.c_int32, ctypes.c_uint32,
+                                                 ctypes.c_uint32, _f32p, _f32p]),
 }
 
 ACCLOG_FAST_REL = 2.0 ** -20     # screening band of the fast log (acclog.h)
@@ -557,6 +560,13 @@ def acclog_fast_device(k0, n, device=0):
     out = np.empty(n, np.float32)
     _check(lib().muca_acclog_fast_device(device, k0, n, _p(out, _f32p)))
     return out
+
+
+def acclog_screen_device(k0, n, device=0):
+    """The screen of the acceptance log: (thi, lim) per draw."""
+    thi, lim = np.empty(n, np.float32), np.empty(n, np.float32)
+    _check(lib().muca_acclog_screen_device(device, k0, n, _p(thi, _f32p), _p(lim, _f32p)))
+    return thi, lim
 
 
 def weight_iteration(ctx, iters, *, seed=SEED, init_nup=1, recursion=False, lnw_init=None,

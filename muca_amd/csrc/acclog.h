@@ -133,7 +133,8 @@ __device__ static inline float acclog_fast_band(float la)
 // lim = 4 band (from |thi|, which differs from |la| by less than 2^-19 |la|)
 // exceeds thi - log(u).  thi < 0 always: |la| > band.  Hence
 //   thi < diff  => accept,   thi - diff >= lim  => reject,
-// and only 0 <= thi - diff < lim needs the exact log.
+// and only 0 <= thi - diff < lim needs the exact log.  thi and lim are checked
+// on the device against the exact log for every one of the 2^23 inputs.
 __device__ static inline float acclog_screen(uint32_t r)
 {
     // u = (k + 1/2) 2^-23, k = r >> 9: 1 + k 2^-23 from its bits, less

@@ -226,6 +226,8 @@ hipError_t prepare_batch_lane(int fp64, int vecs, size_t lds_bytes);
 hipError_t launch_batch_update(hipStream_t st, const BatchArgs &b);
 hipError_t launch_acclog(hipStream_t st, uint32_t k0, uint32_t n, float *out);
 hipError_t launch_acclog_fast(hipStream_t st, uint32_t k0, uint32_t n, float *out);
+// out[0..n): acclog_screen, out[n..2n): acclog_screen_lim of it
+hipError_t launch_acclog_screen(hipStream_t st, uint32_t k0, uint32_t n, float *out);
 
 // Exact per-D moments of a walker block, accumulated by the update kernel in
 // place of the joint histogram: kMomWords arrays of N+1 uint64 each,

@@ -916,4 +916,20 @@ int muca_acclog_fast_device(int32_t device, uint32_t k0, uint32_t n, float *out)
     return MUCA_OK;
 }
 
+int muca_acclog_screen_device(int32_t device, uint32_t k0, uint32_t n, float *thi, float *lim)
+{
+    if (!thi || !lim || n == 0) return fail(MUCA_E_ARG, "bad arguments");
+    HIP_TRY(hipSetDevice(device));
+    float *d = nullptr;
+    int rc = dev_alloc(&d, 2ull * n, "acclog_screen");
+    if (rc) return rc;
+    hipError_t e = muca::launch_acclog_screen(nullptr, k0, n, d);
+    if (e == hipSuccess) e = hipMemcpy(thi, d, (size_t)n * 4, hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(lim, d + n, (size_t)n * 4, hipMemcpyDeviceToHost);
+    hipFree(d);
+    if (e != hipSuccess)
+        return fail(MUCA_E_HIP, std::string("acclog_screen: ") + hipGetErrorString(e));
+    return MUCA_OK;
+}
+
 }  // extern "C"

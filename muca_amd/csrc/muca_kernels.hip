@@ -662,6 +662,21 @@ hipError_t launch_acclog_fast(hipStream_t st, uint32_t k0, uint32_t n, float *ou
     return hipGetLastError();
 }
 
+__global__ void k_acclog_screen(uint32_t k0, uint32_t n, float *out)
+{
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const float thi = acclog_screen((k0 + t) << 9);
+    out[t] = thi;
+    out[(uint64_t)n + t] = acclog_screen_lim(thi);
+}
+
+hipError_t launch_acclog_screen(hipStream_t st, uint32_t k0, uint32_t n, float *out)
+{
+    hipLaunchKernelGGL(k_acclog_screen, dim3((n + 255) / 256), dim3(256), 0, st, k0, n, out);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // produce path: exact per-D moments (S0, S1, limb words of S2 and S4) -> FP64
 // in the layout of k_joint_moments' output

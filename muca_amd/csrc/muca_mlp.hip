@@ -77,8 +77,11 @@ __device__ inline float silu(float z)
 // a = silu(z) = z / q and d = silu'(z) = s (1 + z (1 - s)), s = 1 / q, with
 // q = 1 + exp(-z).  Both quotients come from one reciprocal, refined once, and
 // a residual correction each; for 1e-30 < |z| < 80 they equal the divisions'
-// results (correctly rounded) for every float z, checked exhaustively on the
-// device, in 8 instructions instead of about 20.  Outside, they are divided.
+// results (correctly rounded) for every float z, in 8 instructions instead of
+// about 20 (division by a refined reciprocal and the residual's correction:
+// P. W. Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", IBM J. Res. Develop. 34 (1990) 111); k_silu_check
+// compares every float.  Outside, they are divided.
 __device__ inline void silu_both(float z, float &a, float &d)
 {
     const float q = 1.0f + expf(-z);
@@ -95,6 +98,27 @@ __device__ inline void silu_both(float z, float &a, float &d)
         }
     }
     d = s * (1.0f + z * (1.0f - s));
+}
+
+// differing[0] counts the floats z = bits 0 .. 2^32 - 1 at which silu_both is not
+// what divisions give (bits compared, any NaN equal to any), differing[1] keeps
+// one of them
+__global__ __launch_bounds__(256) void k_silu_check(uint64_t *differing)
+{
+    const uint64_t step = (uint64_t)gridDim.x * 256;
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < 1ull << 32; i += step) {
+        const float z = __uint_as_float((uint32_t)i);
+        float a, d;
+        silu_both(z, a, d);
+        const float s = 1.0f / (1.0f + expf(-z));
+        const float ra = z / (1.0f + expf(-z)), rd = s * (1.0f + z * (1.0f - s));
+        const bool same_a = __float_as_uint(a) == __float_as_uint(ra) || (a != a && ra != ra);
+        const bool same_d = __float_as_uint(d) == __float_as_uint(rd) || (d != d && rd != rd);
+        if (!same_a || !same_d) {
+            atomicAdd((unsigned long long *)&differing[0], 1ull);
+            differing[1] = i;
+        }
+    }
 }
 
 // BF16 copies of the weights used by the products.  The square ones are kept as
@@ -658,6 +682,28 @@ int muca_mlp_create(int32_t device, muca_mlp **out)
     g->wb.w3t = g->wb.w3 + kH * kH;
     g->wb.w4 = g->wb.w3t + kH * kH;
     *out = g;
+    return MUCA_OK;
+}
+
+int muca_mlp_silu_check(int32_t device, uint64_t *differing, uint32_t *example)
+{
+    if (!differing || !example) return mfail(MUCA_E_ARG, "NULL argument");
+    MHIP(hipSetDevice(device));
+    struct Buf {
+        uint64_t *p = nullptr;
+        ~Buf()
+        {
+            if (p) (void)hipFree(p);
+        }
+    } d;
+    uint64_t h[2] = {0, 0};
+    MHIP(hipMalloc((void **)&d.p, sizeof(h)));
+    MHIP(hipMemcpy(d.p, h, sizeof(h), hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_silu_check, dim3(8192), dim3(256), 0, nullptr, d.p);
+    MHIP(hipGetLastError());
+    MHIP(hipMemcpy(h, d.p, sizeof(h), hipMemcpyDeviceToHost));
+    *differing = h[0];
+    *example = (uint32_t)h[1];
     return MUCA_OK;
 }
 
