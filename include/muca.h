@@ -40,8 +40,9 @@ extern "C" {
 #define MUCA_KEYING_WEIGHT 0   /* muca_delta_multigpu.cu:340-343,740-742 */
 #define MUCA_KEYING_PRODUCE 1  /* produce2_multigpu.cu:129-130,406-409 */
 
-/* update-kernel variants (MUCA_KERNEL_AUTO: chosen from the walkers per
- * compute unit and the layout; muca_autotune chooses by measurement) */
+/* update-kernel variants (MUCA_KERNEL_AUTO: chosen for each launch from the
+ * walkers per compute unit, the layout, what is accumulated and the attempts;
+ * muca_autotune chooses by measurement, for all launches) */
 #define MUCA_KERNEL_AUTO 0
 #define MUCA_KERNEL_GENERIC 1  /* one lane per walker, reference site order from tables */
 #define MUCA_KERNEL_TEAM 2     /* sixteen lanes per walker (8 <= L <= 256; lattices and ln W in
@@ -77,7 +78,7 @@ typedef struct muca_params {
 
 typedef struct muca_info {
     uint32_t L, N, walkers, nbins;
-    int32_t device, kernel;
+    int32_t device, kernel;       /* kernel: with MUCA_KERNEL_AUTO that of full-length launches */
     uint32_t cus, block;          /* compute units, threads per block of the update */
     uint64_t lattice_bytes, joint_bins;
     uint32_t lds_per_block;       /* bytes of LDS one workgroup may use */
@@ -151,6 +152,12 @@ int muca_set_test_hist_preload(muca_ctx *ctx, uint32_t preload);
  * device of `cus` compute units (no device call). */
 int muca_test_lane_shape(uint32_t L, uint64_t walkers, uint32_t cus, uint32_t block,
                          uint32_t *lanes, uint32_t *per_lane);
+/* Test hook: the kernel and workgroup that MUCA_KERNEL_AUTO takes for a launch
+ * (observables: 0 the D histogram, 1 the joint histogram, 2 per-D moments; no
+ * device call). */
+int muca_test_choose_kernel(uint32_t L, uint64_t walkers, int32_t precision, int32_t observables,
+                            uint64_t therm, uint64_t nup, uint32_t lds, uint32_t cus,
+                            int32_t *kernel, uint32_t *block);
 /* Test hook: the team kernel's layout for a launch on a device of `cus` compute
  * units with `lds` bytes of LDS per workgroup (no device call).  out: eligible,
  * lattices in LDS, histogram in LDS, ln W in HBM, rounds per chunk, chunk order

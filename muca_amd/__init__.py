@@ -149,6 +149,9 @@ _SIGS = {
     "muca_set_test_hist_preload": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_uint32]),
     "muca_test_lane_shape": (ctypes.c_int, [_u32, ctypes.c_uint64, _u32, _u32,
                                             ctypes.POINTER(_u32), ctypes.POINTER(_u32)]),
+    "muca_test_choose_kernel": (ctypes.c_int, [_u32, ctypes.c_uint64, ctypes.c_int32,
+                                               ctypes.c_int32, ctypes.c_uint64, ctypes.c_uint64,
+                                               _u32, _u32, _i32p, ctypes.POINTER(_u32)]),
     "muca_test_team_layout": (ctypes.c_int, [_u32, ctypes.c_uint64, ctypes.c_int32, ctypes.c_int32,
                                              _u32, _u32, ctypes.POINTER(_u32)]),
     "muca_autotune": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_uint64, _i32p,

@@ -59,5 +59,6 @@ struct muca_ctx {
     int d_state = 1;
     uint32_t hist_preload = 0;   // test hook, see muca_set_test_hist_preload
     muca::Launch cfg{};
+    bool tuned = false;          // cfg's kernel and block are muca_autotune's
     uint32_t cus = 0;
 };

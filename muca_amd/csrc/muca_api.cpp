@@ -85,10 +85,114 @@ bool probe_team(uint32_t L, uint64_t W, int fp64, bool moments, size_t lds, uint
     return muca::team_layout(a, fp64, lds, cus, lay);
 }
 
-// The launch configuration for the context's walkers as they are: its own where
-// D is the lattice's (looked up once after D or the lattice were set from
-// outside), else the generic kernel, whose accesses stay in bounds for any D.
-int launch_config(muca_ctx *c, muca::Launch &cfg)
+// What the choice of a kernel depends on.  obs: 0 the D histogram, 1 the joint
+// histogram, 2 per-D moments (of launches with nup > 0)
+struct Shape {
+    uint32_t L;
+    uint64_t W;
+    int fp64, obs;
+    size_t lds;
+    uint64_t cus;
+};
+
+Shape shape_of(const muca_ctx &c)
+{
+    const int obs = c.p.joint_blocks == 0 ? 0 : c.p.observables == MUCA_OBS_MOMENTS ? 2
+                                            : c.cfg.fp64 ? 1 : 0;
+    return {c.p.L, c.W, c.cfg.fp64, obs, c.cfg.lds_max, c.cus ? c.cus : 256u};
+}
+
+// Kernel choice (attempts/ns on MI355X).  The team kernel keeps every SIMD
+// busy when walkers are few (L = 72: 82 at 4096 walkers; 76 at 16 384
+// against 37 for one lane per walker); the lane kernel wins once there
+// are enough wavefronts to hide its memory latency.  They meet near 128
+// walkers per compute unit (L = 64, 32 768 walkers: 80 against 73; 65 536:
+// 80 against 149; L = 128 the same).  Where several workgroups of teams
+// share a compute unit's LDS and half-rows fill a round the teams lead
+// to twice that (L = 32, 65 536 walkers: 185 against 142; 131 072: 198
+// against 243).  At odd L the alternative is the generic kernel; times of
+// the teams over its at 24 576, 32 768, 49 152 and 65 536 walkers: L = 9 0.82,
+// 1.11, 1.45, 1.86; L = 11 0.67, 0.93, 1.18, 1.49 (few of a team's lanes
+// have work); L = 17 0.46, 0.62, 0.80, 1.01; two workgroups per compute
+// unit, L = 33 0.22, 0.32, 0.36, 0.47 and L = 51 0.30, 0.44, 0.53, 0.72; one,
+// L = 57 0.47, 0.72, 0.88, 1.21 and L = 63 0.45, 0.67, 0.83, 1.14.  With the
+// joint histogram, at 8192, 16 384, 24 576 and 32 768: L = 9 0.77, 1.42, 1.90,
+// 2.30; L = 11 0.64, 1.18, 1.53, 1.93; L = 13 0.37, 0.72, 0.95, 1.18; L = 17
+// 0.28, 0.47, 0.58, 0.94.  With per-D moments the alternative is the generic
+// kernel, whose atomics collide: at even L and below L = 64 teams lead at any
+// number (L = 9, 98 304 walkers: half its time; L = 72, 65 536: 85 against 25;
+// L = 128: 97 against 45; L = 48, 262 144: 67 against 43), at larger odd L to
+// 256 per compute unit (L = 65, 65 536: 0.66 of its time).  muca_autotune
+// replaces this rule by measurement.
+// A thermalisation of production keeps no observable and is chosen for as without
+// (even L, 262 144 walkers, team over generic kernel: L = 8 4.45, L = 24 1.09, L = 64
+// 1.65 times its time; the lane kernel is faster still).  Where it is part of a
+// production launch and far longer than the rest, it decides (team over generic,
+// therm = N, nup = N / 16: L = 8 1.3, L = 10 1.2, both from 65 536 walkers; L = 56 to
+// 64, 262 144 walkers 1.03 to 1.56; nup = N / 3: L = 8 1.1, others below 1).
+//   The team kernel moves whole lattices to LDS and back and sets up tables whatever
+// a launch's length, so short launches go to the others.  The attempts from which it
+// leads, as a share of N: 4096 walkers L = 10 0.08, L = 24 0.012, L = 72 0.008; 16 384
+// walkers 0.16, 0.036, 0.062; 32 768 walkers L = 24 0.10, L = 48 0.13, L = 72 0.33, L =
+// 128 0.26; 65 536 walkers L = 33 0.11, L = 45 0.16; that is about 8 + N w^2 / 65536
+// with w <= 128 walkers per compute unit.  With moments (16 384 / 65 536 walkers): L =
+// 24 0.013 / 0.035, L = 48 0.014 / 0.058, L = 72 0.000 / 0.007.  Where ln W and the
+// lattices stay in HBM nothing is set up (L = 160, 16 384 walkers: from one attempt).
+int choose_kernel(const Shape &q, uint64_t therm, uint64_t nup)
+{
+    const uint32_t L = q.L;
+    const uint64_t N = (uint64_t)L * L, n = therm + nup, w = q.W / q.cus;
+    const bool odd = L % 2 != 0, moments = q.obs == 2 && nup > 0, joint = q.obs == 1 && nup > 0;
+    muca::TeamLayout lay{};
+    const bool team_ok = probe_team(L, q.W, q.fp64, moments, q.lds, (uint32_t)q.cus, lay);
+    muca::McsArgs a{};
+    a.N = (uint32_t)N;
+    a.L = L;
+    const int other = !moments && muca::lane_eligible(a, q.fp64, q.lds) ? MUCA_KERNEL_LANE
+                                                                        : MUCA_KERNEL_GENERIC;
+    if (!team_ok) return other;
+    uint64_t per_cu = 128;   // walkers per compute unit up to which teams lead
+    if (moments)
+        per_cu = !odd || L < 64 ? UINT64_MAX / q.cus : 256;
+    else if (joint)
+        per_cu = !odd || L >= 17 ? 128 : L >= 13 ? 96 : 32;
+    else if (odd)
+        per_cu = L < 11 ? 96 : L < 32 ? 128 : lay.bytes * 2 <= q.lds ? 256 : 192;
+    else if (L >= 32 && lay.bytes * 3 <= q.lds)
+        per_cu = 256;
+    if (q.W > per_cu * q.cus) return other;
+    if (moments) {
+        if (w > 128 && (L <= 10 ? 2 * nup < therm : L >= 56 && w > 512 && 8 * nup < therm))
+            return other;
+        const uint64_t v = w < 64 ? w : 64;
+        if (L < 132 && n < 4 + N * v / (L < 64 ? 1536 : 8192)) return other;
+    } else if (!lay.lnw_global) {
+        const uint64_t v = w < 128 ? w : 128;
+        if (n < 8 + N * v * v / 65536) return other;
+    }
+    return MUCA_KERNEL_TEAM;
+}
+
+// Lanes per workgroup where none are asked for.  Lane kernel, four walkers per lane
+// (lane_walkers): 256, or 512 where its LDS (ln W and the histogram) admits one
+// workgroup per compute unit (524 288 walkers, L = 72: 570 attempts/ns either way).
+// One walker per lane: with room for several workgroups 512 once they fill the device
+// (L = 72, 262 144 walkers: 335 attempts/ns against 195 with 256); with room for one
+// the walkers of a compute unit in one workgroup (L = 128, 131 072 walkers: 186 with
+// 512 lanes against 103 with 256; 262 144: 324 with 1024).
+int default_block(int kernel, const Shape &q)
+{
+    if (kernel == MUCA_KERNEL_GENERIC) return muca::generic_block(q.W, q.cus);
+    if (kernel != MUCA_KERNEL_LANE) return 256;
+    const size_t lds = (size_t)(q.L * q.L + 1) * ((q.fp64 ? 8 : 4) + 4);
+    const bool one = lds * 2 > q.lds;
+    if (muca::lane_walkers(q.L, q.W, (uint32_t)q.cus) == 4) return one ? 512 : 256;
+    if (one) return q.W > 512 * q.cus ? 1024 : q.W > 256 * q.cus ? 512 : 256;
+    return q.W >= 1024 * q.cus ? 512 : 256;
+}
+
+// c->d_state looked up if it is not known
+int consistent(muca_ctx *c)
 {
     if (c->d_state == 0) {
         const uint64_t W = c->W;
@@ -113,10 +217,25 @@ int launch_config(muca_ctx *c, muca::Launch &cfg)
         }
         c->d_state = differ ? -1 : 1;
     }
+    return MUCA_OK;
+}
+
+// The configuration of a launch: the context's kernel (chosen for this launch where
+// none was asked for or tuned) if the walkers' D is their lattices' (looked up once
+// after either was set from outside), else the generic kernel, whose accesses stay
+// in bounds for any D.
+int launch_config(muca_ctx *c, uint64_t therm, uint64_t nup, muca::Launch &cfg)
+{
     cfg = c->cfg;
+    if (c->p.kernel == MUCA_KERNEL_AUTO && !c->tuned) {
+        cfg.kernel = choose_kernel(shape_of(*c), therm, nup);
+        if (c->p.block == 0) cfg.block = default_block(cfg.kernel, shape_of(*c));
+    }
+    if (cfg.kernel == MUCA_KERNEL_GENERIC) return MUCA_OK;
+    if (int rc = consistent(c)) return rc;
     if (c->d_state < 0) {
         cfg.kernel = MUCA_KERNEL_GENERIC;
-        if (c->p.block == 0) cfg.block = muca::generic_block(c->W, c->cus ? c->cus : 256);
+        if (c->p.block == 0) cfg.block = default_block(cfg.kernel, shape_of(*c));
     }
     return MUCA_OK;
 }
@@ -186,87 +305,15 @@ int muca_create(const muca_params *params, muca_ctx **out)
     c->cfg.fp64 = p.precision == MUCA_FP64;
     c->cfg.keying = p.keying;
     c->cfg.cus = c->cus;
-    // Kernel choice (attempts/ns on MI355X).  The team kernel keeps every SIMD
-    // busy when walkers are few (L = 72: 82 at 4096 walkers; 76 at 16 384
-    // against 37 for one lane per walker); the lane kernel wins once there
-    // are enough wavefronts to hide its memory latency.  They meet near 128
-    // walkers per compute unit (L = 64, 32 768 walkers: 80 against 73; 65 536:
-    // 80 against 149; L = 128 the same).  Where several workgroups of teams
-    // share a compute unit's LDS and half-rows fill a round the teams lead
-    // to twice that (L = 32, 65 536 walkers: 185 against 142; 131 072: 198
-    // against 243).  At odd L the alternative is the generic kernel; times of
-    // the teams over its at 24 576, 32 768, 49 152 and 65 536 walkers: L = 9 0.82,
-    // 1.11, 1.45, 1.86; L = 11 0.67, 0.93, 1.18, 1.49 (few of a team's lanes
-    // have work); L = 17 0.46, 0.62, 0.80, 1.01; two workgroups per compute
-    // unit, L = 33 0.22, 0.32, 0.36, 0.47 and L = 51 0.30, 0.44, 0.53, 0.72; one,
-    // L = 57 0.47, 0.72, 0.88, 1.21 and L = 63 0.45, 0.67, 0.83, 1.14.  With the
-    // joint histogram, at 8192, 16 384, 24 576 and 32 768: L = 9 0.77, 1.42, 1.90,
-    // 2.30; L = 11 0.64, 1.18, 1.53, 1.93; L = 13 0.37, 0.72, 0.95, 1.18; L = 17
-    // 0.28, 0.47, 0.58, 0.94.  With per-D moments the alternative is the generic
-    // kernel, whose atomics collide: at even L and below L = 64 teams lead at any
-    // number (L = 9, 98 304 walkers: half its time; L = 72, 65 536: 85 against 25;
-    // L = 128: 97 against 45; L = 48, 262 144: 67 against 43), at larger odd L to
-    // 256 per compute unit (L = 65, 65 536: 0.66 of its time).  muca_autotune
-    // replaces this rule by measurement.
-    const uint64_t ncu = (uint64_t)(cu > 0 ? cu : 256);
-    if (p.kernel == MUCA_KERNEL_AUTO) {
-        // eligibility as the launch decides it (layout in this device's LDS)
-        const size_t lds_probe = (size_t)(lds > 0 ? lds : 65536);
-        muca::TeamLayout lay_probe{};
-        const bool team_ok = probe_team(p.L, W, p.precision == MUCA_FP64, moments, lds_probe,
-                                        c->cus, lay_probe);
-        muca::McsArgs probe{};
-        probe.N = p.L * p.L;
-        probe.L = p.L;
-        const bool lane_ok = muca::lane_eligible(probe, p.precision == MUCA_FP64, lds_probe);
-        const bool odd = p.L % 2 != 0, joint = p.joint_blocks > 0;
-        uint64_t per_cu = 128;
-        if (moments)
-            per_cu = !odd || p.L < 64 ? UINT64_MAX / ncu : 256;
-        else if (joint)
-            per_cu = !odd || p.L >= 17 ? 128 : p.L >= 13 ? 96 : 32;
-        else if (odd)
-            per_cu = p.L < 11 ? 96 : p.L < 32 ? 128 : lay_probe.bytes * 2 <= lds_probe ? 256 : 192;
-        else if (p.L >= 32 && lay_probe.bytes * 3 <= lds_probe)
-            per_cu = 256;
-        if (team_ok && (uint64_t)W <= per_cu * ncu)
-            c->cfg.kernel = MUCA_KERNEL_TEAM;
-        else if (moments)
-            c->cfg.kernel = MUCA_KERNEL_GENERIC;
-        else if (lane_ok)
-            c->cfg.kernel = MUCA_KERNEL_LANE;
-        else
-            c->cfg.kernel = MUCA_KERNEL_GENERIC;
-    } else {
-        c->cfg.kernel = p.kernel;
-    }
+    c->cfg.lds_max = (size_t)(lds > 0 ? lds : 65536);
+    // the kernel of full-length launches; a launch that differs chooses for itself
+    c->cfg.kernel = p.kernel != MUCA_KERNEL_AUTO ? p.kernel
+                                                 : choose_kernel(shape_of(*c), c->N, c->N);
     if (p.block != 0 && (p.block < 64 || p.block > 1024 || p.block % 64 != 0)) {
         delete c;
         return fail(MUCA_E_ARG, "block must be 0 or a multiple of 64 in [64, 1024]");
     }
-    c->cfg.block = p.block ? (int)p.block : 256;
-    if (p.block == 0 && c->cfg.kernel == MUCA_KERNEL_GENERIC)
-        c->cfg.block = muca::generic_block(W, ncu);
-    if (p.block == 0 && c->cfg.kernel == MUCA_KERNEL_LANE) {
-        // Four walkers per lane (lane_walkers): 256 lanes, or 512 where the
-        // lane kernel's LDS (ln W and the histogram) admits one workgroup per
-        // compute unit (524 288 walkers, L = 72: 570 attempts/ns either way).
-        // One walker per lane: with room for several workgroups 512 lanes once
-        // they fill the device (L = 72, 262 144 walkers: 335 attempts/ns
-        // against 195 with 256 lanes); with room for one the walkers of a
-        // compute unit in one workgroup (L = 128, 131 072 walkers: 186 with
-        // 512 lanes against 103 with 256; 262 144: 324 with 1024).
-        const size_t tsz = p.precision == MUCA_FP64 ? 8 : 4;
-        const size_t lds_lane = (size_t)(p.L * p.L + 1) * (tsz + 4);
-        const bool one = lds_lane * 2 > (size_t)(lds > 0 ? lds : 65536);
-        if (muca::lane_walkers(p.L, W, (uint32_t)ncu) == 4)
-            c->cfg.block = one ? 512 : 256;
-        else if (one)
-            c->cfg.block = W > 512ull * ncu ? 1024 : W > 256ull * ncu ? 512 : 256;
-        else
-            c->cfg.block = W >= 1024ull * ncu ? 512 : 256;
-    }
-    c->cfg.lds_max = (size_t)(lds > 0 ? lds : 65536);
+    c->cfg.block = p.block ? (int)p.block : default_block(c->cfg.kernel, shape_of(*c));
     const uint64_t N = c->N;
     int rc = MUCA_OK;
     if (!rc) rc = dev_alloc(&c->lat, N * W, "lattice");
@@ -507,7 +554,7 @@ int muca_run(muca_ctx *c, uint32_t iter, uint32_t seed, uint64_t therm, uint64_t
     a.joint_blocks = c->p.joint_blocks;
     a.hist_preload = c->hist_preload;
     muca::Launch cfg;
-    if (int rc = launch_config(c, cfg)) return rc;
+    if (int rc = launch_config(c, therm, nup, cfg)) return rc;
     HIP_TRY(hipEventRecord(c->ev0, c->st));
     HIP_TRY(muca::launch_mcs(c->st, cfg, a));
     HIP_TRY(hipEventRecord(c->ev1, c->st));
@@ -539,6 +586,17 @@ int muca_test_lane_shape(uint32_t L, uint64_t walkers, uint32_t cus, uint32_t bl
     return MUCA_OK;
 }
 
+int muca_test_choose_kernel(uint32_t L, uint64_t walkers, int32_t precision, int32_t observables,
+                            uint64_t therm, uint64_t nup, uint32_t lds, uint32_t cus,
+                            int32_t *kernel, uint32_t *block)
+{
+    if (!kernel || !block) return fail(MUCA_E_ARG, "NULL argument");
+    const Shape q{L, walkers, precision == MUCA_FP64, observables, lds, cus};
+    *kernel = choose_kernel(q, therm, nup);
+    *block = (uint32_t)default_block(*kernel, q);
+    return MUCA_OK;
+}
+
 int muca_test_team_layout(uint32_t L, uint64_t walkers, int32_t precision, int32_t moments,
                           uint32_t lds, uint32_t cus, uint32_t *out)
 {
@@ -562,8 +620,7 @@ int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *blo
     if (attempts == 0) return fail(MUCA_E_ARG, "attempts must be > 0");
     HIP_TRY(hipSetDevice(c->p.device));
     const uint64_t N = c->N, W = c->W;
-    muca::Launch cfg0;
-    int rc = launch_config(c, cfg0);
+    int rc = consistent(c);
     if (rc) return rc;
     int8_t *lat0 = nullptr;
     int32_t *st0 = nullptr;
@@ -667,6 +724,7 @@ int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *blo
     hipFree(lat0);
     hipFree(st0);
     if (e != hipSuccess) return fail(MUCA_E_HIP, std::string("autotune: ") + hipGetErrorString(e));
+    c->tuned = true;
     c->cfg.kernel = pick.kernel;
     c->cfg.block = pick.block;
     if (kernel) *kernel = pick.kernel;

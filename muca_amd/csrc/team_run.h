@@ -295,9 +295,6 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     // launch against 0.83 one at a time; L = 16, 30 003 walkers 0.086 against 0.093.
     const bool lat_vec = LATLDS && W % kTeams == 0 && wbase + kTeams <= W &&
                          ((uintptr_t)a.lat & 15) == 0;
-    const bool mine = wbase + tl < W;
-    const uint32_t byte_site = (lat_vec ? N & ~3u : 0u) + team;
-    int8_t *const byte_row = latl + tl * lay.lat_stride;
     if (LATLDS) {
         if (lat_vec) {
             for (uint32_t q = tid; q < N / 4; q += blockDim.x) {
@@ -319,10 +316,14 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 }
             }
         }
-        // walkers past the last one read the first's spins, which are not used
-        const int8_t *const g = a.lat + wbase + (mine ? tl : 0);
+        int t = tid;   // a copy of its own here and below, so that nothing made of it
+        asm volatile("" : "+v"(t));   // stays in registers between the two
+        const uint32_t wl = t & 15;
+        const int8_t *const g = a.lat + wbase + (wbase + wl < W ? wl : 0);
+        int8_t *const l = latl + wl * lay.lat_stride;
 #pragma unroll 4
-        for (uint32_t site = byte_site; site < N; site += kTeams) byte_row[site] = g[(uint64_t)site * W];
+        for (uint32_t site = (lat_vec ? N & ~3u : 0u) + ((uint32_t)t >> 4); site < N; site += kTeams)
+            l[site] = g[(uint64_t)site * W];
     }
     __syncthreads();
     if (FP64 && !LNWG)
@@ -966,9 +967,14 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
                 }
             }
         }
-        if (mine) {
-            int8_t *const g = a.lat + wbase + tl;
-            for (uint32_t site = byte_site; site < N; site += kTeams) g[(uint64_t)site * W] = byte_row[site];
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        const uint32_t wl = t & 15;
+        if (wbase + wl < W) {
+            int8_t *const g = a.lat + wbase + wl;
+            const int8_t *const l = latl + wl * lay.lat_stride;
+            for (uint32_t site = (lat_vec ? N & ~3u : 0u) + ((uint32_t)t >> 4); site < N; site += kTeams)
+                g[(uint64_t)site * W] = l[site];
         }
     }
 }
