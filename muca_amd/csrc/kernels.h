@@ -213,8 +213,9 @@ const void *batch_team_function(int fp64);   // the build for every kind of inst
 
 // persistent kernels: every workgroup takes tiles (batch_take) until none is left
 // lat_modes: bit 0 set if some instance keeps its tile's lattices in LDS,
-// bit 1 if some reads them from HBM; nrs: the rounds per chunk (1..4) that
-// every instance has, else 0.  The kernel built for just those is launched.
+// bit 1 if some reads them from HBM; nrs: the rounds per chunk (1..4, 8 more where
+// chunks run on over row ends) that every instance has, else 0.  The kernel built
+// for just those is launched.
 hipError_t launch_batch_team(hipStream_t st, int fp64, const BatchArgs &b, uint32_t grid,
                              size_t lds_bytes, int lat_modes, int nrs);
 hipError_t launch_batch_lane(hipStream_t st, int fp64, int vecs, const BatchArgs &b, uint32_t grid,

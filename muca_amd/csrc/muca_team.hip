@@ -203,6 +203,8 @@ static void (*batch_team_kernel(int lat_modes, int nrs))(BatchArgs)
         default: return k_batch_team<FP64, 1, 0>;
         }
     }
+    // lattices in HBM, chunks of four rounds (L = 98 to 128): 15.5 ms for 8 iterations
+    // of L = 128, 4096 walkers, against 15.75 in the build for any
     if (lat_modes == 2 && nrs == 4) return k_batch_team<FP64, 2, 4>;
     return lat_modes == 2 ? k_batch_team<FP64, 2, 0> : k_batch_team<FP64, 3, 0>;
 }

@@ -34,7 +34,8 @@
 //   diff = ((T)(-dE*beta) + lnW[D+dDel]) - lnW[D];  accept iff diff >= 0 or
 //   acclog(r1) < diff.  Because acclog(r1) < 0 always, that is exactly
 //   acclog(r1) < diff.  Results are bit-identical to the one-lane kernel.
-// Requires 8 <= L <= 256.  A half-row need not be a whole number of Philox
+// Requires 8 <= L <= 256, and walkers whose D is their lattice's (D indexes LDS and
+// HBM unchecked).  A half-row need not be a whole number of Philox
 // blocks: a chunk starts at word rs % 4 of its first block.  Odd L (ODD, while
 // the lattices fit in LDS): the reference's order visits the even linear
 // indices 0, 2, .., N-3 twice and then N-2 (muca_delta_multigpu.cu:173).  Two
@@ -979,8 +980,9 @@ __device__ __forceinline__ void team_run(const McsArgs &a, const TeamLayout &lay
     }
 }
 
-// LNWG launches are the large lattices (L >= 136) with many walkers: they
-// are held to 128 VGPRs, four wavefronts per SIMD
+// LNWG launches are those of large lattices (FP64 from L = 138, with moments from
+// 132; FP32 from 194) and, with moments, of more walkers than LDS keeps resident
+// (from L = 54): they are held to 128 VGPRs, four wavefronts per SIMD
 template <int R, bool FP64, int KEYING, bool LATLDS, bool LDSHIST, int OBS, bool LNWG, int NR,
           int ORD = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LNWG ? 4 : 1))) void
@@ -1016,8 +1018,7 @@ hipError_t launch_team_nr(hipStream_t st, const McsArgs &a, const TeamLayout &la
             : joint ? k_mcs_team<R, FP64, KEYING, true, false, 1, false, NR, ORD>
                     : k_mcs_team<R, FP64, KEYING, true, false, 0, false, NR, ORD>;
     } else if (lay.lnw_global) {
-        // ln W too large for LDS (L >= 136): lattices and histogram stay in
-        // HBM as well
+        // ln W read through windows: lattices and histogram stay in HBM as well
         if constexpr (NR == kLnwgRounds) {
             k = moms ? k_mcs_team<R, FP64, KEYING, false, false, MO, true, NR>
                 : joint ? k_mcs_team<R, FP64, KEYING, false, false, 1, true, NR>
