@@ -626,11 +626,22 @@ int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *blo
     int32_t *st0 = nullptr;
     rc = dev_alloc(&lat0, N * W, "autotune lattice copy");
     if (rc) return rc;
-    rc = dev_alloc(&st0, 3 * W, "autotune state copy");
+    // walkers whose D is not their lattice's are tuned with their lattice's state
+    // (the lane and team kernels run no others); their own follows the copies
+    const bool own = c->d_state > 0;
+    rc = dev_alloc(&st0, (own ? 3 : 6) * W, "autotune state copy");
     if (rc) {
         hipFree(lat0);
         return rc;
     }
+    int32_t *const state[3] = {c->E, c->D, c->M};
+    auto keep_state = [&](bool save) -> hipError_t {
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < 3 && e == hipSuccess; k++)
+            e = hipMemcpyAsync(save ? st0 + (3 + k) * W : state[k], save ? state[k] : st0 + (3 + k) * W,
+                               W * 4, hipMemcpyDeviceToDevice, c->st);
+        return e;
+    };
     auto save_restore = [&](bool save) -> hipError_t {
         hipError_t e;
         if (save) {
@@ -686,13 +697,15 @@ int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *blo
         a.joint_blocks = c->p.joint_blocks;
         a.block_walkers = c->block_walkers ? c->block_walkers : c->W;
     }
-    const bool any = c->d_state > 0;   // D is the lattice's: any kernel may run
-    if (any && muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, c->cus, lay))
+    if (muca::team_layout(a, c->cfg.fp64, c->cfg.lds_max, c->cus, lay))
         cands.push_back({MUCA_KERNEL_TEAM, 256});
-    if (any && !moments && muca::lane_eligible(a, c->cfg.fp64, c->cfg.lds_max))
+    if (!moments && muca::lane_eligible(a, c->cfg.fp64, c->cfg.lds_max))
         for (int b : {256, 512, 1024}) cands.push_back({MUCA_KERNEL_LANE, b});
     for (int b : {64, 128, 256}) cands.push_back({MUCA_KERNEL_GENERIC, b});
-    hipError_t e = save_restore(true);
+    hipError_t e = own ? hipSuccess : keep_state(true);
+    if (e == hipSuccess && !own)
+        e = muca::launch_state(c->st, c->lat, W, c->p.L, c->E, c->D, c->M);
+    if (e == hipSuccess) e = save_restore(true);
     float best = 0;
     Cand pick = {c->cfg.kernel, c->cfg.block};
     for (const Cand &cd : cands) {
@@ -720,6 +733,7 @@ int muca_autotune(muca_ctx *c, uint64_t attempts, int32_t *kernel, uint32_t *blo
         }
     }
     if (e == hipSuccess) e = save_restore(false);
+    if (e == hipSuccess && !own) e = keep_state(false);
     if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     hipFree(lat0);
     hipFree(st0);

@@ -68,15 +68,30 @@ def test_foreign_state_runs_as_generic(L, W, obs, blocks, prepare):
         assert np.array_equal(a, b)
 
 
-def test_lane_kernel_and_autotune():
+def test_lane_kernel():
     for prepare in (_no_state, _zero, _full):
         got = _run(10, 64, M.OBS_JOINT, 1, M.KERNEL_LANE, prepare)
         for a, b in zip(got, _run(10, 64, M.OBS_JOINT, 1, M.KERNEL_GENERIC, prepare)):
             assert np.array_equal(a, b)
-    with M.Context(24, 64) as ctx:
-        _zero(ctx)
+
+
+def test_autotune_keeps_a_foreign_state_and_every_candidate():
+    """Tuned before the state is computed: the choice is made among all kernels
+    (4096 walkers: teams by a factor of five) and the walkers are left as they were."""
+    with M.Context(64, 4096) as ctx:
+        _full(ctx)
+        E, _, Mg = ctx.get_state()
+        ctx.set_state(E + 1, None, Mg - 1)
+        lat, state = ctx.get_lattice(), ctx.get_state()
         ctx.set_log_weight(np.zeros(ctx.N + 1))
-        assert ctx.autotune(100)[0] == M.KERNEL_GENERIC
+        assert ctx.autotune(4000)[0] == M.KERNEL_TEAM
+        assert np.array_equal(ctx.get_lattice(), lat)
+        for a, b in zip(ctx.get_state(), state):
+            assert np.array_equal(a, b)
+        ctx.compute_state()
+        ctx.run(0, 1, 10, 10)
+        D = ctx.get_state()[1]
+        assert np.array_equal(D, np.abs(ctx.get_lattice().astype(np.int32)).sum(0))
 
 
 def test_own_state_set_from_outside(orc):
